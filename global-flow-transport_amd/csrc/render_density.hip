@@ -448,20 +448,17 @@ __global__ __launch_bounds__(256) void k_render_density_bwd_pixel(const float* _
   }
 }
 
-// Gather: one wave per block of WX x WY x WZ voxels, accumulated in a
-// wave-private FP64 LDS region. For each view the wave enumerates the pixels
-// whose rays can cross the block's support box (x0-1, x0+WX) x ... (the
-// projected box; lanes take consecutive pixels in row order), cuts each ray by
-// the box and adds every inside sample's gradient alpha c_i + beta,
-// trilinear-weighted, to the corner voxels that lie in the block (a sample
-// q reaches voxel c with weight prod_a max(0, 1 - |q_a - c_a|)). The pixel loop
-// is amortised over a whole block. Only this wave touches its region, so the
-// sums run in a fixed order (deterministic) and one store per voxel follows.
+// Gather: one workgroup of NW waves per block of WX x WY x WZ voxels, each wave
+// accumulating in an FP64 LDS region of its own. For each view the waves
+// enumerate the pixels whose rays can cross the block's support box (x0-1,
+// x0+WX) x ... (the projected box, in batches of 64 consecutive pixels in row
+// order, which the waves take in turn), cut each ray by the box and add every
+// inside sample's gradient alpha c_i + beta, trilinear-weighted, to the corner
+// voxels that lie in the block (a sample q reaches voxel c with weight prod_a
+// max(0, 1 - |q_a - c_a|)). The pixel loop is amortised over a whole block. Only
+// its own wave touches a region, and the store adds the NW regions in wave
+// order, so the sums run in a fixed order (deterministic); one store per voxel.
 constexpr int kGatherBatch = 4;  // saved values loaded per round trip (2: 0.187 ms, 8: 0.211 ms at c2)
-// voxel blocks (one per wave) per workgroup: every c2 block is resident at
-// once, so 4 per workgroup costs no waiting there (c2: 0.175 ms; 1: 0.178);
-// c5 runs several rounds (1: 1.648 ms against 1.676)
-constexpr int kRGatherWaves = 4;
 //
 // LIT (the spot-lit render): a second region sums the emission gradients
 // alpha u_i * w of the d * lambda grid; the store then writes
@@ -471,41 +468,40 @@ constexpr int kRGatherWaves = 4;
 // folded in), workgroup 0 first sums the pixel pass's per-tile loss partials
 // of every view in a fixed order; the kernel boundary after the pixel pass
 // makes them visible, so no separate launch is needed.
-template <int WX, int WY, int WZ, bool LIT = false>
-__global__ __launch_bounds__(256) void k_render_density_bwd_gather(RenderSaved sv, float* __restrict__ grad,
-                                                                   RayDims rd, ProjLaunch PL,
-                                                                   const float* __restrict__ dens,
-                                                                   const float* __restrict__ lam,
-                                                                   float* __restrict__ lam_grad,
-                                                                   float* __restrict__ loss, float loss_scale) {
+template <int WX, int WY, int WZ, int NW, bool LIT>
+__global__ __launch_bounds__(64 * NW) void k_render_density_bwd_gather(RenderSaved sv, float* __restrict__ grad,
+                                                                       RayDims rd, ProjLaunch PL,
+                                                                       const float* __restrict__ dens,
+                                                                       const float* __restrict__ lam,
+                                                                       float* __restrict__ lam_grad,
+                                                                       float* __restrict__ loss, float loss_scale) {
   if (loss && blockIdx.x == 0) {
-    __shared__ float red[256];
+    __shared__ float red[64 * NW];
     loss_sum_block(sv.partials, sv.n_partials, loss_scale, loss, red);
   }
   // rows padded to WX + 1 doubles: lanes at one x in neighbouring rows fall on
   // different LDS banks (16 doubles are 128 bytes, the banks' width)
   constexpr int kRX = WX + 1;
   constexpr int kVox = kRX * WY * WZ;
-  __shared__ double region[LIT ? 2 * kRGatherWaves : kRGatherWaves][kVox];
+  __shared__ double region[LIT ? 2 * NW : NW][kVox];
   typedef __attribute__((address_space(3))) double lds_double;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   lds_double* acc = (lds_double*)region[wave];
-  lds_double* acc2 = (lds_double*)region[LIT ? kRGatherWaves + wave : wave];
+  lds_double* acc2 = (lds_double*)region[LIT ? NW + wave : wave];
   const Dims3 d = rd.in;
-  const int nbx = (d.x + WX - 1) / WX, nby = (d.y + WY - 1) / WY, nbz = (d.z + WZ - 1) / WZ;
-  const int blk = blockIdx.x * kRGatherWaves + wave;
-  const bool live = blk < nbx * nby * nbz;  // a wave past the last block only joins the barriers
+  const int nbx = (d.x + WX - 1) / WX, nby = (d.y + WY - 1) / WY, blk = (int)blockIdx.x;
   const int x0 = (blk % nbx) * WX, y0 = ((blk / nbx) % nby) * WY, z0 = (blk / (nbx * nby)) * WZ;
   for (int k = lane; k < kVox; k += 64) acc[k] = 0.0;
   if (LIT)
     for (int k = lane; k < kVox; k += 64) acc2[k] = 0.0;
+  int turn = wave;  // pixel batches, counted through the views, until this wave's next one
   const size_t plane = size_t(rd.out_w) * rd.out_h;
   const float fx0 = (float)x0, fy0 = (float)y0, fz0 = (float)z0;
   // support box in ray coordinates (which carry the +0.5 cell-centre offset)
   const float bx0 = fx0 - 0.5f, by0 = fy0 - 0.5f, bz0 = fz0 - 0.5f;
   const float bx1 = bx0 + (float)(WX + 1), by1 = by0 + (float)(WY + 1), bz1 = bz0 + (float)(WZ + 1);
   const float hx = 0.5f * (float)(WX + 1), hy = 0.5f * (float)(WY + 1), hz = 0.5f * (float)(WZ + 1);
-  for (int vi = 0; vi < PL.num_views && live; ++vi) {
+  for (int vi = 0; vi < PL.num_views; ++vi) {
     const ProjView& pv = PL.view[vi];
     const float* A = pv.pmv;
     const float4 cc = mat_vec(A, fx0 + 0.5f * (float)WX, fy0 + 0.5f * (float)WY, fz0 + 0.5f * (float)WZ, 1.f);
@@ -537,22 +533,25 @@ __global__ __launch_bounds__(256) void k_render_density_bwd_gather(RenderSaved s
     const float4* rview = sv.records + (size_t)pv.out_slot * plane;
     {
       const int nx = xe - xs + 1, cnt = nx * (ye - ys + 1);
-      // lane k of the box's row-major pixel list; the next record (k + 64) is
-      // loaded while the current one is walked
-      const int dy64 = 64 / nx, dx64 = 64 - dy64 * nx;
-      int px = xs + lane % nx, py = ys + lane / nx;
-      float4 rec_next = lane < cnt ? rview[size_t(py) * rd.out_w + px] : make_float4(0.f, 0.f, 0.f, 0.f);
-      for (int k = lane; k < cnt; k += 64) {
-        const size_t pix = size_t(py) * rd.out_w + px;
+      // this lane's first place in the box's row-major pixel list; its next
+      // record (64 NW on) is loaded while the current one is walked
+      constexpr int kStride = 64 * NW;
+      const int first = turn * 64 + lane;
+      turn -= (cnt + 63) / 64 % NW;
+      turn += turn < 0 ? NW : 0;
+      const int dys = kStride / nx, dxs = kStride - dys * nx;
+      int px = xs + first % nx, py = ys + first / nx;
+      float4 rec_next = first < cnt ? rview[size_t(py) * rd.out_w + px] : make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int k = first; k < cnt; k += kStride) {
         const float fpx = (float)px, fpy = (float)py;
         const float4 rec = rec_next;
-        px += dx64;
-        py += dy64;
+        px += dxs;
+        py += dys;
         if (px > xe) {
           px -= nx;
           ++py;
         }
-        if (k + 64 < cnt) rec_next = rview[size_t(py) * rd.out_w + px];
+        if (k + kStride < cnt) rec_next = rview[size_t(py) * rd.out_w + px];
         const int lo = __float_as_int(rec.x), hi = __float_as_int(rec.y);
         if (lo > hi) continue;
         const float4 gn = make_float4(fmaf(fpy, pv.gy[0], fmaf(fpx, pv.gx[0], pv.near0[0])),
@@ -643,20 +642,24 @@ __global__ __launch_bounds__(256) void k_render_density_bwd_gather(RenderSaved s
     }
   }
   __syncthreads();
-  if (!live) return;
-  for (int k0 = lane; k0 < WX * WY * WZ; k0 += 64) {
+  for (int k0 = threadIdx.x; k0 < WX * WY * WZ; k0 += 64 * NW) {
     const int x = x0 + k0 % WX, y = y0 + (k0 / WX) % WY, z = z0 + k0 / (WX * WY);
     const int k = (k0 / WX) * kRX + k0 % WX;
     if (x < d.x && y < d.y && z < d.z) {
       const size_t f = flat3(x, y, z, d);
       float* g = grad + f;
+      double ss = region[0][k];
+#pragma unroll
+      for (int w = 1; w < NW; ++w) ss += region[w][k];
       if (LIT) {
-        const double se = acc2[k];
-        const float v = (float)(acc[k] + (double)lam[f] * se), vl = (float)((double)dens[f] * se);
+        double se = region[NW][k];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) se += region[NW + w][k];
+        const float v = (float)(ss + (double)lam[f] * se), vl = (float)((double)dens[f] * se);
         *g = PL.accumulate ? *g + v : v;
         lam_grad[f] = PL.accumulate ? lam_grad[f] + vl : vl;
       } else {
-        const float v = (float)acc[k];
+        const float v = (float)ss;
         *g = PL.accumulate ? *g + v : v;
       }
     }
@@ -992,17 +995,43 @@ hipError_t render_density_pixel_launch(bool l2, hipStream_t s, const float* img,
   return hipGetLastError();
 }
 
-constexpr int kGatherWX = 16, kGatherWY = 16, kGatherWZ = 2;
+template <int WX, int WY, int WZ, int NW, bool LIT>
+static void launch_render_gather(hipStream_t s, const RenderSaved& sv, const float* dens, const float* lam,
+                                 float* grad, float* lam_grad, const RayDims& rd, const ProjLaunch& PL, float* loss,
+                                 float loss_scale) {
+  const int nb = ((rd.in.x + WX - 1) / WX) * ((rd.in.y + WY - 1) / WY) * ((rd.in.z + WZ - 1) / WZ);
+  auto kern = k_render_density_bwd_gather<WX, WY, WZ, NW, LIT>;
+  hipLaunchKernelGGL(kern, dim3(nb), dim3(64 * NW), 0, s, sv, grad, rd, PL, dens, lam, lam_grad, loss, loss_scale);
+}
+
+// Block shape and waves per block, by the number of 16x16x2-voxel blocks nb.
+// A block's waves share its pixels, so more of them help wherever blocks
+// alone do not fill the 256 CUs evenly; each costs a region to clear and sum.
+// Measured (gather alone, us; 1 / 2 / 4 / 8 waves per 16x16x2 block):
+//   nb = 29900 (200x356x200, 8 views)  1619 / 1529 / 1520 / 1640
+//   nb = 14400 (160x280x160, 5 views)   246 /  223 /  246 /  318
+//   nb =  7168 (128x224x128, 5 views)   172 /  163 /  163 /  188
+//   nb =  4200 (100x178x100, 6 views)   278 /  223 /  203 /  205
+//   nb =   868 (61x107x59, 5 views)      93 /   57 /   43 /   41
+//   nb =   432 (48x86x48, 5 views)      186 /  104 /   63 /   50
+//   nb =    64 (32x32x32, 2 views)      428 /  208 /  119 /   96
+// The last has a block for every fourth CU only: 4x4x4-voxel blocks, 512 of
+// them, take 29 us with 8 waves (8x4x4 blocks: 31, 8x8x2: 34).
+template <bool LIT>
+static void render_gather(hipStream_t s, const RenderSaved& sv, const float* dens, const float* lam, float* grad,
+                          float* lam_grad, const RayDims& rd, const ProjLaunch& PL, float* loss, float loss_scale) {
+  const int64_t nb = (int64_t)((rd.in.x + 15) / 16) * ((rd.in.y + 15) / 16) * ((rd.in.z + 1) / 2);
+  if (nb < 256) launch_render_gather<4, 4, 4, 8, LIT>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
+  else if (nb < 640) launch_render_gather<16, 16, 2, 8, LIT>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
+  else if (nb < 8192) launch_render_gather<16, 16, 2, 4, LIT>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
+  else launch_render_gather<16, 16, 2, 2, LIT>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
+}
 
 // loss: null, or where workgroup 0 writes loss_scale * the sum of the loss partials
 hipError_t render_density_gather_launch(hipStream_t s, const RenderSaved& sv, float* grad, const RayDims& rd,
                                         const ProjLaunch& PL, float* loss, float loss_scale) {
-  const int nb = ((rd.in.x + kGatherWX - 1) / kGatherWX) * ((rd.in.y + kGatherWY - 1) / kGatherWY) *
-                 ((rd.in.z + kGatherWZ - 1) / kGatherWZ);
   KernelTimer t(s, "render_bwd_gather");
-  auto kern = k_render_density_bwd_gather<kGatherWX, kGatherWY, kGatherWZ>;
-  hipLaunchKernelGGL(kern, dim3((nb + kRGatherWaves - 1) / kRGatherWaves), dim3(64 * kRGatherWaves), 0, s, sv, grad, rd,
-                     PL, nullptr, nullptr, nullptr, loss, loss_scale);
+  render_gather<false>(s, sv, nullptr, nullptr, grad, nullptr, rd, PL, loss, loss_scale);
   return hipGetLastError();
 }
 
@@ -1010,12 +1039,8 @@ hipError_t render_density_gather_launch(hipStream_t s, const RenderSaved& sv, fl
 hipError_t render_density_lit_gather_launch(hipStream_t s, const RenderSaved& sv, const float* dens,
                                             const float* lam, float* grad, float* lam_grad, const RayDims& rd,
                                             const ProjLaunch& PL, float* loss, float loss_scale) {
-  const int nb = ((rd.in.x + kGatherWX - 1) / kGatherWX) * ((rd.in.y + kGatherWY - 1) / kGatherWY) *
-                 ((rd.in.z + kGatherWZ - 1) / kGatherWZ);
   KernelTimer t(s, "render_lit_bwd_gather");
-  auto kern = k_render_density_bwd_gather<kGatherWX, kGatherWY, kGatherWZ, true>;
-  hipLaunchKernelGGL(kern, dim3((nb + kRGatherWaves - 1) / kRGatherWaves), dim3(64 * kRGatherWaves), 0, s, sv, grad, rd,
-                     PL, dens, lam, lam_grad, loss, loss_scale);
+  render_gather<true>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
   return hipGetLastError();
 }
 

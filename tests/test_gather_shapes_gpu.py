@@ -1,0 +1,51 @@
+"""The render backward's voxel-block gathers at the edges of their rules: block
+shapes and waves per block are picked by the grid's block count, so grids on
+both sides of each line, ragged against the blocks, against the FP64 oracle
+(gradients 1e-4 normalised max error, as the other render backward tests),
+with more than 16 views (two accumulating launches) and repeated bit for bit.
+"""
+import numpy as np
+import pytest
+import torch
+
+from helpers import norm_err, scene
+from oracle import oracle as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def _t(a):
+    return torch.from_numpy(np.ascontiguousarray(a, dtype=np.float32)).cuda()
+
+
+# blocks of 16x16x2: 1, 189, 260, 612, 660, 756
+RENDER_GRIDS = [((1, 1, 1), (9, 7), 1), ((41, 97, 33), (60, 34), 3), ((52, 72, 31), (66, 40), 2),
+                ((67, 81, 33), (50, 30), 18), ((66, 65, 49), (40, 90), 2), ((36, 90, 97), (70, 40), 3)]
+
+
+@pytest.mark.parametrize("grid,image,views", RENDER_GRIDS)
+@pytest.mark.parametrize("lit", [False, True])
+def test_render_gather_block_rules(cuda, grid, image, views, lit):
+    from gft.pipeline import render_density, render_density_lit
+    sc = scene(grid=grid, image=image, views=views, seed=sum(grid))
+    cam = (sc["M"], sc["V"], sc["P"], sc["F"], sc["out_dhw"], sc["step"])
+    rng = np.random.Generator(np.random.PCG64(views))
+    lam = rng.uniform(0.2, 1.2, size=sc["data"].shape).astype(np.float32)
+    w = rng.uniform(-1, 1, size=(1, views) + tuple(image) + (4,)).astype(np.float32)
+
+    def grads():
+        d, l = _t(sc["data"]).requires_grad_(True), _t(lam).requires_grad_(True)
+        img = render_density_lit(d, l, *cam, ambient=0.4) if lit else render_density(d, *cam)
+        img.backward(_t(w))
+        torch.cuda.synchronize()
+        return img.detach().cpu().numpy(), d.grad, l.grad
+
+    img, gd, gl = grads()
+    if lit:
+        rd, rl = orc.render_lit_bwd(sc["data"], lam, img, w, *cam, ambient=0.4)
+        assert norm_err(gl.cpu().numpy(), rl) < 1e-4
+    else:
+        rd = orc.render_density_bwd(sc["data"], img, w, *cam)
+    assert norm_err(gd.cpu().numpy(), rd) < 1e-4
+    _, gd2, gl2 = grads()
+    assert torch.equal(gd, gd2) and (not lit or torch.equal(gl, gl2))
