@@ -26,7 +26,7 @@
 //                      ray, clipped to the grid box, marches its samples
 //                      keeping each sample's c_k, writes its pixel, its loss
 //                      term, its gradient record and the view's largest LoD;
-//   k_batch_gather(m)  one wave per block of level-m voxels: for every view
+//   k_batch_gather(m)  a few waves per block of level-m voxels: for every view
 //                      whose samples read level m, the candidate pixels of the
 //                      block's support box, each column cut by the box, every
 //                      sample's gradient alpha c_k + beta times its level-m
@@ -499,8 +499,8 @@ __global__ __launch_bounds__(kTilePix) void k_batch_fwd(const BatchRec* __restri
 }
 
 // ------------------------------------------------------------------- gather
-// The transpose of the resample's trilinear scatter: one wave per voxel block,
-// accumulated in wave-private FP64 LDS regions. PAIR: levels 0 and 1 at once,
+// The transpose of the resample's trilinear scatter: kGatherWaves waves per voxel
+// block, accumulated in wave-private FP64 LDS regions that the store adds up. PAIR: levels 0 and 1 at once,
 // a block of bw x bh x bd level-0 voxels and the (bw/2) x (bh/2) x (bd/2)
 // level-1 cells over it (the level-1 cells' support box contains the level-0
 // voxels', so one walk over the candidate samples serves both); otherwise
@@ -515,20 +515,20 @@ __global__ __launch_bounds__(kTilePix) void k_batch_fwd(const BatchRec* __restri
 // a fixed order and one store per voxel follows.
 typedef __attribute__((address_space(3))) double lds_f64;  // an FP64 LDS region
 constexpr int kGatherBatch = 4;  // c_k loaded per round trip
-// voxel blocks (one per wave) per gather item: the waves of an item meet at
-// its barriers, so with several the fast blocks wait for the slow one; one
-// wave per workgroup measured best (c4: 4.84 ms against 4.95 with 2 and 5.15
-// with 4)
-constexpr int kGatherWaves = 1;
+// waves that share a voxel block: they take its pixel batches in turn, each
+// into regions of its own
+// (ten uneven reconstructions, gather: 1 wave 2.80 ms, 2: 2.02, 4: 1.66, 8:
+// 1.93; 32 of them 6.15 / 5.11 / 4.86 / 5.65; three small ones seen through
+// large images 2.09 / 1.19 / 0.75 / 0.64)
+constexpr int kGatherWaves = 4;
 // copies of the level-1 region, lane l adding into copy l % kL1Copies: the
 // level-1 cells are 8 times the volume of level 0's, so neighbouring pixels'
 // samples often hit the same cell, and same-address LDS atomics of one
 // instruction serialize; the copies are summed in a fixed order at the store
 constexpr int kL1Copies = 4;
 constexpr int kL1Stride = kBlockVox / 8 + 1;  // odd: the copies start on different banks
-// the same for the block's own level: one copy (two, twice the LDS and the
+// the block's own level: one copy a wave (two, twice the LDS and the
 // clearing, measured 5.05 ms against 4.74 for the c4 gathers)
-constexpr int kL0Copies = 1;
 constexpr int kL0Stride = kBlockVox + 1;
 
 // add a sample's level tap to the block region acc (block W x H x Z with
@@ -578,17 +578,19 @@ __device__ __forceinline__ bool inside_level(float qx, float qy, float qz, Dims3
 // R at level m (PAIR: levels 0 and 1), with the block shape WX x WY x WZ as
 // compile-time constants (index arithmetic and bounds on immediates).
 template <bool PAIR, int WX, int WY, int WZ>
-__device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, int wave, int lane, lds_f64* accs,
-                                            lds_f64* acc, lds_f64* acc1s, lds_f64* acc1) {
-  constexpr int kVox = kL0Copies * kL0Stride + (PAIR ? kL1Copies * kL1Stride : 0);
+__device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, int wave, int lane, lds_f64* all) {
+  constexpr int kVox = kL0Stride + (PAIR ? kL1Copies * kL1Stride : 0);
+  lds_f64* acc = all + wave * kVox;                                     // this wave's block cells
+  lds_f64* acc1s = acc + kL0Stride;                                     // PAIR: the level-1 cells' copies
+  lds_f64* acc1 = acc1s + (threadIdx.x % kL1Copies) * kL1Stride;        // this lane's copy
   const Dims3 dm = R.mt.dims[m];
   const bool two = PAIR && R.mt.levels > 0;
   const Dims3 d1 = R.mt.dims[two ? 1 : 0];
   const int nbx = (dm.x + WX - 1) / WX, nby = (dm.y + WY - 1) / WY, nbz = (dm.z + WZ - 1) / WZ;
-  const int blk = (item - R.pass_item0[kGatherPass + m]) * kGatherWaves + wave;
-  const bool live = m <= R.mt.levels && blk < nbx * nby * nbz;  // other waves only join the barriers
+  const int blk = item - R.pass_item0[kGatherPass + m];
   const int x0 = (blk % nbx) * WX, y0 = ((blk / nbx) % nby) * WY, z0 = (blk / (nbx * nby)) * WZ;
-  for (int k = lane; k < kVox; k += 64) accs[k] = 0.0;
+  for (int k = lane; k < kVox; k += 64) acc[k] = 0.0;
+  int turn = wave;  // pixel batches, counted through the views, until this wave's next one
   // support box (object space) of the block's cells; PAIR: of its level-1 cells
   const int mb = two ? 1 : m;
   const float s2 = (float)(1 << mb), sc = 1.f / (float)(1 << m);
@@ -603,7 +605,7 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
   const float lmaxf = (float)R.mt.levels;
   const int per_view = R.tiles_x * R.tiles_y;
   const float4* __restrict__ recv = reinterpret_cast<const float4*>(R.records);
-  for (int vi = 0; vi < R.num_views && live; ++vi) {
+  for (int vi = 0; vi < R.num_views; ++vi) {
     if (!PAIR && __int_as_float(R.lodmax[vi]) <= (float)(m - 1)) continue;  // no sample reads level m
     const ColumnView& cv = R.view[vi];
     const float* A = cv.pmv;
@@ -630,30 +632,34 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
     }
     if (xs > xe || ys > ye) continue;
     const int nxr = xe - xs + 1, cnt = nxr * (ye - ys + 1);
-    // lane k of the box's row-major pixel list; the next record (k + 64) is
-    // loaded while the current one is walked
-    const int dy64 = 64 / nxr, dx64 = 64 - dy64 * nxr;
-    int px = xs + lane % nxr, py = ys + lane / nxr;
+    // this lane's first place in the box's row-major pixel list; its next
+    // record (64 kGatherWaves on) is loaded while the current one is walked
+    constexpr int kStride = 64 * kGatherWaves;
+    const int first = turn * 64 + lane;
+    turn -= (cnt + 63) / 64 % kGatherWaves;
+    turn += turn < 0 ? kGatherWaves : 0;
+    const int dys = kStride / nxr, dxs = kStride - dys * nxr;
+    int px = xs + first % nxr, py = ys + first / nxr;
     auto rec_at = [&](int qx, int qy, int& it, int& slot) {
       it = vi * per_view + (qy / kTileH) * R.tiles_x + qx / kTileW;
       slot = (qy % kTileH) * kTileW + qx % kTileW;
     };
     int it_n = 0, slot_n = 0;
     float4 rec_n = make_float4(__int_as_float(1), __int_as_float(0), 0.f, 0.f);
-    if (lane < cnt) {
+    if (first < cnt) {
       rec_at(px, py, it_n, slot_n);
       rec_n = recv[(size_t)it_n * kTilePix + slot_n];
     }
-    for (int k = lane; k < cnt; k += 64) {
+    for (int k = first; k < cnt; k += kStride) {
       const float4 rec = rec_n;
       const int it = it_n, slot = slot_n, cpx = px, cpy = py;
-      px += dx64;
-      py += dy64;
+      px += dxs;
+      py += dys;
       if (px > xe) {
         px -= nxr;
         ++py;
       }
-      if (k + 64 < cnt) {
+      if (k + kStride < cnt) {
         rec_at(px, py, it_n, slot_n);
         rec_n = recv[(size_t)it_n * kTilePix + slot_n];
       }
@@ -709,13 +715,13 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
     }
   }
   __syncthreads();
-  if (live && PAIR) {
+  if (PAIR) {
     // the density gradient: g_0 + sum_l 8^-l g_l(ancestor), level 1 from
-    // this wave's region (the level-1 cells over the block), levels 2 and 3
+    // the block's regions (the level-1 cells over the block), levels 2 and 3
     // from their gathers, which ran before; each level's value rounded to
     // float and accumulated by fma from level 1 up
     const int W1 = WX / 2, H1 = WY / 2;
-    for (int k = lane; k < kBlockVox; k += 64) {
+    for (int k = threadIdx.x; k < kBlockVox; k += 64 * kGatherWaves) {
       const int lx = k % WX, ly = (k / WX) % WY, lz = k / (WX * WY);
       const int x = x0 + lx, y = y0 + ly, z = z0 + lz;
       if (x >= dm.x || y >= dm.y || z >= dm.z) continue;
@@ -728,9 +734,11 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
           float gl;
           if (l == 1) {
             const int c1 = (lx >> 1) + W1 * ((ly >> 1) + H1 * (lz >> 1));
-            double t1 = acc1s[c1];
+            double t1 = 0.0;
 #pragma unroll
-            for (int c = 1; c < kL1Copies; ++c) t1 += acc1s[c * kL1Stride + c1];
+            for (int w = 0; w < kGatherWaves; ++w)
+#pragma unroll
+              for (int c = 0; c < kL1Copies; ++c) t1 += all[w * kVox + kL0Stride + c * kL1Stride + c1];
             gl = (float)t1;
           } else {
             gl = grad_cells(R, l)[pad_index(px + 1, py + 1, pz + 1, o)];
@@ -738,12 +746,12 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
           g = fmaf(s, gl, g);
         }
       }
-      double t0 = accs[k];
+      double t0 = all[k];
 #pragma unroll
-      for (int c = 1; c < kL0Copies; ++c) t0 += accs[c * kL0Stride + k];
+      for (int w = 1; w < kGatherWaves; ++w) t0 += all[w * kVox + k];
       R.grad[flat3(x, y, z, dm)] = (float)t0 + g;
     }
-    if (blk == 0) {
+    if (blk == 0 && wave == 0) {
       // the reconstruction's loss: lane-strided sums of its per-tile
       // partials, then a butterfly over the wave (a fixed order)
       const int np = R.num_views * R.tiles_x * R.tiles_y;
@@ -752,14 +760,14 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
       for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
       if (lane == 0) R.loss[0] = t * R.loss_scale;
     }
-  } else if (live) {
+  } else {
     float* __restrict__ gout = grad_cells(R, m);
-    for (int k = lane; k < kBlockVox; k += 64) {
+    for (int k = threadIdx.x; k < kBlockVox; k += 64 * kGatherWaves) {
       const int x = x0 + k % WX, y = y0 + (k / WX) % WY, z = z0 + k / (WX * WY);
       if (x >= dm.x || y >= dm.y || z >= dm.z) continue;
-      double t0 = accs[k];
+      double t0 = all[k];
 #pragma unroll
-      for (int c = 1; c < kL0Copies; ++c) t0 += accs[c * kL0Stride + k];
+      for (int w = 1; w < kGatherWaves; ++w) t0 += all[w * kVox + k];
       gout[pad_index(x + 1, y + 1, z + 1, dm)] = (float)t0;
     }
   }
@@ -767,23 +775,21 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
 }
 
 template <bool PAIR>
-__global__ __launch_bounds__(256) void k_batch_gather(const BatchRec* __restrict__ recs, int nrec, int m,
-                                                      int total_items) {
-  constexpr int kVox = kL0Copies * kL0Stride + (PAIR ? kL1Copies * kL1Stride : 0);
-  __shared__ double region[kGatherWaves][kVox];
+__global__ __launch_bounds__(64 * kGatherWaves) void k_batch_gather(const BatchRec* __restrict__ recs, int nrec, int m,
+                                                                    int total_items) {
+  constexpr int kVox = kL0Stride + (PAIR ? kL1Copies * kL1Stride : 0);
+  __shared__ double region[kGatherWaves * kVox];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  lds_f64* accs = (lds_f64*)region[wave];                        // the block's cells' copies
-  lds_f64* acc = accs + (threadIdx.x % kL0Copies) * kL0Stride;    // this lane's copy
-  lds_f64* acc1s = accs + kL0Copies * kL0Stride;                  // PAIR: the level-1 cells' copies
-  lds_f64* acc1 = acc1s + (threadIdx.x % kL1Copies) * kL1Stride;  // this lane's copy
-  int r = -1;
-  for (int item = blockIdx.x; item < total_items; item += gridDim.x) {
-    r = rec_from(recs, nrec, item, kGatherPass + m, r);
-    const BatchRec& R = recs[r];
+  lds_f64* all = (lds_f64*)region;
+  for (int at = blockIdx.x; at < total_items; at += gridDim.x) {
+    // from the table's end: the blocks with the most work (see gather_load)
+    // start first and the light ones fill the launch's tail
+    const int item = total_items - 1 - at;
+    const BatchRec& R = recs[rec_of(recs, nrec, item, kGatherPass + m)];
     // the reconstruction's block shape (bricks 0, 1, 2: 16x16x2, 8x8x8, 16x8x4)
-    if (R.bd == 2) gather_item<PAIR, 16, 16, 2>(R, m, item, wave, lane, accs, acc, acc1s, acc1);
-    else if (R.bd == 8) gather_item<PAIR, 8, 8, 8>(R, m, item, wave, lane, accs, acc, acc1s, acc1);
-    else gather_item<PAIR, 16, 8, 4>(R, m, item, wave, lane, accs, acc, acc1s, acc1);
+    if (R.bd == 2) gather_item<PAIR, 16, 16, 2>(R, m, item, wave, lane, all);
+    else if (R.bd == 8) gather_item<PAIR, 8, 8, 8>(R, m, item, wave, lane, all);
+    else gather_item<PAIR, 16, 8, 4>(R, m, item, wave, lane, all);
   }
 }
 
@@ -845,8 +851,7 @@ static int pass_items(const MipTable& mt, int bw, int bh, int bd, int p) {
   const int m = p - kGatherPass;
   if (m > mt.levels || m == 1) return 0;  // level 1 is gathered with level 0
   const Dims3 d = mt.dims[m];
-  const int64_t blocks = (int64_t)((d.x + bw - 1) / bw) * ((d.y + bh - 1) / bh) * ((d.z + bd - 1) / bd);
-  return (int)((blocks + kGatherWaves - 1) / kGatherWaves);  // a block per wave
+  return (int)((int64_t)((d.x + bw - 1) / bw) * ((d.y + bh - 1) / bh) * ((d.z + bd - 1) / bd));
 }
 
 static int batch_layout(int32_t n, const gft_batch_recon* rs, int32_t num_mipmaps, BatchLayout& L) {
@@ -902,6 +907,32 @@ static int batch_layout(int32_t n, const gft_batch_recon* rs, int32_t num_mipmap
   }
   L.total = off;
   return GFT_OK;
+}
+
+// Pixels that look through one cell at the grid's centre, summed over the
+// views: the work of one gather block goes with it. The table holds the
+// reconstructions in its increasing order: the forward, whose items grow with
+// the grid and so mostly against it, takes the table from the front, the
+// gather from the back, both with their long items first.
+static double gather_load(const gft_batch_recon& c) {
+  const Mat4d m = mat_from_colmajor(c.M);
+  const double x = 0.5 * c.grid_dhw[2], y = 0.5 * c.grid_dhw[1], z = 0.5 * c.grid_dhw[0];
+  double load = 0.0;
+  for (int v = 0; v < c.num_views; ++v) {
+    const Mat4d A = mat_mul(mat_from_colmajor(c.P + 16 * v), mat_mul(mat_from_colmajor(c.V + 16 * v), m));
+    auto row = [&](int r) { return A.m[r] * x + A.m[4 + r] * y + A.m[8 + r] * z + A.m[12 + r]; };
+    const double cx = row(0), cy = row(1), cw = row(3);
+    double gx[3], gy[3];  // the pixel coordinates' derivatives along the grid's axes
+    for (int a = 0; a < 3; ++a) {
+      gx[a] = 0.5 * c.output_shape[2] * (A.m[4 * a] * cw - cx * A.m[4 * a + 3]) / (cw * cw);
+      gy[a] = 0.5 * c.output_shape[1] * (A.m[4 * a + 1] * cw - cy * A.m[4 * a + 3]) / (cw * cw);
+    }
+    const double n0 = gx[1] * gy[2] - gx[2] * gy[1], n1 = gx[2] * gy[0] - gx[0] * gy[2],
+                 n2 = gx[0] * gy[1] - gx[1] * gy[0];
+    const double area = std::sqrt(n0 * n0 + n1 * n1 + n2 * n2);
+    if (std::isfinite(area)) load += area;
+  }
+  return load;
 }
 
 // item counts of the launches: render items; the level passes (bordered
@@ -974,11 +1005,18 @@ int gft_batch_render_prepare(void* stream, int32_t n, const gft_batch_recon* rec
   std::vector<BatchRec> recs(n);
   char* ws = (char*)workspace;
   int item = 0, pass_item[kBatchPasses] = {};
+  std::vector<std::pair<double, int>> order(n);
   for (int r = 0; r < n; ++r) {
     const gft_batch_recon& c = recons[r];
     if (!c.density || !c.targets || !c.images || !c.density_grad || !c.loss || !c.M || !c.V || !c.P || !c.frustum)
       return fail(GFT_ERR_INVALID_ARGUMENT, "reconstruction %d: null pointer argument", r);
-    BatchRec& R = recs[r];
+    order[r] = {gather_load(c), r};
+  }
+  std::sort(order.begin(), order.end());
+  for (int at = 0; at < n; ++at) {
+    const int r = order[at].second;
+    const gft_batch_recon& c = recons[r];
+    BatchRec& R = recs[at];
     std::memset(&R, 0, sizeof(R));
     const Dims3 d{c.grid_dhw[2], c.grid_dhw[1], c.grid_dhw[0]};
     R.mt = batch_mip_table(d, num_mipmaps);

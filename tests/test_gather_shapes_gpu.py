@@ -49,3 +49,31 @@ def test_render_gather_block_rules(cuda, grid, image, views, lit):
     assert norm_err(gd.cpu().numpy(), rd) < 1e-4
     _, gd2, gl2 = grads()
     assert torch.equal(gd, gd2) and (not lit or torch.equal(gl, gl2))
+
+
+@pytest.mark.parametrize("brick", [0, 1, 2])
+def test_batch_gather_shared_blocks(cuda, brick):
+    """The batched gather's waves share a block's pixels: reconstructions with
+    fewer pixel batches than waves, with many (a small grid in large images) and
+    out of the table's cost order, each against the FP64 oracle."""
+    from gft.batch import BatchedRenderStep
+    specs = [((20, 33, 18), (50, 40), 2), ((5, 6, 7), (90, 70), 3), ((17, 16, 31), (4, 5), 8)]
+    recons, dens, tgts = [], [], []
+    for k, (grid, image, views) in enumerate(specs):
+        sc = scene(grid=grid, image=image, views=views, seed=90 + k)
+        recons.append(dict(grid=grid, M=sc["M"], V=sc["V"], P=sc["P"], F=sc["F"], out_dhw=sc["out_dhw"],
+                           depth_step=sc["step"], brick=brick))
+        dens.append(sc["data"])
+        tgts.append(np.random.Generator(np.random.PCG64(k)).uniform(0, 0.5, size=(views,) + image + (3,)))
+    b = BatchedRenderStep(recons, num_mipmaps=3)
+    b.bind([_t(d) for d in dens], [_t(t) for t in tgts])
+    b.run()
+    torch.cuda.synchronize()
+    first = [g.clone() for g in b.grads]
+    b.run()
+    torch.cuda.synchronize()
+    for r, d, t, g, g0 in zip(recons, dens, tgts, b.grads, first):
+        ref = orc.mip_render_fwd_bwd(d, t.astype(np.float32), r["M"], r["V"], r["P"], r["F"], r["out_dhw"],
+                                     r["depth_step"], num_mipmaps=3)
+        assert norm_err(g.cpu().numpy(), ref["gd"]) < 1e-4
+        assert torch.equal(g, g0)
