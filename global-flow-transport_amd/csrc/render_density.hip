@@ -673,16 +673,21 @@ __global__ __launch_bounds__(64 * NW) void k_render_density_bwd_gather(RenderSav
 // sample (the index->object map is projective), so their trilinear corners fit
 // in an axis-aligned brick; the scatter is accumulated there with LDS atomics
 // and flushed once per segment with coalesced global atomics (zero entries
-// skipped). A brick over the LDS capacity, or a corner outside the brick
-// through rounding, goes straight to a global atomic.
+// skipped). A brick over the LDS capacity goes straight to global atomics.
 constexpr int kSegK = 8;
 constexpr int kCap = 6144;  // FP64 brick cells: ds_add_f64 is ~20x faster than ds_add_f32 on gfx950
+// more than any rounding of a sample's position against the corner rays'
+constexpr float kBrickSlack = 1e-2f;
 
 struct Brick {
-  int lo[3], n[3];
-  int size;
+  int lo[3], n[3];  // first cell, cells: every floor corner in [lo, lo + n - 2], its upper corner one on
+  int size;         // 0: no sample of the segment reaches the grid
 };
 
+// The segment's floor corners, of positions clamped into the grid (CLAMP) or of
+// the samples inside it (BORDER: floor -1 to dims - 1); cells outside the grid
+// take part as a rim that the flush drops.
+template <int BM>
 __device__ __forceinline__ Brick segment_brick(const float3* cn, const float3* cs, int ia, int ib, Dims3 d) {
   float mn[3] = {3.4e38f, 3.4e38f, 3.4e38f}, mx[3] = {-3.4e38f, -3.4e38f, -3.4e38f};
 #pragma unroll
@@ -704,12 +709,18 @@ __device__ __forceinline__ Brick segment_brick(const float3* cn, const float3* c
   b.size = 1;
 #pragma unroll
   for (int a = 0; a < 3; ++a) {
-    // every corner index is clamp(floor(p)) or clamp(floor(p)+1)
-    const int lo = clampi((int)floorf(mn[a] - 1e-3f), 0, dim[a] - 1);
-    const int hi = clampi((int)floorf(mx[a] + 1e-3f) + 1, 0, dim[a] - 1);
+    int lo = (int)floorf(fminf(fmaxf(mn[a] - kBrickSlack, -2.f), (float)dim[a] + 1.f));
+    int hi = (int)floorf(fminf(fmaxf(mx[a] + kBrickSlack, -2.f), (float)dim[a] + 1.f));
+    if (BM == B_CLAMP) {
+      lo = clampi(lo, 0, dim[a] - 1);
+      hi = clampi(hi, 0, dim[a] - 1);
+    } else {
+      lo = max(lo, -1);
+      hi = min(hi, dim[a] - 1);
+    }
     b.lo[a] = lo;
-    b.n[a] = hi - lo + 1;
-    b.size *= b.n[a];
+    b.n[a] = hi - lo + 2;
+    b.size = hi < lo ? 0 : b.size * b.n[a];
   }
   return b;
 }
@@ -718,6 +729,15 @@ __device__ __forceinline__ Brick segment_brick(const float3* cn, const float3* c
 // forward's copy): a segment's 8 samples are read with all their loads in
 // flight, and give the forward's sigma_i bit for bit (the same corners,
 // weights and lerp order).
+// The scatter of a CLAMP sample is that of its position clamped into the grid:
+// along an axis where the sample lies outside, the boundary cell gets weight 1
+// and the next one weight 0. Most of a CLAMP ray's samples lie outside along
+// some axis, often a whole wave's, so the upper corners of an axis are left
+// out where no lane of the wave has a weight there.
+// The kernel is bound by VALU work (half its cycles) and LDS atomics (0.4)
+// together at 12 waves a CU; 128x224x128, 5 views of 256x456: 0.912 ms, 1.060
+// with a bounds test per corner and a flush per segment; segments of 4, 5, 6 or
+// 12 samples and bricks of 3072 to 8192 cells: 0.95 to 2.6 ms.
 // BORDER (the recompute alternative to the saved-state gather: nothing is
 // kept from the forward but the images) walks only the segments of the
 // tile's clipped sample ranges; samples outside the grid read 0 and corners
@@ -731,6 +751,8 @@ __global__ __launch_bounds__(256) void k_render_density_bwd_clamp(const float4* 
                                                                   RayDims rd, RayLaunch L, RenderParams rp) {
   __shared__ double lg[kCap];
   __shared__ int seg_range[2];
+  typedef __attribute__((address_space(3))) double lds_double;
+  lds_double* brick = (lds_double*)lg;
   const RayView& v = L.view[blockIdx.z];
   const int x0 = blockIdx.x * kRTileX, y0 = blockIdx.y * kRTileY;
   const int x = x0 + (threadIdx.x % kRTileX), y = y0 + (threadIdx.x / kRTileX);
@@ -752,6 +774,7 @@ __global__ __launch_bounds__(256) void k_render_density_bwd_clamp(const float4* 
   const bool walk = active && (G != 0.f || gD != 0.f);
   for (int i = threadIdx.x; i < kCap; i += 256) lg[i] = 0.0;
   const int S = rd.out_d;
+  const float mx = (float)(rd.in.x - 1), my = (float)(rd.in.y - 1), mz = (float)(rd.in.z - 1);
   int sg_lo = 0, sg_hi = (S + kSegK - 1) / kSegK - 1;
   if (BM == B_BORDER) {
     // the union of the tile's clipped ranges, in whole segments
@@ -773,10 +796,48 @@ __global__ __launch_bounds__(256) void k_render_density_bwd_clamp(const float4* 
   } else {
     __syncthreads();
   }
+  // adds the brick's sums to the gradient and clears it (every thread of the workgroup)
+  auto flush = [&](const Brick& br) {
+    if (br.size == 0 || br.size > kCap) return;
+    __syncthreads();
+    const int nx = br.n[0], ny = br.n[1];
+    const int q = 256 / nx, r = 256 - q * nx;
+    int bx = threadIdx.x % nx, t = threadIdx.x / nx;
+    int by = t % ny, bz = t / ny;
+    for (int idx = threadIdx.x; idx < br.size; idx += 256) {
+      const float val = (float)lg[idx];
+      if (val != 0.f) {
+        const int cx = br.lo[0] + bx, cy = br.lo[1] + by, cz = br.lo[2] + bz;
+        if (((unsigned)cx < (unsigned)rd.in.x) & ((unsigned)cy < (unsigned)rd.in.y) & ((unsigned)cz < (unsigned)rd.in.z))
+          atomic_addf(gout + flat3(cx, cy, cz, rd.in), val);
+      }
+      lg[idx] = 0.0;
+      bx += r;
+      by += q;
+      if (bx >= nx) {
+        bx -= nx;
+        ++by;
+      }
+      while (by >= ny) {
+        by -= ny;
+        ++bz;
+      }
+    }
+    __syncthreads();
+  };
+  // consecutive segments often share a brick (all their samples clamp to the
+  // same boundary cells): it is flushed when the next one differs
+  Brick held{};
   for (int sgi = sg_hi; sgi >= sg_lo; --sgi) {
     const int ia = sgi * kSegK, ib = min(ia + kSegK, S) - 1;
-    const Brick br = segment_brick(cn, cs, ia, ib, rd.in);
-    const bool use_lds = br.size <= kCap;
+    const Brick br = segment_brick<BM>(cn, cs, ia, ib, rd.in);
+    const bool use_lds = br.size > 0 && br.size <= kCap;
+    if (br.lo[0] != held.lo[0] || br.lo[1] != held.lo[1] || br.lo[2] != held.lo[2] || br.n[0] != held.n[0] ||
+        br.n[1] != held.n[1] || br.n[2] != held.n[2]) {
+      flush(held);
+      held = br;
+    }
+    const int sy = br.n[0], sz = br.n[0] * br.n[1];
     if (walk) {
       float val[kSegK];
       bool inr[kSegK];
@@ -785,70 +846,59 @@ __global__ __launch_bounds__(256) void k_render_density_bwd_clamp(const float4* 
       for (int u = 0; u < kSegK; ++u) {
         const int i = ib - u;
         if (i < ia) break;
-        const float fi = (float)i;
-        const Taps tp = make_taps<BM>(fmaf(fi, step.x, nearp.x) - 0.5f, fmaf(fi, step.y, nearp.y) - 0.5f,
-                                      fmaf(fi, step.z, nearp.z) - 0.5f, rd.in);
         const float sigma = rp.step * val[u];
         const float e = __expf(-D);
         D = fmaxf(D - sigma, 0.f);
         const float esg = e * sigma * G;
-        const float gds = rp.step * (e * G + (gD - esg));
+        const float g = rp.step * (e * G + (gD - esg));
         gD -= esg;
         if (BM == B_BORDER && !inr[u]) continue;  // outside the grid: no gradient
-        float wx[2] = {1.f - tp.wx, tp.wx}, wy[2] = {1.f - tp.wy, tp.wy}, wz[2] = {1.f - tp.wz, tp.wz};
+        const float fi = (float)i;
+        float px = fmaf(fi, step.x, nearp.x) - 0.5f, py = fmaf(fi, step.y, nearp.y) - 0.5f,
+              pz = fmaf(fi, step.z, nearp.z) - 0.5f;
         if (BM == B_CLAMP) {
-          // an axis whose two corners clamp to one cell (the sample lies outside
-          // the grid, or in the last half cell, along it) gives that cell both
-          // weights: one tap of weight 1 instead of two. Most of a CLAMP ray's
-          // samples lie outside the grid and would otherwise spend 8 atomics on
-          // 4, 2 or 1 distinct cells.
-          if (tp.ix[0] == tp.ix[1]) { wx[0] = 1.f; wx[1] = 0.f; }
-          if (tp.iy[0] == tp.iy[1]) { wy[0] = 1.f; wy[1] = 0.f; }
-          if (tp.iz[0] == tp.iz[1]) { wz[0] = 1.f; wz[1] = 0.f; }
+          px = __builtin_amdgcn_fmed3f(px, 0.f, mx);
+          py = __builtin_amdgcn_fmed3f(py, 0.f, my);
+          pz = __builtin_amdgcn_fmed3f(pz, 0.f, mz);
         }
+        const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
+        const float tx = px - fx, ty = py - fy, tz = pz - fz;
+        const float ux = 1.f - tx, uy = 1.f - ty, uz = 1.f - tz;
+        const bool hx = __ballot(tx != 0.f) != 0, hy = __ballot(ty != 0.f) != 0, hz = __ballot(tz != 0.f) != 0;
+        // (a gradient that is not finite takes the exact corner test below: its product with a weight of 0 is not 0)
+        if (use_lds && __ballot(!(fabsf(g) < 3.4e38f)) == 0) {
+          const int lx = clampi((int)fx - br.lo[0], 0, br.n[0] - 2), ly = clampi((int)fy - br.lo[1], 0, br.n[1] - 2),
+                    lz = clampi((int)fz - br.lo[2], 0, br.n[2] - 2);
+          lds_double* at = brick + (__mul24(lz, sz) + __mul24(ly, sy) + lx);
+          const float gz[2] = {g * uz, g * tz};
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
+          for (int k = 0; k < 2; ++k) {
+            if (k && !hz) break;
 #pragma unroll
-          for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int ii = 0; ii < 2; ++ii) {
-              const float w = wx[ii] * wy[j] * wz[k];
-              if (w == 0.f) continue;
-              if (BM == B_BORDER && !(tp.vx[ii] & tp.vy[j] & tp.vz[k])) continue;
-              const int bx = tp.ix[ii] - br.lo[0], by = tp.iy[j] - br.lo[1], bz = tp.iz[k] - br.lo[2];
-              const bool in = use_lds & ((unsigned)bx < (unsigned)br.n[0]) & ((unsigned)by < (unsigned)br.n[1]) &
-                              ((unsigned)bz < (unsigned)br.n[2]);
-              if (in) atomicAdd(&lg[(bz * br.n[1] + by) * br.n[0] + bx], (double)(gds * w));
-              else atomic_addf(gout + flat3(tp.ix[ii], tp.iy[j], tp.iz[k], rd.in), gds * w);
+            for (int j = 0; j < 2; ++j) {
+              if (j && !hy) break;
+              const float w = gz[k] * (j ? ty : uy);
+              lds_double* row = at + (k ? sz : 0) + (j ? sy : 0);
+              __hip_atomic_fetch_add(row, (double)(w * ux), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+              if (hx)
+                __hip_atomic_fetch_add(row + 1, (double)(w * tx), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
-      }
-    }
-    if (use_lds) {
-      __syncthreads();
-      const int nx = br.n[0], ny = br.n[1];
-      const int q = 256 / nx, r = 256 - q * nx;
-      int bx = threadIdx.x % nx, t = threadIdx.x / nx;
-      int by = t % ny, bz = t / ny;
-      for (int idx = threadIdx.x; idx < br.size; idx += 256) {
-        const float val = (float)lg[idx];
-        if (val != 0.f) {
-          atomic_addf(gout + flat3(br.lo[0] + bx, br.lo[1] + by, br.lo[2] + bz, rd.in), val);
-          lg[idx] = 0.0;
-        }
-        bx += r;
-        by += q;
-        if (bx >= nx) {
-          bx -= nx;
-          ++by;
-        }
-        while (by >= ny) {
-          by -= ny;
-          ++bz;
+          }
+        } else {
+#pragma unroll
+          for (int k = 0; k < 8; ++k) {
+            const float w = (k & 1 ? tx : ux) * (k & 2 ? ty : uy) * (k & 4 ? tz : uz);
+            const int cx = (int)fx + (k & 1), cy = (int)fy + ((k >> 1) & 1), cz = (int)fz + (k >> 2);
+            if (w == 0.f || (unsigned)cx >= (unsigned)rd.in.x || (unsigned)cy >= (unsigned)rd.in.y ||
+                (unsigned)cz >= (unsigned)rd.in.z)
+              continue;
+            atomic_addf(gout + flat3(cx, cy, cz, rd.in), g * w);
+          }
         }
       }
-      __syncthreads();
     }
   }
+  flush(held);
   if (L2) block_loss(sq, loss, rp.loss_scale);
 }
 

@@ -77,3 +77,25 @@ def test_batch_gather_shared_blocks(cuda, brick):
                                      r["depth_step"], num_mipmaps=3)
         assert norm_err(g.cpu().numpy(), ref["gd"]) < 1e-4
         assert torch.equal(g, g0)
+
+
+@pytest.mark.parametrize("boundary", ["CLAMP", "BORDER"])
+@pytest.mark.parametrize("grid,image,views", [((1, 5, 1), (20, 18), 2), ((33, 20, 47), (70, 35), 3),
+                                              ((9, 70, 12), (33, 50), 5)])
+def test_scatter_walk_bricks(cuda, boundary, grid, image, views):
+    """The recompute walk's scatter: one-cell axes, tiles whose segments share a
+    brick, rim cells outside the grid (BORDER), ragged tiles; FP64 oracle 1e-4."""
+    from gft.pipeline import TransportRenderStep
+    sc = scene(grid=grid, image=image, views=views, seed=sum(grid))
+    tgt = np.random.Generator(np.random.PCG64(1)).uniform(0, 0.5, size=(1, views) + image + (3,)).astype(np.float32)
+    step = TransportRenderStep(grid, sc["M"], sc["V"], sc["P"], sc["F"], sc["out_dhw"], sc["step"], boundary=boundary,
+                               reduction="scatter", order=1)
+    d, v = _t(sc["data"]), torch.zeros((1,) + grid + (3,), device="cuda")
+    loss, gd, _ = step.run(d, v, _t(tgt))
+    torch.cuda.synchronize()
+    img = step.images.cpu().numpy()
+    rl, gimg = orc.l2_loss_and_grad(img.astype(np.float64), tgt)
+    ref = orc.render_density_bwd(sc["data"], img, gimg, sc["M"], sc["V"], sc["P"], sc["F"], sc["out_dhw"], sc["step"],
+                                 boundary=boundary)
+    assert norm_err(gd.cpu().numpy(), ref) < 1e-4
+    assert abs(loss.item() - rl) <= 1e-5 * rl
