@@ -10,8 +10,9 @@ namespace gft {
 
 
 hipError_t fill_launch(hipStream_t s, float* p, size_t n, float v);
-hipError_t mip_down_launch(int C, hipStream_t st, const float* src, size_t src_stride, Dims3 s, float* dst,
-                           size_t dst_stride, Dims3 o, int batches, float scale);
+hipError_t mip_down_launch(hipStream_t st, const float* src, size_t src_stride, const MipTable& mt, int first, int n,
+                           float* atlas, int batches, float scale);
+int mip_levels_per_launch();
 hipError_t mip_collapse_launch(int C, hipStream_t st, const float* gp, size_t gp_stride, Dims3 o, float* gc,
                                size_t gc_stride, Dims3 s, int batches);
 hipError_t sample_transform_launch(int C, int bm, bool sum, hipStream_t st, const float* in, const float* atlas,
@@ -28,7 +29,7 @@ hipError_t shadow_fwd_launch(int bm, int fm, int bl, hipStream_t st, const float
 hipError_t shadow_bwd_launch(int bm, int bl, hipStream_t st, const float* saved, const float* gt, const float* mask,
                              Dims3 dout, float* gs);
 hipError_t sample_transform_gather_launch(int C, bool ref, int fm, hipStream_t st, const float* og, Dims3 din,
-                                          Dims3 dout, const SampleLaunch& L, const SampleLaunch& Linv, int accumulate,
+                                          Dims3 dout, const SampleLaunch& L, const ReverseLaunch& Linv, int accumulate,
                                           float* grad);
 hipError_t normalize_count_launch(int C, hipStream_t st, float* grad, const unsigned* cnt, size_t nvox);
 hipError_t sample_lut_launch(int C, int bm, hipStream_t st, const float* in, const float* atlas, const MipTable& mt,
@@ -79,11 +80,11 @@ static size_t atlas_bytes(Dims3 d, int C, int levels, int batches) {
 // grid's values as they are read (the pyramid of base * base_scale).
 static hipError_t build_atlas(hipStream_t st, const float* base, const MipTable& mt, int batches, float* atlas,
                               float base_scale = 1.f) {
-  for (int m = 1; m <= mt.levels; ++m) {
-    const float* src = m == 1 ? base : atlas + mt.offset[m - 1];
-    size_t src_stride = m == 1 ? mt.base_stride : mt.atlas_stride;
-    hipError_t e = mip_down_launch(mt.C, st, src, src_stride, mt.dims[m - 1], atlas + mt.offset[m], mt.atlas_stride,
-                                   mt.dims[m], batches, m == 1 ? base_scale : 1.f);
+  for (int m = 0; m < mt.levels; m += mip_levels_per_launch()) {
+    const float* src = m == 0 ? base : atlas + mt.offset[m];
+    const size_t src_stride = m == 0 ? mt.base_stride : mt.atlas_stride;
+    hipError_t e = mip_down_launch(st, src, src_stride, mt, m, std::min(mt.levels - m, mip_levels_per_launch()), atlas,
+                                   batches, m == 0 ? base_scale : 1.f);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
@@ -133,15 +134,17 @@ static int check_transform_attrs(int32_t interpolation, int32_t boundary, int32_
   return GFT_OK;
 }
 
-// Camera records of `count` views. Forward coordinate modes need P^-1 and
-// (V M)^-1, reverse modes V M and P (transformations.hpp:44-64); the inverses
-// are formed in double precision.
+// Camera records of `count` views: the coordinate map of each (SampleView),
+// from P^-1 and (V M)^-1 (forward modes) or P and V M (reverse modes;
+// transformations.hpp:44-64,86-145). `din` is the sampled grid, `dout` the
+// output cells. The linear forms and the inverses are formed in double.
 static int build_sample_views(const std::vector<ViewPair>& pairs, size_t first, size_t count, const float* M,
-                              int m_index_override, const float* V, const float* P, const float* F, int cm,
-                              SampleLaunch& L) {
+                              int m_index_override, const float* V, const float* P, const float* F, int cm, Dims3 din,
+                              Dims3 dout, SampleLaunch& L) {
   L.num_views = (int)count;
   L.cm = cm;
   L.accumulate = 0;
+  const double od[3] = {(double)dout.x, (double)dout.y, (double)dout.z};
   for (size_t i = 0; i < count; ++i) {
     const ViewPair& vp = pairs[first + i];
     int mi = m_index_override >= 0 ? m_index_override : vp.batch;
@@ -150,22 +153,65 @@ static int build_sample_views(const std::vector<ViewPair>& pairs, size_t first, 
     Mat4d p = mat_from_colmajor(P + 16 * vp.cam);
     Mat4d mv = mat_mul(v, m);
     SampleView& sv = L.view[i];
+    sv = SampleView{};
+    sv.in_batch = vp.batch;
+    sv.out_slot = vp.slot;
+    const double p22 = P[16 * vp.cam + 4 * 2 + 2], p32 = P[16 * vp.cam + 4 * 3 + 2];
+    const double nearp = F[6 * vp.cam + 0], range = (double)F[6 * vp.cam + 1] - nearp;
+    for (int k = 0; k < 3; ++k) sv.mid[k] = (float)(0.5 * od[k]);
     if (cm == CM_LINDEPTH || cm == CM_TRANSFORM) {
       Mat4d mvinv, pinv;
       if (!mat_inverse(mv, mvinv)) return fail(GFT_ERR_INVALID_ARGUMENT, "model-view matrix is singular");
       if (!mat_inverse(p, pinv)) return fail(GFT_ERR_INVALID_ARGUMENT, "projection matrix is singular");
-      mat_to_float(pinv, sv.A);
-      mat_to_float(mvinv, sv.B);
+      // position = (mvinv vs).xyz / vs.w with vs = pinv (nx, ny, nz, 1)
+      double a[4], b[4], c[4], e[4];
+      Mat4d C = mat_mul(mvinv, pinv);
+      for (int col = 0; col < 4; ++col) C.m[4 * col + 3] = pinv.m[4 * col + 3];
+      for (int r = 0; r < 4; ++r) {
+        const double c0 = C.m[r], c1 = C.m[4 + r], c2 = C.m[8 + r], c3 = C.m[12 + r];
+        a[r] = 2.0 * c0 / od[0];
+        b[r] = 2.0 * c1 / od[1];
+        if (cm == CM_LINDEPTH) {  // nz = -p22 - p32 / s; the form is multiplied by s
+          c[r] = -p32 * c2;
+          e[r] = c3 - p22 * c2;  // (nx and ny are 0 in the middle)
+        } else {
+          c[r] = 2.0 * c2 / od[2];
+          e[r] = c3;
+        }
+      }
+      const double z1 = -range / od[2], z0 = -nearp - 0.5 * range;
+      double unit = 0.0, rest;
+      if (cm == CM_LINDEPTH) {
+        const double smax = std::fabs(z0) + std::fabs(z1) * (0.5 * od[2] + 1.0);
+        rest = (std::fabs(a[3]) * (od[0] + 1.0) + std::fabs(b[3]) * (od[1] + 1.0) + std::fabs(e[3])) * smax;
+        unit = c[3];
+      } else {
+        rest = std::fabs(a[3]) * (od[0] + 1.0) + std::fabs(b[3]) * (od[1] + 1.0) + std::fabs(c[3]) * (od[2] + 1.0);
+        unit = e[3];
+      }
+      if (std::isfinite(1.0 / unit) && rest <= 1e-10 * std::fabs(unit)) {
+        for (int r = 0; r < 4; ++r) a[r] /= unit, b[r] /= unit, c[r] /= unit, e[r] /= unit;
+        sv.unit = 1;
+      }
+      sv.z0 = (float)z0;
+      sv.z1 = (float)z1;
+      for (int r = 0; r < 4; ++r) {
+        sv.a[r] = (float)a[r];
+        sv.b[r] = (float)b[r];
+        sv.c[r] = (float)c[r];
+        sv.e[r] = (float)e[r];
+      }
     } else {
-      mat_to_float(mv, sv.A);
-      mat_to_float(p, sv.B);
+      mat_to_float(mv, sv.rev.A);
+      mat_to_float(p, sv.rev.B);
+      sv.rev.idims[0] = (float)din.x;
+      sv.rev.idims[1] = (float)din.y;
+      sv.rev.idims[2] = (float)din.z;
+      sv.rev.p22 = (float)p22;
+      sv.rev.p32 = (float)p32;
+      sv.rev.nearp = (float)nearp;
+      sv.rev.farp = F[6 * vp.cam + 1];
     }
-    sv.p22 = P[16 * vp.cam + 4 * 2 + 2];
-    sv.p32 = P[16 * vp.cam + 4 * 3 + 2];
-    sv.nearp = F[6 * vp.cam + 0];
-    sv.farp = F[6 * vp.cam + 1];
-    sv.in_batch = vp.batch;
-    sv.out_slot = vp.slot;
   }
   return GFT_OK;
 }
@@ -233,7 +279,7 @@ int gft_sample_grid_transform_fwd(void* stream, const float* input, const int64_
   for (size_t first = 0; first < pairs.size(); first += kMaxSampleViews) {
     size_t cnt = std::min(pairs.size() - first, (size_t)kMaxSampleViews);
     SampleLaunch L;
-    if ((rc = build_sample_views(pairs, first, cnt, M, -1, V, P, frustum, coordinate_mode, L))) return rc;
+    if ((rc = build_sample_views(pairs, first, cnt, M, -1, V, P, frustum, coordinate_mode, din, dout, L))) return rc;
     if ((rc = check_hip(sample_transform_launch(C, boundary, false, st, input, atlas, mt, s, dout, L, output),
                         "sample transform launch")))
       return rc;
@@ -300,9 +346,13 @@ int gft_sample_grid_transform_bwd(void* stream, const float* input, const int64_
           if (vp.batch == b) mine.push_back(vp);
         for (size_t first = 0; first < mine.size(); first += kMaxSampleViews) {
           size_t n = std::min(mine.size() - first, (size_t)kMaxSampleViews);
-          SampleLaunch L, Linv;
-          if ((rc = build_sample_views(mine, first, n, M, -1, V, P, frustum, coordinate_mode, L))) return rc;
-          if ((rc = build_sample_views(mine, first, n, M, -1, V, P, frustum, coordinate_mode ^ 1, Linv))) return rc;
+          SampleLaunch L, R;
+          ReverseLaunch Linv;
+          if ((rc = build_sample_views(mine, first, n, M, -1, V, P, frustum, coordinate_mode, din, dout, L))) return rc;
+          if ((rc = build_sample_views(mine, first, n, M, -1, V, P, frustum, coordinate_mode ^ 1, dout, din, R)))
+            return rc;
+          for (size_t k = 0; k < n; ++k) Linv.view[k] = R.view[k].rev;
+          Linv.cm = R.cm;
           if ((rc = check_hip(sample_transform_gather_launch(C, grad_mode == GFT_GRAD_REFERENCE, interpolation, st,
                                                              output_grad, din, dout, L, Linv, first > 0,
                                                              input_grad + bstride * b),
@@ -325,7 +375,7 @@ int gft_sample_grid_transform_bwd(void* stream, const float* input, const int64_
       for (size_t first = 0; first < mine.size(); first += kMaxSampleViews) {
         size_t n = std::min(mine.size() - first, (size_t)kMaxSampleViews);
         SampleLaunch L;
-        if ((rc = build_sample_views(mine, first, n, M, -1, V, P, frustum, coordinate_mode, L))) return rc;
+        if ((rc = build_sample_views(mine, first, n, M, -1, V, P, frustum, coordinate_mode, din, dout, L))) return rc;
         if ((rc = check_hip(sample_transform_scatter_ref_launch(C, boundary, st, output_grad, din, dout, L,
                                                                 input_grad + bstride * b, cnt),
                             "gradient scatter launch")))
@@ -349,7 +399,7 @@ int gft_sample_grid_transform_bwd(void* stream, const float* input, const int64_
   for (size_t first = 0; first < pairs.size(); first += kMaxSampleViews) {
     size_t n = std::min(pairs.size() - first, (size_t)kMaxSampleViews);
     SampleLaunch L;
-    if ((rc = build_sample_views(pairs, first, n, M, -1, V, P, frustum, coordinate_mode, L))) return rc;
+    if ((rc = build_sample_views(pairs, first, n, M, -1, V, P, frustum, coordinate_mode, din, dout, L))) return rc;
     if ((rc = check_hip(sample_transform_adjoint_launch(C, boundary, st, input, atlas, mt, s, dout, L, output_grad,
                                                         input_grad, gatlas),
                         "gradient adjoint launch")))
@@ -415,7 +465,7 @@ int gft_sample_grid_transform_gather_grad(void* stream, const float* output_grad
     for (size_t first = 0; first < pairs.size(); first += kMaxSampleViews) {
       size_t n = std::min(pairs.size() - first, (size_t)kMaxSampleViews);
       SampleLaunch L;
-      if ((rc = build_sample_views(pairs, first, n, M, (int)i, V, P, frustum, rev, L))) return rc;
+      if ((rc = build_sample_views(pairs, first, n, M, (int)i, V, P, frustum, rev, dfr, dvol, L))) return rc;
       L.accumulate = first > 0;
       if ((rc = check_hip(sample_transform_launch(C, boundary, true, st, output_grad, atlas, mt, s, dvol, L,
                                                   input_grad + vstride * i),
@@ -556,7 +606,9 @@ int gft_lod_transform(void* stream, const int32_t input_dhw[3], const float* MV,
   for (size_t first = 0; first < pairs.size(); first += kMaxSampleViews) {
     size_t n = std::min(pairs.size() - first, (size_t)kMaxSampleViews);
     SampleLaunch L;
-    if ((rc = build_sample_views(pairs, first, n, nullptr, -1, MV, P, frustum, cm, L))) return rc;
+    if ((rc = build_sample_views(pairs, first, n, nullptr, -1, MV, P, frustum, cm, dims_dhw(input_dhw),
+                                 dims_dhw(output_shape), L)))
+      return rc;
     if ((rc = check_hip(lod_transform_launch(st, dims_dhw(input_dhw), dims_dhw(output_shape), L, output),
                         "lod transform launch")))
       return rc;
@@ -617,7 +669,8 @@ int gft_shadow_transmission_fwd(void* stream, const float* density, const int64_
   SampleCfg cfg{interpolation, mipmapping, levels, mip_bias, 0.5f};
   std::vector<ViewPair> pairs{{0, 0, 0}};
   SampleLaunch L;
-  if ((rc = build_sample_views(pairs, 0, 1, M, -1, V, P, frustum, CM_LINDEPTH, L))) return rc;
+  if ((rc = build_sample_views(pairs, 0, 1, M, -1, V, P, frustum, CM_LINDEPTH, din, dims_dhw(shadow_shape), L)))
+    return rc;
   return check_hip(shadow_fwd_launch(boundary, interpolation, blending_mode, st, density, atlas, mt, cfg, L.view[0],
                                      dims_dhw(shadow_shape), depth_step, mask, saved, transmission),
                    "shadow transmission launch");

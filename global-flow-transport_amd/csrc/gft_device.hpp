@@ -154,31 +154,61 @@ __device__ __forceinline__ void clip_ray(float3 n, float3 st, Dims3 d, int S, fl
   }
 }
 
-// Trilinear value, lerp order x, y, z as in read3DInterpolated.
+// Trilinear value, lerp order x, y, z as in read3DInterpolated. Where every
+// lane's 8 corners lie in the grid (most waves) they are read from one base
+// address without clamping or corner tests; the values are the same.
 template <int C, int BM>
 __device__ __forceinline__ Vec<C> read_linear(const float* __restrict__ buf, Dims3 d, float px, float py, float pz) {
-  Taps t = make_taps<BM>(px, py, pz, d);
-  Vec<C> r = vzero<C>();
-  if (BM == B_BORDER && !t.inside) return r;
   Vec<C> c[2][2][2];
+  float wx, wy, wz;
+  if constexpr (BM == B_BORDER) {
+    const float qx = px + 0.5f, qy = py + 0.5f, qz = pz + 0.5f;
+    if (!((0.f <= qx) & (qx < (float)d.x) & (0.f <= qy) & (qy < (float)d.y) & (0.f <= qz) & (qz < (float)d.z)))
+      return vzero<C>();
+  }
+  const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
+  const int ix = (int)fx, iy = (int)fy, iz = (int)fz;
+  const bool inner = ((unsigned)ix < (unsigned)(d.x - 1)) & ((unsigned)iy < (unsigned)(d.y - 1)) &
+                     ((unsigned)iz < (unsigned)(d.z - 1));
+  if (__ballot(!inner) == 0) {
+    wx = px - fx;
+    wy = py - fy;
+    wz = pz - fz;
+    const float* p = buf + flat3(ix, iy, iz, d) * C;
+    const size_t row = (size_t)d.x * C, slice = row * d.y;
 #pragma unroll
-  for (int k = 0; k < 2; ++k)
+    for (int k = 0; k < 2; ++k)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        c[k][j][i] = vload<C>(buf, flat3(t.ix[i], t.iy[j], t.iz[k], d));
-        if (BM == B_BORDER && !(t.vx[i] & t.vy[j] & t.vz[k])) c[k][j][i] = vzero<C>();
+      for (int j = 0; j < 2; ++j) {
+        const float* r = p + (k ? slice : 0) + (j ? row : 0);
+        c[k][j][0] = vload<C>(r, 0);
+        c[k][j][1] = vload<C>(r, 1);
       }
+  } else {
+    const Taps t = make_taps<BM>(px, py, pz, d);
+    wx = t.wx;
+    wy = t.wy;
+    wz = t.wz;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          c[k][j][i] = vload<C>(buf, flat3(t.ix[i], t.iy[j], t.iz[k], d));
+          if (BM == B_BORDER && !(t.vx[i] & t.vy[j] & t.vz[k])) c[k][j][i] = vzero<C>();
+        }
+  }
+  Vec<C> r;
 #pragma unroll
   for (int ch = 0; ch < C; ++ch) {
-    float v00 = lerpf(c[0][0][0].v[ch], c[0][0][1].v[ch], t.wx);
-    float v01 = lerpf(c[0][1][0].v[ch], c[0][1][1].v[ch], t.wx);
-    float v0 = lerpf(v00, v01, t.wy);
-    float v10 = lerpf(c[1][0][0].v[ch], c[1][0][1].v[ch], t.wx);
-    float v11 = lerpf(c[1][1][0].v[ch], c[1][1][1].v[ch], t.wx);
-    float v1 = lerpf(v10, v11, t.wy);
-    r.v[ch] = lerpf(v0, v1, t.wz);
+    float v00 = lerpf(c[0][0][0].v[ch], c[0][0][1].v[ch], wx);
+    float v01 = lerpf(c[0][1][0].v[ch], c[0][1][1].v[ch], wx);
+    float v0 = lerpf(v00, v01, wy);
+    float v10 = lerpf(c[1][0][0].v[ch], c[1][0][1].v[ch], wx);
+    float v11 = lerpf(c[1][1][0].v[ch], c[1][1][1].v[ch], wx);
+    float v1 = lerpf(v10, v11, wy);
+    r.v[ch] = lerpf(v0, v1, wz);
   }
   return r;
 }
@@ -484,18 +514,40 @@ struct SampleCfg {
   float offset;  // cell-centre offset subtracted before the tap
 };
 
-// One (batch, camera) view of a transform resample. Forward coordinate modes
-// (idx -> object space) use A = P^-1, B = (V M)^-1; reverse modes (object
-// space -> idx) use A = V M, B = P. p22/p32 are P's entries (col 2, row 2)
-// and (col 3, row 2) for the linear-depth remap.
-struct SampleView {
-  float A[16];
-  float B[16];
+// One (batch, camera) view of a transform resample: the map from an output
+// index q = (x, y, z) (cell centres at + 0.5) to the input position.
+// Forward modes: linear forms with the components X, Y, Z, W, folded on the
+// host in double precision from the index scales, projection, model-view and
+// linear-depth remap; x, y, z count from the middle of the output (mid):
+//   TRANSFORM_LINDEPTH  h = (a x + b y + e) s + c, s = z0 + z1 z (the view depth)
+//   TRANSFORM           h = a x + b y + c z + e
+// and the position is h.XYZ / h.W. A perspective camera's LINDEPTH map has a
+// constant W (the position is affine along a pixel's column), which is divided
+// out (unit): a position then takes ten multiply-adds.
+// Reverse modes: step by step through model-view and projection (ReverseMap).
+// Linear depth cancels most of a depth's digits there, so a folded form rounds
+// elsewhere: gradients as near to 64 bits as this (1.3 to 2.3e-5 against 1.4 to
+// 2.2e-5), but up to 2.7e-5 away from it.
+struct ReverseMap {
+  float A[16], B[16];  // model-view, projection
+  float idims[3];      // the input's dims (x, y, z)
   float p22, p32, nearp, farp;
+};
+struct SampleView {
+  float a[4], b[4], c[4], e[4];
+  float mid[3];
+  float z0, z1;
+  ReverseMap rev;
+  int unit;  // W is 1
   int in_batch;
   int out_slot;
 };
 constexpr int kMaxSampleViews = 8;
+// the reverse maps of a forward launch's views (kernel arguments stay below 4 KiB)
+struct ReverseLaunch {
+  ReverseMap view[kMaxSampleViews];
+  int cm;  // Coord: a reverse mode
+};
 struct SampleLaunch {
   SampleView view[kMaxSampleViews];
   int num_views;

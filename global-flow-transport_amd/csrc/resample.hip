@@ -7,6 +7,8 @@
 // records travel as kernel arguments (no __constant__ state, re-entrant).
 // Sampler semantics follow the v1 sampler of the reference
 // (phitest/render/cuda/src/sampling.hpp:158-252,356-491,539-764).
+#include <algorithm>
+
 #include "gft_device.hpp"
 #include "sampler_v1.hpp"
 
@@ -14,6 +16,13 @@ namespace gft {
 
 // ---------------------------------------------------------------- helpers
 __device__ __forceinline__ void unflat(size_t f, Dims3 d, int& x, int& y, int& z) {
+  if ((f >> 32) == 0) {
+    const unsigned g = (unsigned)f, r = g / (unsigned)d.x, k = r / (unsigned)d.y;
+    x = (int)(g - r * (unsigned)d.x);
+    y = (int)(r - k * (unsigned)d.y);
+    z = (int)k;
+    return;
+  }
   x = (int)(f % (size_t)d.x);
   size_t r = f / (size_t)d.x;
   y = (int)(r % (size_t)d.y);
@@ -73,59 +82,138 @@ __device__ __forceinline__ Vec<C> fetch_v1(const float* __restrict__ buf, Dims3 
   return read_minmax_v1<C, BM>(buf, d, px, py, pz, fm == F_MAX, nullptr);
 }
 
+// The levels are walked with one index for the whole wave (lanes of a wave
+// rarely need more than two), so that a level's dims and address are scalars.
 template <int C, int BM>
 __device__ __forceinline__ Vec<C> sample_v1(const float* base, const float* atlas, const MipTable& mt, int b,
                                             const SampleCfg& s, float3 p, float lod) {
   int lv[2];
   float w[2];
-  int n = level_taps(s, lod, lv, w);
-  float sc = 1.f / (float)(1 << lv[0]);
-  Vec<C> a = fetch_v1<C, BM>(level_ptr(base, atlas, mt, b, lv[0]), mt.dims[lv[0]], s.fm, p.x * sc - s.offset,
-                             p.y * sc - s.offset, p.z * sc - s.offset);
-  if (n == 2) {
-    float sc1 = 1.f / (float)(1 << lv[1]);
-    Vec<C> c = fetch_v1<C, BM>(level_ptr(base, atlas, mt, b, lv[1]), mt.dims[lv[1]], s.fm, p.x * sc1 - s.offset,
-                               p.y * sc1 - s.offset, p.z * sc1 - s.offset);
+  const int n = level_taps(s, lod, lv, w);
+  Vec<C> a = vzero<C>();
+  for (int m = 0; m <= s.levels; ++m) {
+    const bool upper = (n == 2) & (lv[1] == m);
+    if (__ballot((lv[0] == m) | upper) == 0) continue;
+    if (!((lv[0] == m) | upper)) continue;
+    const float sc = level_scale(m);
+    const Vec<C> c = fetch_v1<C, BM>(level_ptr(base, atlas, mt, b, m), mt.dims[m], s.fm, p.x * sc - s.offset,
+                                     p.y * sc - s.offset, p.z * sc - s.offset);
 #pragma unroll
-    for (int ch = 0; ch < C; ++ch) a.v[ch] = lerpf(a.v[ch], c.v[ch], w[1]);
+    for (int ch = 0; ch < C; ++ch) a.v[ch] = upper ? lerpf(a.v[ch], c.v[ch], w[1]) : c.v[ch];
   }
   return a;
 }
 
+// Most cells of a camera frustum lie outside the grid: a BORDER LINEAR sample
+// outside the box [0, dims) reads 0 at every mip level (a level's box is no
+// larger), so its level of detail and taps are left out. The samplers decide
+// on a rounded position; the slack covers that.
+template <int BM> __device__ __forceinline__ bool may_read(int fm, float3 p, Dims3 d) {
+  return BM != B_BORDER || fm != F_LINEAR ||
+         ((-1e-2f <= p.x) & (p.x < (float)d.x) & (-1e-2f <= p.y) & (p.y < (float)d.y) & (-1e-2f <= p.z) &
+          (p.z < (float)d.z));
+}
+
 // ---------------------------------------------------------------- mips
 // kGenerateMip3D (resample_grid.cu.cc:46-72): pairwise means in z, then y,
-// then x. One thread per coarse voxel; blockIdx.y = batch. Every source value
-// is multiplied by `scale` first (1 leaves it unchanged): the pyramid of a
-// scaled grid without materialising the scaled grid.
+// then x; blockIdx.y = batch. Every source value is multiplied by `scale` first
+// (1 leaves it unchanged): the pyramid of a scaled grid without materialising
+// the scaled grid.
+// A workgroup takes a tile of 32 x 16 x 16 source cells and builds up to
+// kMipLevels levels of it, each from the one before in LDS (a level's cells only
+// read the two cells under them per axis, so tiles are independent): one launch
+// reads the source once instead of a launch and a read per level. A pyramid of
+// a 128x224x128 grid took 4 launches of 4 us and more each, mostly latency.
+constexpr int kMipLevels = 4;
+constexpr int kMipX = 16, kMipY = 8, kMipZ = 8;  // level-1 cells of a tile
+struct MipChain {
+  Dims3 dims[kMipLevels + 1];      // the source and the levels
+  size_t offset[kMipLevels + 1];   // of each level in a batch's atlas block
+  int levels;
+};
+
 template <int C>
-__global__ __launch_bounds__(256) void k_mip_down(const float* __restrict__ src, size_t src_stride, Dims3 s,
-                                                  float* __restrict__ dst, size_t dst_stride, Dims3 o, float scale) {
+__device__ __forceinline__ Vec<C> mip_mean(const Vec<C> v[2][2][2]) {  // [x][y][z]
 #pragma clang fp contract(off)
-  size_t n = (size_t)o.x * o.y * o.z;
-  size_t f = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= n) return;
-  const float* in = src + (size_t)blockIdx.y * src_stride;
-  float* out = dst + (size_t)blockIdx.y * dst_stride;
-  int x, y, z;
-  unflat(f, o, x, y, z);
-  Vec<C> ya[2];
-#pragma unroll
-  for (int xi = 0; xi < 2; ++xi) {
-    Vec<C> za[2];
-#pragma unroll
-    for (int yi = 0; yi < 2; ++yi) {
-      Vec<C> a = vload<C>(in, flat3(2 * x + xi, 2 * y + yi, 2 * z, s));
-      Vec<C> b = vload<C>(in, flat3(2 * x + xi, 2 * y + yi, 2 * z + 1, s));
-#pragma unroll
-      for (int ch = 0; ch < C; ++ch) za[yi].v[ch] = (a.v[ch] * scale + b.v[ch] * scale) * 0.5f;
-    }
-#pragma unroll
-    for (int ch = 0; ch < C; ++ch) ya[xi].v[ch] = (za[0].v[ch] + za[1].v[ch]) * 0.5f;
-  }
   Vec<C> r;
 #pragma unroll
-  for (int ch = 0; ch < C; ++ch) r.v[ch] = (ya[0].v[ch] + ya[1].v[ch]) * 0.5f;
-  vstore<C>(out, f, r);
+  for (int ch = 0; ch < C; ++ch) {
+    float ya[2];
+#pragma unroll
+    for (int xi = 0; xi < 2; ++xi) {
+      const float z0 = (v[xi][0][0].v[ch] + v[xi][0][1].v[ch]) * 0.5f;
+      const float z1 = (v[xi][1][0].v[ch] + v[xi][1][1].v[ch]) * 0.5f;
+      ya[xi] = (z0 + z1) * 0.5f;
+    }
+    r.v[ch] = (ya[0] + ya[1]) * 0.5f;
+  }
+  return r;
+}
+
+template <int C>
+__global__ __launch_bounds__(256) void k_mip_down(const float* __restrict__ src, size_t src_stride,
+                                                  float* __restrict__ dst, size_t dst_stride, MipChain m,
+                                                  float scale) {
+#pragma clang fp contract(off)
+  __shared__ float lds[(kMipX * kMipY * kMipZ + kMipX * kMipY * kMipZ / 8) * C];
+  const int ntx = (m.dims[1].x + kMipX - 1) / kMipX, nty = (m.dims[1].y + kMipY - 1) / kMipY;
+  const int t = (int)blockIdx.x;
+  const int x0 = (t % ntx) * kMipX, y0 = ((t / ntx) % nty) * kMipY, z0 = (t / (ntx * nty)) * kMipZ;
+  const float* in = src + (size_t)blockIdx.y * src_stride;
+  float* atlas = dst + (size_t)blockIdx.y * dst_stride;
+#pragma unroll
+  for (int k = 0; k < kMipX * kMipY * kMipZ / 256; ++k) {
+    const int c = k * 256 + (int)threadIdx.x;
+    const int x = x0 + c % kMipX, y = y0 + c / kMipX % kMipY, z = z0 + c / (kMipX * kMipY);
+    Vec<C> r = vzero<C>();
+    if ((x < m.dims[1].x) & (y < m.dims[1].y) & (z < m.dims[1].z)) {
+      Vec<C> v[2][2][2];
+#pragma unroll
+      for (int zi = 0; zi < 2; ++zi)
+#pragma unroll
+        for (int yi = 0; yi < 2; ++yi) {
+          const size_t f = flat3(2 * x, 2 * y + yi, 2 * z + zi, m.dims[0]);
+#pragma unroll
+          for (int xi = 0; xi < 2; ++xi) {
+            v[xi][yi][zi] = vload<C>(in, f + xi);
+#pragma unroll
+            for (int ch = 0; ch < C; ++ch) v[xi][yi][zi].v[ch] *= scale;
+          }
+        }
+      r = mip_mean<C>(v);
+      vstore<C>(atlas + m.offset[1], flat3(x, y, z, m.dims[1]), r);
+    }
+    if (m.levels > 1) vstore<C>(lds, c, r);
+  }
+  int wx = kMipX, wy = kMipY, wz = kMipZ;
+  float *from = lds, *to = lds + kMipX * kMipY * kMipZ * C;
+  for (int l = 2; l <= m.levels; ++l) {
+    __syncthreads();
+    const int hx = wx / 2, hy = wy / 2, hz = wz / 2, c = (int)threadIdx.x;
+    if (c < hx * hy * hz) {
+      const int lx = c % hx, ly = c / hx % hy, lz = c / (hx * hy);
+      Vec<C> v[2][2][2];
+#pragma unroll
+      for (int zi = 0; zi < 2; ++zi)
+#pragma unroll
+        for (int yi = 0; yi < 2; ++yi)
+#pragma unroll
+          for (int xi = 0; xi < 2; ++xi)
+            v[xi][yi][zi] = vload<C>(from, ((2 * lz + zi) * wy + 2 * ly + yi) * wx + 2 * lx + xi);
+      const Vec<C> r = mip_mean<C>(v);
+      const int x = (x0 >> (l - 1)) + lx, y = (y0 >> (l - 1)) + ly, z = (z0 >> (l - 1)) + lz;
+      if ((x < m.dims[l].x) & (y < m.dims[l].y) & (z < m.dims[l].z))
+        vstore<C>(atlas + m.offset[l], flat3(x, y, z, m.dims[l]), r);
+      vstore<C>(to, c, r);
+    }
+    // the level just read is free for the next one but one
+    float* const f = from;
+    from = to;
+    to = f;
+    wx = hx;
+    wy = hy;
+    wz = hz;
+  }
 }
 
 // Adjoint of one mip step: every fine voxel under a coarse voxel receives 1/8
@@ -150,43 +238,64 @@ __global__ __launch_bounds__(256) void k_mip_collapse(const float* __restrict__ 
 }
 
 // ------------------------------------------------------ transform forward
-// kSample3D (resample_grid.cu.cc:240-252). blockIdx.y = view of the launch.
+// kSample3D (resample_grid.cu.cc:240-252). blockIdx.z = view of the launch. A
+// wave takes 8 x 8 cells in x and z, the block's four waves consecutive y, and
+// a thread `runs` of its cells at every fourth y.
+// Neighbours in the output's xz-plane are neighbours in the input's for cameras
+// that orbit around y, so an 8 x 8 wave reads a compact patch; 64 cells of a row
+// per wave touch a cache line each. The view-summed gather (C = 4, 3 views,
+// LINEAR mips, 100x178x100) takes 123 us, 224-265 with rows, and C = 1 of a
+// 256x128x128 light volume 60, before 71. VALU work bounds it: the folded forms
+// and leaving out what lies outside the grid took the forward from 825 us (IEEE
+// divides, four maps per level of detail) to 332.
 // SUM: one thread loops over the launch's views and writes (or adds) the sum
 // into slot 0, the view-summed gather of the production sampling gradient.
-template <int C, int BM, bool SUM>
+constexpr int kSampleX = 8, kSampleY = 4, kSampleZ = 8;
+template <int C, int BM, bool SUM, bool LOD>
 __global__ __launch_bounds__(256) void k_sample_transform(const float* __restrict__ in,
                                                           const float* __restrict__ atlas, MipTable mt, SampleCfg s,
-                                                          Dims3 dout, SampleLaunch L, float* __restrict__ out) {
-  size_t n = (size_t)dout.x * dout.y * dout.z;
-  size_t f = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (f >= n) return;
-  int x, y, z;
-  unflat(f, dout, x, y, z);
-  const float3 oinv = make_float3(1.f / dout.x, 1.f / dout.y, 1.f / dout.z);
-  const float3 idims = make_float3((float)mt.dims[0].x, (float)mt.dims[0].y, (float)mt.dims[0].z);
-  const bool lod = s.mm != MIP_NONE;
-  if constexpr (SUM) {
-    Vec<C> acc = vzero<C>();
-    for (int vi = 0; vi < L.num_views; ++vi) {
-      const SampleView& v = L.view[vi];
+                                                          Dims3 dout, SampleLaunch L, int runs,
+                                                          float* __restrict__ out) {
+  const unsigned ntx = (unsigned)(dout.x + kSampleX - 1) / kSampleX, ty = blockIdx.x / ntx, tx = blockIdx.x - ty * ntx;
+  const int x = (int)tx * kSampleX + (int)(threadIdx.x % kSampleX);
+  const int y0 = (int)ty * kSampleY * runs + (int)(threadIdx.x / (kSampleX * kSampleZ));
+  const size_t n = (size_t)dout.x * dout.y * dout.z;
+  // (one z tile per block, but for grids deeper than the launch limit)
+  for (int z = (int)(blockIdx.y * kSampleZ + threadIdx.x / kSampleX % kSampleZ); z < dout.z;
+       z += (int)(gridDim.y * kSampleZ)) {
+    for (int k = 0; k < runs; ++k) {
+      const int y = y0 + k * kSampleY;
+      if ((x >= dout.x) | (y >= dout.y)) break;
+      const size_t f = flat3(x, y, z, dout);
       float l;
-      float3 p = sample_pos(v, L.cm, lod, x + 0.5f, y + 0.5f, z + 0.5f, oinv, idims, l);
-      Vec<C> r = sample_v1<C, BM>(in, atlas, mt, v.in_batch, s, p, l);
+      if constexpr (SUM) {
+        Vec<C> acc = vzero<C>();
+        for (int vi = 0; vi < L.num_views; ++vi) {
+          const SampleView& v = L.view[vi];
+          const float3 p0 = map_pos(v, L.cm, x + 0.5f, y + 0.5f, z + 0.5f);
+          if (!may_read<BM>(s.fm, p0, mt.dims[0])) continue;
+          const float3 p = map_sample<LOD>(v, L.cm, x + 0.5f, y + 0.5f, z + 0.5f, l);
+          const Vec<C> r = sample_v1<C, BM>(in, atlas, mt, v.in_batch, s, p, l);
 #pragma unroll
-      for (int ch = 0; ch < C; ++ch) acc.v[ch] += r.v[ch];
-    }
-    if (L.accumulate) {
-      Vec<C> o = vload<C>(out, f);
+          for (int ch = 0; ch < C; ++ch) acc.v[ch] += r.v[ch];
+        }
+        if (L.accumulate) {
+          const Vec<C> o = vload<C>(out, f);
 #pragma unroll
-      for (int ch = 0; ch < C; ++ch) acc.v[ch] += o.v[ch];
+          for (int ch = 0; ch < C; ++ch) acc.v[ch] += o.v[ch];
+        }
+        vstore<C>(out, f, acc);
+      } else {
+        const SampleView& v = L.view[blockIdx.z];
+        Vec<C> r = vzero<C>();
+        const float3 p0 = map_pos(v, L.cm, x + 0.5f, y + 0.5f, z + 0.5f);
+        if (may_read<BM>(s.fm, p0, mt.dims[0])) {
+          const float3 p = map_sample<LOD>(v, L.cm, x + 0.5f, y + 0.5f, z + 0.5f, l);
+          r = sample_v1<C, BM>(in, atlas, mt, v.in_batch, s, p, l);
+        }
+        vstore<C>(out + (size_t)v.out_slot * n * C, f, r);
+      }
     }
-    vstore<C>(out, f, acc);
-  } else {
-    const SampleView& v = L.view[blockIdx.y];
-    float l;
-    float3 p = sample_pos(v, L.cm, lod, x + 0.5f, y + 0.5f, z + 0.5f, oinv, idims, l);
-    Vec<C> r = sample_v1<C, BM>(in, atlas, mt, v.in_batch, s, p, l);
-    vstore<C>(out + (size_t)v.out_slot * n * C, f, r);
   }
 }
 
@@ -276,10 +385,7 @@ __global__ __launch_bounds__(256) void k_sample_transform_scatter_ref(const floa
   const SampleView& v = L.view[blockIdx.y];
   int x, y, z;
   unflat(f, dout, x, y, z);
-  const float3 oinv = make_float3(1.f / dout.x, 1.f / dout.y, 1.f / dout.z);
-  const float3 idims = make_float3((float)din.x, (float)din.y, (float)din.z);
-  float l;
-  float3 p = sample_pos(v, L.cm, false, x + 0.5f, y + 0.5f, z + 0.5f, oinv, idims, l);
+  const float3 p = map_pos(v, L.cm, x + 0.5f, y + 0.5f, z + 0.5f);
   Vec<C> g = vload<C>(og + (size_t)v.out_slot * n * C, f);
   scatter_reference<C, BM>(grad, cnt, din, p.x - 0.5f, p.y - 0.5f, p.z - 0.5f, g);
 }
@@ -299,17 +405,15 @@ __global__ __launch_bounds__(256) void k_sample_transform_adjoint(const float* _
   const SampleView& v = L.view[blockIdx.y];
   int x, y, z;
   unflat(f, dout, x, y, z);
-  const float3 oinv = make_float3(1.f / dout.x, 1.f / dout.y, 1.f / dout.z);
-  const float3 idims = make_float3((float)mt.dims[0].x, (float)mt.dims[0].y, (float)mt.dims[0].z);
   float l;
-  float3 p = sample_pos(v, L.cm, s.mm != MIP_NONE, x + 0.5f, y + 0.5f, z + 0.5f, oinv, idims, l);
+  const float3 p = map_sample<true>(v, L.cm, x + 0.5f, y + 0.5f, z + 0.5f, l);
   Vec<C> g = vload<C>(og + (size_t)v.out_slot * n * C, f);
   int lv[2];
   float w[2];
   int nt = level_taps(s, l, lv, w);
   for (int t = 0; t < nt; ++t) {
     int m = lv[t];
-    float sc = 1.f / (float)(1 << m);
+    const float sc = level_scale(m);
     fetch_v1_adjoint<C, BM>(level_ptr(in, atlas, mt, v.in_batch, m), level_ptr_mut(grad, gatlas, mt, v.in_batch, m),
                             mt.dims[m], s.fm, p.x * sc - s.offset, p.y * sc - s.offset, p.z * sc - s.offset, g, w[t]);
   }
@@ -334,7 +438,7 @@ constexpr int kGBX = 16, kGBY = 8, kGBZ = 4, kGBVox = kGBX * kGBY * kGBZ;
 
 // frustum-space bounds [lo, hi] (cell indices) of the cells whose sample can
 // land in the position box b0..b1 (vinv: the view in the reverse coordinate
-// mode, grid position -> frustum position, as map_pos computes it). The x and
+// mode, grid position -> frustum position, as map_reverse computes it). The x and
 // y images are projective in the position (extremes at the corners while
 // every corner is in front of the camera, w > 0); the linear-depth image
 // -p32 / (ndz + p22) is monotonic on each side of its pole, and frustum cells
@@ -342,8 +446,8 @@ constexpr int kGBX = 16, kGBY = 8, kGBZ = 4, kGBVox = kGBX * kGBY * kGBZ;
 // hull, all on the positive side -> no cell, straddling the pole (possible
 // for orthographic projections) -> every depth. Out-of-front corners or NaN
 // widen to every cell.
-__device__ __forceinline__ void gather_cell_bounds(const SampleView& vinv, int cm_inv, float3 b0, float3 b1,
-                                                   float3 idims_out, Dims3 dout, int lo[3], int hi[3]) {
+__device__ __forceinline__ void gather_cell_bounds(const ReverseMap& vinv, int cm_inv, float3 b0, float3 b1, Dims3 dout,
+                                                   int lo[3], int hi[3]) {
   float mn[3] = {3.4e38f, 3.4e38f, 3.4e38f}, mx[3] = {-3.4e38f, -3.4e38f, -3.4e38f};
   bool ok = true;
   int neg = 0, pos = 0;
@@ -352,17 +456,13 @@ __device__ __forceinline__ void gather_cell_bounds(const SampleView& vinv, int c
     // positions are in sample units; the coordinate maps take cell-centre units (+0.5)
     const float qx = ((k & 1) ? b1.x : b0.x) + 0.5f, qy = ((k & 2) ? b1.y : b0.y) + 0.5f,
                 qz = ((k & 4) ? b1.z : b0.z) + 0.5f;
-    const float4 vs = mat_vec(vinv.A, qx, qy, qz, 1.f);
-    const float4 ndc = mat_vec(vinv.B, vs.x, vs.y, vs.z, vs.w);
-    ok &= ndc.w > 0.f;
-    const float ndx = ndc.x / ndc.w, ndy = ndc.y / ndc.w, ndz = ndc.z / ndc.w;
-    float r[3] = {(ndx * 0.5f + 0.5f) * idims_out.x, (ndy * 0.5f + 0.5f) * idims_out.y,
-                  (ndz * 0.5f + 0.5f) * idims_out.z};
+    float w, z;
+    const float3 im = map_reverse(vinv, cm_inv, qx, qy, qz, w, z);
+    ok &= w > 0.f;
+    const float r[3] = {im.x, im.y, im.z};
     if (cm_inv == CM_LINDEPTH_REVERSE) {
-      const float z = -vinv.p32 / (ndz + vinv.p22);
       neg += z < 0.f;
       pos += z > 0.f;
-      r[2] = -(z + vinv.nearp) / (vinv.farp - vinv.nearp) * idims_out.z;
     }
 #pragma unroll
     for (int a = 0; a < 3; ++a) {
@@ -397,7 +497,7 @@ __device__ __forceinline__ void gather_cell_bounds(const SampleView& vinv, int c
 
 template <int C, bool REF, int FM>
 __global__ __launch_bounds__(256) void k_sample_transform_gather_adj(const float* __restrict__ og, Dims3 din,
-                                                                     Dims3 dout, SampleLaunch L, SampleLaunch Linv,
+                                                                     Dims3 dout, SampleLaunch L, ReverseLaunch Linv,
                                                                      int accumulate, float* __restrict__ grad) {
   __shared__ double acc[kGBVox * C];
   __shared__ unsigned cnt[REF ? kGBVox : 1];
@@ -413,16 +513,13 @@ __global__ __launch_bounds__(256) void k_sample_transform_gather_adj(const float
     for (int k = threadIdx.x; k < kGBVox; k += 256) cnt[k] = 0u;
   __syncthreads();
   const size_t n = (size_t)dout.x * dout.y * dout.z;
-  const float3 oinv = make_float3(1.f / dout.x, 1.f / dout.y, 1.f / dout.z);
-  const float3 idims = make_float3((float)din.x, (float)din.y, (float)din.z);
-  const float3 idims_out = make_float3((float)dout.x, (float)dout.y, (float)dout.z);
   // nearest truncates p + 0.5 toward zero, so p down to x0 - 1.5 can reach x0 = 0
   const float3 b0 = make_float3((float)x0 - 2.f, (float)y0 - 2.f, (float)z0 - 2.f);
   const float3 b1 = make_float3((float)(x0 + kGBX), (float)(y0 + kGBY), (float)(z0 + kGBZ));
   for (int vi = 0; vi < L.num_views; ++vi) {
     const SampleView& v = L.view[vi];
     int lo[3], hi[3];
-    gather_cell_bounds(Linv.view[vi], Linv.cm, b0, b1, idims_out, dout, lo, hi);
+    gather_cell_bounds(Linv.view[vi], Linv.cm, b0, b1, dout, lo, hi);
     if (lo[0] > hi[0] || lo[1] > hi[1] || lo[2] > hi[2]) continue;
     const unsigned nx = hi[0] - lo[0] + 1, ny = hi[1] - lo[1] + 1;
     const unsigned cells = nx * ny * (unsigned)(hi[2] - lo[2] + 1);  // the caller keeps n below 2^31
@@ -430,8 +527,7 @@ __global__ __launch_bounds__(256) void k_sample_transform_gather_adj(const float
     for (unsigned k = threadIdx.x; k < cells; k += 256) {
       const unsigned r = k / nx;
       const int cx = lo[0] + (int)(k - r * nx), cy = lo[1] + (int)(r % ny), cz = lo[2] + (int)(r / ny);
-      float l;
-      const float3 q = sample_pos(v, L.cm, false, cx + 0.5f, cy + 0.5f, cz + 0.5f, oinv, idims, l);
+      const float3 q = map_pos(v, L.cm, cx + 0.5f, cy + 0.5f, cz + 0.5f);
       const float px = q.x - 0.5f, py = q.y - 0.5f, pz = q.z - 0.5f;
       if (!((px >= b0.x) & (px <= b1.x) & (py >= b0.y) & (py <= b1.y) & (pz >= b0.z) & (pz <= b1.z))) continue;
       const Vec<C> g = vload<C>(ogv, ((size_t)cz * dout.y + cy) * dout.x + cx);
@@ -842,12 +938,10 @@ __global__ __launch_bounds__(kLodTX * kLodTY * kLodTZ) void k_lod_transform(Dims
   const int ntx = (dout.x + kLodTX - 1) / kLodTX, nty = (dout.y + kLodTY - 1) / kLodTY;
   const int t = (int)blockIdx.x;
   const int x0 = (t % ntx) * kLodTX, y0 = ((t / ntx) % nty) * kLodTY, z0 = (t / (ntx * nty)) * kLodTZ;
-  const float3 oinv = make_float3(1.f / dout.x, 1.f / dout.y, 1.f / dout.z);
-  const float3 idims = make_float3((float)din.x, (float)din.y, (float)din.z);
   for (int k = threadIdx.x; k < NH; k += blockDim.x) {
     const int hx = k % HX, hy = (k / HX) % HY, hz = k / (HX * HY);
     const float3 p = map_pos(v, L.cm, (float)(x0 + hx - 1) + 0.5f, (float)(y0 + hy - 1) + 0.5f,
-                             (float)(z0 + hz - 1) + 0.5f, oinv, idims);
+                             (float)(z0 + hz - 1) + 0.5f);
     hp[0][k] = p.x;
     hp[1][k] = p.y;
     hp[2][k] = p.z;
@@ -910,21 +1004,49 @@ __device__ __forceinline__ float fetch_scaled(const float* __restrict__ buf, Dim
     bool ok = nearest_index<BM>(px, py, pz, d, f);
     return ok ? scaled_load(buf + f, sc) : 0.f;
   } else {
-    Taps t = make_taps<BM>(px, py, pz, d);
-    if (BM == B_BORDER && !t.inside) return 0.f;
-    float c[2][2][2];
+    // as read_linear: waves whose corners all lie in the grid read them from one base address
+    if constexpr (BM == B_BORDER) {
+      const float qx = px + 0.5f, qy = py + 0.5f, qz = pz + 0.5f;
+      if (!((0.f <= qx) & (qx < (float)d.x) & (0.f <= qy) & (qy < (float)d.y) & (0.f <= qz) & (qz < (float)d.z)))
+        return 0.f;
+    }
+    const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
+    const int ix = (int)fx, iy = (int)fy, iz = (int)fz;
+    const bool inner = ((unsigned)ix < (unsigned)(d.x - 1)) & ((unsigned)iy < (unsigned)(d.y - 1)) &
+                       ((unsigned)iz < (unsigned)(d.z - 1));
+    float c[2][2][2], wx, wy, wz;
+    if (__ballot(!inner) == 0) {
+      wx = px - fx;
+      wy = py - fy;
+      wz = pz - fz;
+      const float* p = buf + flat3(ix, iy, iz, d);
+      const size_t row = d.x, slice = row * d.y;
 #pragma unroll
-    for (int k = 0; k < 2; ++k)
+      for (int k = 0; k < 2; ++k)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          c[k][j][i] = scaled_load(buf + flat3(t.ix[i], t.iy[j], t.iz[k], d), sc);
-          if (BM == B_BORDER && !(t.vx[i] & t.vy[j] & t.vz[k])) c[k][j][i] = 0.f;
+        for (int j = 0; j < 2; ++j) {
+          const float* r = p + (k ? slice : 0) + (j ? row : 0);
+          c[k][j][0] = scaled_load(r, sc);
+          c[k][j][1] = scaled_load(r + 1, sc);
         }
-    float v0 = lerpf(lerpf(c[0][0][0], c[0][0][1], t.wx), lerpf(c[0][1][0], c[0][1][1], t.wx), t.wy);
-    float v1 = lerpf(lerpf(c[1][0][0], c[1][0][1], t.wx), lerpf(c[1][1][0], c[1][1][1], t.wx), t.wy);
-    return lerpf(v0, v1, t.wz);
+    } else {
+      const Taps t = make_taps<BM>(px, py, pz, d);
+      wx = t.wx;
+      wy = t.wy;
+      wz = t.wz;
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            c[k][j][i] = scaled_load(buf + flat3(t.ix[i], t.iy[j], t.iz[k], d), sc);
+            if (BM == B_BORDER && !(t.vx[i] & t.vy[j] & t.vz[k])) c[k][j][i] = 0.f;
+          }
+    }
+    float v0 = lerpf(lerpf(c[0][0][0], c[0][0][1], wx), lerpf(c[0][1][0], c[0][1][1], wx), wy);
+    float v1 = lerpf(lerpf(c[1][0][0], c[1][0][1], wx), lerpf(c[1][1][0], c[1][1][1], wx), wy);
+    return lerpf(v0, v1, wz);
   }
 }
 
@@ -941,15 +1063,16 @@ __device__ __forceinline__ float sample_scaled(const float* __restrict__ base, c
                                                float step) {
   int lv[2];
   float w[2];
-  int n = level_taps(s, lod, lv, w);
-  float sc = 1.f / (float)(1 << lv[0]);
-  float a = fetch_scaled<BM, FM>(level_ptr(base, atlas, mt, 0, lv[0]), mt.dims[lv[0]], p.x * sc - s.offset,
-                                 p.y * sc - s.offset, p.z * sc - s.offset, lv[0] == 0 ? step : 1.f);
-  if (n == 2) {
-    float sc1 = 1.f / (float)(1 << lv[1]);
-    float c = fetch_scaled<BM, FM>(level_ptr(base, atlas, mt, 0, lv[1]), mt.dims[lv[1]], p.x * sc1 - s.offset,
-                                   p.y * sc1 - s.offset, p.z * sc1 - s.offset, lv[1] == 0 ? step : 1.f);
-    a = lerpf(a, c, w[1]);
+  const int n = level_taps(s, lod, lv, w);
+  float a = 0.f;
+  for (int m = 0; m <= s.levels; ++m) {
+    const bool upper = (n == 2) & (lv[1] == m);
+    if (__ballot((lv[0] == m) | upper) == 0) continue;
+    if (!((lv[0] == m) | upper)) continue;
+    const float sc = level_scale(m);
+    const float c = fetch_scaled<BM, FM>(level_ptr(base, atlas, mt, 0, m), mt.dims[m], p.x * sc - s.offset,
+                                         p.y * sc - s.offset, p.z * sc - s.offset, m == 0 ? step : 1.f);
+    a = upper ? lerpf(a, c, w[1]) : c;
   }
   return a;
 }
@@ -967,8 +1090,6 @@ __global__ __launch_bounds__(kShadowWaves * 64) void k_shadow_fwd(const float* _
   const size_t p = (size_t)blockIdx.x * 64 + lane;
   const bool live = p < plane;
   const int x = live ? (int)(p % (size_t)dout.x) : 0, y = live ? (int)(p / (size_t)dout.x) : 0;
-  const float3 oinv = make_float3(1.f / dout.x, 1.f / dout.y, 1.f / dout.z);
-  const float3 idims = make_float3((float)mt.dims[0].x, (float)mt.dims[0].y, (float)mt.dims[0].z);
   const float mk = (mask && live) ? mask[p] : 1.f;
   float* row = s_lds + lane * kShadowPitch;
   float carry = 0.f;
@@ -981,8 +1102,10 @@ __global__ __launch_bounds__(kShadowWaves * 64) void k_shadow_fwd(const float* _
       float val = 0.f;
       if (live && z < dout.z) {
         float l;
-        float3 q = sample_pos(v, CM_LINDEPTH, LOD, x + 0.5f, y + 0.5f, z + 0.5f, oinv, idims, l);
-        val = sample_scaled<BM, FM>(dens, atlas, mt, cfg, q, l, step);
+        if (may_read<BM>(FM, map_pos(v, CM_LINDEPTH, x + 0.5f, y + 0.5f, z + 0.5f), mt.dims[0])) {
+          const float3 q = map_sample<LOD>(v, CM_LINDEPTH, x + 0.5f, y + 0.5f, z + 0.5f, l);
+          val = sample_scaled<BM, FM>(dens, atlas, mt, cfg, q, l, step);
+        }
       }
       row[w * kShadowSeg + i] = val;
     }
@@ -1103,13 +1226,23 @@ static inline dim3 grid_for(size_t n, unsigned views) { return dim3((unsigned)((
     default: { constexpr int BB = B_WRAP; __VA_ARGS__; } break;         \
   }
 
-hipError_t mip_down_launch(int C, hipStream_t st, const float* src, size_t src_stride, Dims3 s, float* dst,
-                           size_t dst_stride, Dims3 o, int batches, float scale) {
-  size_t n = (size_t)o.x * o.y * o.z;
-  GFT_DISPATCH_C(C, hipLaunchKernelGGL(k_mip_down<CC>, grid_for(n, batches), dim3(256), 0, st, src, src_stride, s,
-                                       dst, dst_stride, o, scale));
+// levels first + 1 .. first + n of the pyramid mt (n <= kMipLevels), from level `first`
+hipError_t mip_down_launch(hipStream_t st, const float* src, size_t src_stride, const MipTable& mt, int first, int n,
+                           float* atlas, int batches, float scale) {
+  MipChain m{};
+  m.levels = n;
+  for (int l = 0; l <= n; ++l) {
+    m.dims[l] = mt.dims[first + l];
+    m.offset[l] = mt.offset[first + l];
+  }
+  const Dims3 o = m.dims[1];
+  const size_t tiles = (size_t)((o.x + kMipX - 1) / kMipX) * ((o.y + kMipY - 1) / kMipY) * ((o.z + kMipZ - 1) / kMipZ);
+  const dim3 grid((unsigned)tiles, batches);
+  GFT_DISPATCH_C(mt.C, hipLaunchKernelGGL(k_mip_down<CC>, grid, dim3(256), 0, st, src, src_stride, atlas,
+                                          mt.atlas_stride, m, scale));
   return hipGetLastError();
 }
+int mip_levels_per_launch() { return kMipLevels; }
 
 hipError_t mip_collapse_launch(int C, hipStream_t st, const float* gp, size_t gp_stride, Dims3 o, float* gc,
                                size_t gc_stride, Dims3 s, int batches) {
@@ -1122,21 +1255,27 @@ hipError_t mip_collapse_launch(int C, hipStream_t st, const float* gp, size_t gp
 hipError_t sample_transform_launch(int C, int bm, bool sum, hipStream_t st, const float* in, const float* atlas,
                                    const MipTable& mt, const SampleCfg& s, Dims3 dout, const SampleLaunch& L,
                                    float* out) {
-  size_t n = (size_t)dout.x * dout.y * dout.z;
+  // y runs per thread (100x178x100 grid, 3 views of 480x270 in 142 slices, C = 4,
+  // LINEAR mips; 1 / 2 / 4 / 8): the frusta 363 / 314 / 315 / 359 us (more cells
+  // share a block's set-up), the view-summed grid 105 / 110 / 119 / 124
+  const int runs = sum ? 1 : 2;
+  const int ntx = (dout.x + kSampleX - 1) / kSampleX, nty = (dout.y + kSampleY * runs - 1) / (kSampleY * runs),
+            ntz = (dout.z + kSampleZ - 1) / kSampleZ;
+  const dim3 grid((unsigned)ntx * (unsigned)nty, (unsigned)std::min(ntz, 65535), sum ? 1 : L.num_views);
+  const bool lod = s.mm != MIP_NONE;
   GFT_DISPATCH_C(C, GFT_DISPATCH_BM(bm, {
-    if (sum)
-      hipLaunchKernelGGL((k_sample_transform<CC, BB, true>), grid_for(n, 1), dim3(256), 0, st, in, atlas, mt, s, dout,
-                         L, out);
-    else
-      hipLaunchKernelGGL((k_sample_transform<CC, BB, false>), grid_for(n, L.num_views), dim3(256), 0, st, in, atlas,
-                         mt, s, dout, L, out);
+    auto run = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, in, atlas, mt, s, dout, L, runs, out); };
+    if (sum && lod) run(k_sample_transform<CC, BB, true, true>);
+    else if (sum) run(k_sample_transform<CC, BB, true, false>);
+    else if (lod) run(k_sample_transform<CC, BB, false, true>);
+    else run(k_sample_transform<CC, BB, false, false>);
   }));
   return hipGetLastError();
 }
 
 // gather-form gradient over the voxel blocks of one batch (grad points at it)
 hipError_t sample_transform_gather_launch(int C, bool ref, int fm, hipStream_t st, const float* og, Dims3 din,
-                                          Dims3 dout, const SampleLaunch& L, const SampleLaunch& Linv, int accumulate,
+                                          Dims3 dout, const SampleLaunch& L, const ReverseLaunch& Linv, int accumulate,
                                           float* grad) {
   const unsigned nb = (unsigned)(((din.x + kGBX - 1) / kGBX) * ((din.y + kGBY - 1) / kGBY) *
                                  ((din.z + kGBZ - 1) / kGBZ));

@@ -635,7 +635,7 @@ class _ShadowFn(torch.autograd.Function):
         else:
             g = _sample_transform_bwd_impl(density, gs, ctx.cams, fm, bm, mm, nmip, bias, cm, True, gm)
         # the op sequence scales the grid by the step before sampling: d/d density = step * d/d(scaled grid)
-        g = g * torch.tensor([step], dtype=torch.float32, device=g.device)
+        g.mul_(step)
         return g, None, None, None, None
 
 
