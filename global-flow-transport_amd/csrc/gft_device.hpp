@@ -213,48 +213,92 @@ __device__ __forceinline__ Vec<C> read_linear(const float* __restrict__ buf, Dim
   return r;
 }
 
-// U trilinear reads with all 8U loads issued before any value is used (the
-// indices make_taps returns are always inside the grid, so the loads need no
-// guard): the same corners, zeroing and lerp order as read_linear, so every
-// value equals read_linear's, and a BORDER sample outside the grid reads 0.
+// True where read_linear_batch may address the grid by 32-bit byte offsets.
+template <int C> __device__ __forceinline__ bool offsets_fit(Dims3 d) {
+  const size_t rows = (size_t)d.y * d.z;
+  return (rows < (1u << 24)) & (d.x < (1 << 24)) & (rows * d.x * C * sizeof(float) < (size_t(1) << 31));
+}
+
+// U trilinear reads with all 8U loads issued before any value is used: the
+// same corners, zeroing and lerp order as read_linear, so every value equals
+// read_linear's, and a BORDER sample outside the grid reads 0. `use` masks
+// samples whose value the caller drops. With `fits` (offsets_fit<C>), where
+// every lane's samples have their 8 corners in the grid or read 0 (most of a
+// ray), they are addressed by one offset each from 4 rows' uniform bases,
+// without clamping or corner tests (a C = 4 sample: 120 instructions, 210 with).
 template <int C, int BM, int U>
-__device__ __forceinline__ void read_linear_batch(const float* __restrict__ buf, Dims3 d, const float px[U],
-                                                  const float py[U], const float pz[U], Vec<C> out[U]) {
-  Taps t[U];
+__device__ __forceinline__ void read_linear_batch(const float* __restrict__ buf, Dims3 d, bool fits, const float px[U],
+                                                  const float py[U], const float pz[U], const bool use[U],
+                                                  Vec<C> out[U]) {
   Vec<C> c[U][2][2][2];
-#pragma unroll
-  for (int u = 0; u < U; ++u) t[u] = make_taps<BM>(px[u], py[u], pz[u], d);
-#pragma unroll
-  for (int u = 0; u < U; ++u)
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int i = 0; i < 2; ++i) c[u][k][j][i] = vload<C>(buf, flat3(t[u].ix[i], t[u].iy[j], t[u].iz[k], d));
+  float wx[U], wy[U], wz[U];
+  bool zero[U];
+  unsigned at[U];
+  bool slow = !fits;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
+    zero[u] = !use[u];
     if (BM == B_BORDER) {
+      const float qx = px[u] + 0.5f, qy = py[u] + 0.5f, qz = pz[u] + 0.5f;
+      zero[u] |=
+          !((0.f <= qx) & (qx < (float)d.x) & (0.f <= qy) & (qy < (float)d.y) & (0.f <= qz) & (qz < (float)d.z));
+    }
+    const float fx = floorf(px[u]), fy = floorf(py[u]), fz = floorf(pz[u]);
+    wx[u] = px[u] - fx;
+    wy[u] = py[u] - fy;
+    wz[u] = pz[u] - fz;
+    const int ix = (int)fx, iy = (int)fy, iz = (int)fz;
+    const bool inner = ((unsigned)ix < (unsigned)(d.x - 1)) & ((unsigned)iy < (unsigned)(d.y - 1)) &
+                       ((unsigned)iz < (unsigned)(d.z - 1));
+    slow |= !(inner | zero[u]);
+    const unsigned f = __umul24(__umul24((unsigned)iz, (unsigned)d.y) + (unsigned)iy, (unsigned)d.x) + (unsigned)ix;
+    at[u] = zero[u] ? 0u : f * (unsigned)(C * sizeof(float));
+  }
+  // (a sample that reads 0 loads from the first cells, which an axis of one
+  // cell does not have)
+  if (__ballot(slow) == 0 && (d.x > 1) & (d.y > 1) & (d.z > 1)) {
+    const char* base = (const char*)buf;
+    const unsigned row = (unsigned)d.x * (unsigned)(C * sizeof(float)), slice = row * (unsigned)d.y;
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const char* r = base + ((k ? slice : 0u) + (j ? row : 0u));
+          c[u][k][j][0] = vload<C>((const float*)(r + at[u]), 0);
+          c[u][k][j][1] = vload<C>((const float*)(r + at[u]), 1);
+        }
+  } else {
+    Taps t[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) t[u] = make_taps<BM>(px[u], py[u], pz[u], d);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
 #pragma unroll
       for (int k = 0; k < 2; ++k)
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
-          for (int i = 0; i < 2; ++i)
-            if (!(t[u].vx[i] & t[u].vy[j] & t[u].vz[k])) c[u][k][j][i] = vzero<C>();
-    }
+          for (int i = 0; i < 2; ++i) {
+            c[u][k][j][i] = vload<C>(buf, flat3(t[u].ix[i], t[u].iy[j], t[u].iz[k], d));
+            if (BM == B_BORDER && !(t[u].vx[i] & t[u].vy[j] & t[u].vz[k])) c[u][k][j][i] = vzero<C>();
+          }
+  }
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
     Vec<C> r;
 #pragma unroll
     for (int ch = 0; ch < C; ++ch) {
-      const float v00 = lerpf(c[u][0][0][0].v[ch], c[u][0][0][1].v[ch], t[u].wx);
-      const float v01 = lerpf(c[u][0][1][0].v[ch], c[u][0][1][1].v[ch], t[u].wx);
-      const float v0 = lerpf(v00, v01, t[u].wy);
-      const float v10 = lerpf(c[u][1][0][0].v[ch], c[u][1][0][1].v[ch], t[u].wx);
-      const float v11 = lerpf(c[u][1][1][0].v[ch], c[u][1][1][1].v[ch], t[u].wx);
-      const float v1 = lerpf(v10, v11, t[u].wy);
-      r.v[ch] = lerpf(v0, v1, t[u].wz);
+      const float v00 = lerpf(c[u][0][0][0].v[ch], c[u][0][0][1].v[ch], wx[u]);
+      const float v01 = lerpf(c[u][0][1][0].v[ch], c[u][0][1][1].v[ch], wx[u]);
+      const float v0 = lerpf(v00, v01, wy[u]);
+      const float v10 = lerpf(c[u][1][0][0].v[ch], c[u][1][0][1].v[ch], wx[u]);
+      const float v11 = lerpf(c[u][1][1][0].v[ch], c[u][1][1][1].v[ch], wx[u]);
+      const float v1 = lerpf(v10, v11, wy[u]);
+      r.v[ch] = lerpf(v0, v1, wz[u]);
     }
-    out[u] = (BM == B_BORDER && !t[u].inside) ? vzero<C>() : r;
+    out[u] = zero[u] ? vzero<C>() : r;
   }
 }
 
@@ -391,6 +435,21 @@ __device__ __forceinline__ Vec<C> blend_grad(Vec<C>& g, const Vec<C>& c, Vec<C>&
   }
   return gc;
 }
+
+// -------------------------------------------------------- pixel tiles
+// Tile of block `id` in a launch of tile_blocks(ntx, nty) blocks per view (rows
+// past nty leave at once). Blocks go round robin to the 8 XCDs, and an XCD's to
+// its shader engines in turn, in order: a block whose engine is full holds up
+// all behind it. With ids in row order an image 2^n tiles wide puts each tile
+// column on one engine of one XCD, the centre's long rays together (a raymarch
+// of 32 x 57 tiles: half the CUs idle from 40 us on of 480). So rows of tiles go
+// to the XCDs in turn, and a row's neighbours to one XCD's engines.
+__device__ __forceinline__ void tile_of_block(unsigned id, int ntx, int& tx, int& ty) {
+  const unsigned xcd = id % 8, j = id / 8, row = j / (unsigned)ntx;
+  tx = (int)(j - row * (unsigned)ntx);
+  ty = (int)(row * 8 + xcd);
+}
+inline unsigned tile_blocks(int ntx, int nty) { return (unsigned)ntx * (unsigned)((nty + 7) / 8 * 8); }
 
 // --------------------------------------------------------- camera records
 // Column-major 4x4: m[4*col + row].

@@ -22,11 +22,20 @@
 
 namespace gft {
 
-constexpr int kTileX = 16;
-constexpr int kTileY = 16;
+// A ray kernel's workgroup is one wave of 8 x 8 pixels: its 64 samples at one
+// depth lie in a compact patch of the grid, of few cache lines.
+constexpr int kTileX = 8;
+constexpr int kTileY = 8;
+constexpr int kTile = kTileX * kTileY;
 // samples read per round trip by the LINEAR ray walks (8 float4 corners per
 // C=4 sample: two samples already hold 64 values in registers)
 template <int C> constexpr int kRayBatch = C == 4 ? 2 : (C == 2 ? 4 : 8);
+
+// LDS asked for to keep 10 waves of a C = 4 walk on a CU (16 fit): a sample
+// reads 8 x 16 bytes, so that more waves evict each other's lines from the 32 KB
+// L1 before the next depth reads them again. 128x224x128, 5 views of 256x456
+// (16 / 12 / 10 / 8 / 6 waves): forward 368 / - / 283 / 292 / 293 us.
+template <int C> constexpr unsigned kRayLds = C == 4 ? 16000 : 0;
 
 template <int C, int FM, int BM>
 __device__ __forceinline__ Vec<C> sample_ray(const float* __restrict__ buf, Dims3 d, float3 p) {
@@ -46,13 +55,24 @@ __device__ __forceinline__ void ray_endpoints(const RayView& v, int x, int y, co
   step = make_float3((farp.x - nearp.x) * iz, (farp.y - nearp.y) * iz, (farp.z - nearp.z) * iz);
 }
 
+// largest v >= 0 of the wave's active lanes
+__device__ __forceinline__ int wave_max(int v) {
+  int m = 0;
+#pragma unroll
+  for (int b = 30; b >= 0; --b)
+    if (__ballot(v >= (m | (1 << b)))) m |= 1 << b;
+  return m;
+}
+
 template <int C, int FM, int BM, int BL>
-__global__ __launch_bounds__(256) void k_raymarch_fwd(const float* __restrict__ input, float* __restrict__ output,
+__global__ __launch_bounds__(kTile) void k_raymarch_fwd(const float* __restrict__ input, float* __restrict__ output,
                                                       RayDims rd, RayLaunch L) {
   const int vi = blockIdx.z;
   const RayView& v = L.view[vi];
-  const int x = blockIdx.x * kTileX + (threadIdx.x % kTileX);
-  const int y = blockIdx.y * kTileY + (threadIdx.x / kTileX);
+  int tx, ty;
+  tile_of_block(blockIdx.x, (rd.out_w + kTileX - 1) / kTileX, tx, ty);
+  const int x = tx * kTileX + (threadIdx.x % kTileX);
+  const int y = ty * kTileY + (threadIdx.x / kTileX);
   if (x >= rd.out_w || y >= rd.out_h) return;
   float3 nearp, farp, step;
   ray_endpoints(v, x, y, rd, nearp, farp, step);
@@ -68,17 +88,20 @@ __global__ __launch_bounds__(256) void k_raymarch_fwd(const float* __restrict__ 
   if constexpr (FM == F_LINEAR) {
     // kRayBatch<C> samples per round trip: all their corner loads in flight
     constexpr int U = kRayBatch<C>;
+    const bool fits = offsets_fit<C>(rd.in);
     for (int i = lo; i <= hi; i += U) {
       float px[U], py[U], pz[U];
+      bool use[U];
       Vec<C> s[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const float fi = (float)min(i + u, hi);  // past the range: a repeat, not blended
+        use[u] = i + u <= hi;
+        const float fi = (float)(i + u);
         px[u] = fmaf(fi, step.x, nearp.x) - 0.5f;
         py[u] = fmaf(fi, step.y, nearp.y) - 0.5f;
         pz[u] = fmaf(fi, step.z, nearp.z) - 0.5f;
       }
-      read_linear_batch<C, BM, U>(buf, rd.in, px, py, pz, s);
+      read_linear_batch<C, BM, U>(buf, rd.in, fits, px, py, pz, use, s);
 #pragma unroll
       for (int u = 0; u < U; ++u)
         if (i + u <= hi) blend<C, BL>(acc, s[u]);
@@ -127,14 +150,16 @@ __device__ __forceinline__ void scatter_sample(float* __restrict__ grad, float* 
 }
 
 template <int C, int BM, int BL, bool EXACT>
-__global__ __launch_bounds__(256) void k_raymarch_bwd(const float* __restrict__ input,
+__global__ __launch_bounds__(kTile) void k_raymarch_bwd(const float* __restrict__ input,
                                                       const float* __restrict__ output,
                                                       const float* __restrict__ output_grad, float* __restrict__ grad,
                                                       float* __restrict__ wsum, RayDims rd, RayLaunch L) {
   const int vi = blockIdx.z;
   const RayView& v = L.view[vi];
-  const int x = blockIdx.x * kTileX + (threadIdx.x % kTileX);
-  const int y = blockIdx.y * kTileY + (threadIdx.x / kTileX);
+  int tx, ty;
+  tile_of_block(blockIdx.x, (rd.out_w + kTileX - 1) / kTileX, tx, ty);
+  const int x = tx * kTileX + (threadIdx.x % kTileX);
+  const int y = ty * kTileY + (threadIdx.x / kTileX);
   if (x >= rd.out_w || y >= rd.out_h) return;
   float3 nearp, farp, step;
   ray_endpoints(v, x, y, rd, nearp, farp, step);
@@ -183,9 +208,9 @@ __global__ __launch_bounds__(256) void k_normalize_add(float* __restrict__ total
 // ------------------------------------------------ BORDER: walk + gather
 // The BORDER backward without atomics: a walk stores every sample's gradient,
 // a voxel-block gather sums them (the transpose of the trilinear scatter).
-//   walk   : one lane per pixel, all lanes walk the whole ray in lock-step
-//            (the blend recurrences see every sample, as the scatter walk does)
-//            and store, for the samples of the pixel's clipped range, the
+//   walk   : one lane per pixel, all lanes walk in lock-step (so that a depth's
+//            stores are adjacent) the samples that can change the blend's state
+//            (below) and store, for those of the pixel's clipped range, the
 //            gradient vector that the scatter would spread, or a NaN mark for
 //            a sample the scatter skips (EXACT: outside the grid; REFERENCE:
 //            outside the band (-1, dims)). Layout [view][S][H][W][C] plus the
@@ -196,15 +221,17 @@ __global__ __launch_bounds__(256) void k_normalize_add(float* __restrict__ total
 //            REFERENCE also sums the weights and divides per view, as
 //            kNormalize3DGradients does per camera.
 template <int C, int BL, bool EXACT>
-__global__ __launch_bounds__(256) void k_raymarch_bwd_walk(const float* __restrict__ input,
+__global__ __launch_bounds__(kTile) void k_raymarch_bwd_walk(const float* __restrict__ input,
                                                            const float* __restrict__ output,
                                                            const float* __restrict__ output_grad,
                                                            float* __restrict__ gsamp, int2* __restrict__ ranges,
                                                            RayDims rd, RayLaunch L) {
   const int vi = blockIdx.z;
   const RayView& v = L.view[vi];
-  const int x = blockIdx.x * kTileX + (threadIdx.x % kTileX);
-  const int y = blockIdx.y * kTileY + (threadIdx.x / kTileX);
+  int tx, ty;
+  tile_of_block(blockIdx.x, (rd.out_w + kTileX - 1) / kTileX, tx, ty);
+  const int x = tx * kTileX + (threadIdx.x % kTileX);
+  const int y = ty * kTileY + (threadIdx.x / kTileX);
   if (x >= rd.out_w || y >= rd.out_h) return;
   float3 nearp, farp, step;
   ray_endpoints(v, x, y, rd, nearp, farp, step);
@@ -227,70 +254,83 @@ __global__ __launch_bounds__(256) void k_raymarch_bwd_walk(const float* __restri
     const float fi = (float)(S - 1 - i);
     return make_float3(fmaf(-fi, step.x, farp.x), fmaf(-fi, step.y, farp.y), fmaf(-fi, step.z, farp.z));
   };
-  for (int ib = S - 1; ib >= 0; ib -= U) {
-    // the batch's samples ib, ib-1, ... are read together when it meets the
-    // clipped range; outside the range the BORDER sample reads 0 (the blend
-    // still runs)
+  // Outside the range the samples are 0. The ADDITIVE recurrence ignores those
+  // and in the BEER_LAMBERT one the first alone can change the state (a negative
+  // or NaN depth, an infinite gradient): these walk the union of the wave's
+  // ranges. The ALPHA forms keep every step.
+  constexpr bool kSkip = C == 1 || BL == BL_ADDITIVE || BL == BL_BEER_LAMBERT;
+  int first = S - 1, last = 0;
+  if (kSkip) {
+    if (hi < S - 1) blend_grad<C, BL, EXACT>(g, vzero<C>(), acc);
+    const bool some = lo <= hi;
+    if (__ballot(some) == 0) return;
+    first = wave_max(some ? hi : 0);
+    last = S - 1 - wave_max(some ? S - 1 - lo : 0);
+  }
+  const bool fits = offsets_fit<C>(rd.in);
+  for (int ib = first; ib >= last; ib -= U) {
+    // the batch's samples ib, ib-1, ... are read together; outside the range
+    // the BORDER sample reads 0
     Vec<C> smps[U];
-    if ((ib - U + 1 <= hi) & (ib >= lo)) {
-      float px[U], py[U], pz[U];
+    float px[U], py[U], pz[U];
+    bool use[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const float3 q = position(max(ib - u, 0));
-        px[u] = q.x - 0.5f;
-        py[u] = q.y - 0.5f;
-        pz[u] = q.z - 0.5f;
-      }
-      read_linear_batch<C, B_BORDER, U>(buf, rd.in, px, py, pz, smps);
+    for (int u = 0; u < U; ++u) {
+      const int i = ib - u;
+      const float3 q = position(max(i, 0));
+      px[u] = q.x - 0.5f;
+      py[u] = q.y - 0.5f;
+      pz[u] = q.z - 0.5f;
+      use[u] = (lo <= i) & (i <= hi);
+    }
+    if (kSkip || ((ib - U + 1 <= hi) & (ib >= lo))) {
+      read_linear_batch<C, B_BORDER, U>(buf, rd.in, fits, px, py, pz, use, smps);
     } else {
 #pragma unroll
       for (int u = 0; u < U; ++u) smps[u] = vzero<C>();
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-    const int i = ib - u;
-    if (i < 0) break;
-    const float3 p = position(i);
-    const bool in_range = (lo <= i) & (i <= hi);
-    const Vec<C> smp = in_range ? smps[u] : vzero<C>();
-    const Vec<C> gs = blend_grad<C, BL, EXACT>(g, smp, acc);
-    if (in_range) {
-      const float px = p.x - 0.5f, py = p.y - 0.5f, pz = p.z - 0.5f;
-      bool counted;
-      if (EXACT) {
-        const float qx = px + 0.5f, qy = py + 0.5f, qz = pz + 0.5f;
-        counted = (0.f <= qx) & (qx < (float)rd.in.x) & (0.f <= qy) & (qy < (float)rd.in.y) & (0.f <= qz) &
-                  (qz < (float)rd.in.z);
-      } else {
-        counted = (-1.f < px) & (px < (float)rd.in.x) & (-1.f < py) & (py < (float)rd.in.y) & (-1.f < pz) &
-                  (pz < (float)rd.in.z);
+      if (ib - u < last) break;
+      Vec<C> gs;
+      if (!kSkip || use[u]) gs = blend_grad<C, BL, EXACT>(g, smps[u], acc);
+      if (use[u]) {
+        bool counted;
+        if (EXACT) {
+          const float qx = px[u] + 0.5f, qy = py[u] + 0.5f, qz = pz[u] + 0.5f;
+          counted = (0.f <= qx) & (qx < (float)rd.in.x) & (0.f <= qy) & (qy < (float)rd.in.y) & (0.f <= qz) &
+                    (qz < (float)rd.in.z);
+        } else {
+          counted = (-1.f < px[u]) & (px[u] < (float)rd.in.x) & (-1.f < py[u]) & (py[u] < (float)rd.in.y) &
+                    (-1.f < pz[u]) & (pz[u] < (float)rd.in.z);
+        }
+        Vec<C> out = gs;
+        if (!counted) out.v[0] = __builtin_nanf("");
+        vstore<C>(gview, (size_t)(ib - u) * plane + pix, out);
       }
-      Vec<C> out = gs;
-      if (!counted) out.v[0] = __builtin_nanf("");
-      vstore<C>(gview, (size_t)i * plane + pix, out);
-    }
     }
   }
 }
 
-template <int C, int WX, int WY, int WZ, bool EXACT>
-__global__ __launch_bounds__(256) void k_raymarch_bwd_gather(const float* __restrict__ gsamp,
+template <int C, int WX, int WY, int WZ, int GW, bool EXACT>
+__global__ __launch_bounds__(64 * GW) void k_raymarch_bwd_gather(const float* __restrict__ gsamp,
                                                              const int2* __restrict__ ranges,
                                                              float* __restrict__ grad, RayDims rd, ProjLaunch PL) {
   constexpr int kVox = WX * WY * WZ;
   constexpr int kCh = EXACT ? C : C + 1;  // REFERENCE keeps the weight sum as the last channel
+  constexpr int kSt = kCh | 1;            // doubles per voxel: odd, so that a row's voxels fall on different banks
   constexpr int kOwn = kVox / 64;         // voxels per lane in the per-view normalisation
   static_assert(kVox % 64 == 0, "block must be a multiple of the wave");
-  __shared__ double region[4][kVox * kCh];
+  __shared__ double region[GW][kVox * kSt];
   typedef __attribute__((address_space(3))) double lds_double;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   lds_double* acc = (lds_double*)region[wave];
   const Dims3 d = rd.in;
   const int nbx = (d.x + WX - 1) / WX, nby = (d.y + WY - 1) / WY, nbz = (d.z + WZ - 1) / WZ;
-  const int blk = blockIdx.x * 4 + wave;
+  const int blk = blockIdx.x * GW + wave;
   const bool live = blk < nbx * nby * nbz;
   const int x0 = (blk % nbx) * WX, y0 = ((blk / nbx) % nby) * WY, z0 = (blk / (nbx * nby)) * WZ;
-  for (int k = lane; k < kVox * kCh; k += 64) acc[k] = 0.0;
+  for (int k = lane; k < kVox * kSt; k += 64) acc[k] = 0.0;
   float tot[kOwn][C];
 #pragma unroll
   for (int j = 0; j < kOwn; ++j)
@@ -367,9 +407,11 @@ __global__ __launch_bounds__(256) void k_raymarch_bwd_gather(const float* __rest
         float qx = fmaf(fi0, sx, nx_) - (fx0 + 0.5f), qy = fmaf(fi0, sy, ny_) - (fy0 + 0.5f),
               qz = fmaf(fi0, sz, nz_) - (fz0 + 0.5f);
         const float* gp = gview + ((size_t)i0 * plane + pix) * C;
+        Vec<C> next = vload<C>(gp, 0);
         for (int i = i0; i <= i1; ++i) {
-          const Vec<C> gs = vload<C>(gp, 0);
+          const Vec<C> gs = next;
           gp += plane * C;
+          if (i < i1) next = vload<C>(gp, 0);
           if (gs.v[0] == gs.v[0]) {  // NaN mark: a sample the scatter skips
             const float flx = floorf(qx), fly = floorf(qy), flz = floorf(qz);
             const float tx = qx - flx, ty = qy - fly, tz = qz - flz;
@@ -389,7 +431,7 @@ __global__ __launch_bounds__(256) void k_raymarch_bwd_gather(const float* __rest
                   const int cx = lx + kx;
                   if ((unsigned)cx >= (unsigned)WX) continue;
                   const float w = wx[kx] * wyz;
-                  lds_double* a = acc + ((cz * WY + cy) * WX + cx) * kCh;
+                  lds_double* a = acc + ((cz * WY + cy) * WX + cx) * kSt;
 #pragma unroll
                   for (int c = 0; c < C; ++c)
                     __hip_atomic_fetch_add(a + c, (double)(gs.v[c] * w), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -409,7 +451,7 @@ __global__ __launch_bounds__(256) void k_raymarch_bwd_gather(const float* __rest
       // per-view normalisation by the weight sum (where positive), then clear
 #pragma unroll
       for (int j = 0; j < kOwn; ++j) {
-        lds_double* a = acc + (lane + 64 * j) * kCh;
+        lds_double* a = acc + (lane + 64 * j) * kSt;
         const float w = (float)a[C];
         if (w > 0.f) {
           const float inv = 1.0f / w;
@@ -430,7 +472,7 @@ __global__ __launch_bounds__(256) void k_raymarch_bwd_gather(const float* __rest
     if (x < d.x && y < d.y && z < d.z) {
       Vec<C> r;
 #pragma unroll
-      for (int c = 0; c < C; ++c) r.v[c] = EXACT ? (float)acc[k * kCh + c] : tot[j][c];
+      for (int c = 0; c < C; ++c) r.v[c] = EXACT ? (float)acc[k * kSt + c] : tot[j][c];
       // the caller cleared grad; chunks of views add up
       Vec<C> o = vload<C>(grad, flat3(x, y, z, d));
 #pragma unroll
@@ -445,10 +487,10 @@ template <int C, int FM, int BM>
 static hipError_t launch_fwd_bl(int bl, dim3 grid, hipStream_t s, const float* in, float* out, const RayDims& rd,
                                 const RayLaunch& L) {
   switch (bl) {
-    case BL_BEER_LAMBERT: hipLaunchKernelGGL((k_raymarch_fwd<C, FM, BM, BL_BEER_LAMBERT>), grid, dim3(256), 0, s, in, out, rd, L); break;
-    case BL_ALPHA: hipLaunchKernelGGL((k_raymarch_fwd<C, FM, BM, BL_ALPHA>), grid, dim3(256), 0, s, in, out, rd, L); break;
-    case BL_ALPHA_ADDITIVE: hipLaunchKernelGGL((k_raymarch_fwd<C, FM, BM, BL_ALPHA_ADDITIVE>), grid, dim3(256), 0, s, in, out, rd, L); break;
-    default: hipLaunchKernelGGL((k_raymarch_fwd<C, FM, BM, BL_ADDITIVE>), grid, dim3(256), 0, s, in, out, rd, L); break;
+    case BL_BEER_LAMBERT: hipLaunchKernelGGL((k_raymarch_fwd<C, FM, BM, BL_BEER_LAMBERT>), grid, dim3(kTile), kRayLds<C>, s, in, out, rd, L); break;
+    case BL_ALPHA: hipLaunchKernelGGL((k_raymarch_fwd<C, FM, BM, BL_ALPHA>), grid, dim3(kTile), kRayLds<C>, s, in, out, rd, L); break;
+    case BL_ALPHA_ADDITIVE: hipLaunchKernelGGL((k_raymarch_fwd<C, FM, BM, BL_ALPHA_ADDITIVE>), grid, dim3(kTile), kRayLds<C>, s, in, out, rd, L); break;
+    default: hipLaunchKernelGGL((k_raymarch_fwd<C, FM, BM, BL_ADDITIVE>), grid, dim3(kTile), kRayLds<C>, s, in, out, rd, L); break;
   }
   return hipGetLastError();
 }
@@ -474,7 +516,7 @@ static hipError_t launch_fwd_fm(int fm, int bm, int bl, dim3 grid, hipStream_t s
 
 hipError_t raymarch_fwd_launch(int C, int fm, int bm, int bl, hipStream_t s, const float* in, float* out,
                                const RayDims& rd, const RayLaunch& L) {
-  dim3 grid((rd.out_w + kTileX - 1) / kTileX, (rd.out_h + kTileY - 1) / kTileY, L.num_views);
+  dim3 grid(tile_blocks((rd.out_w + kTileX - 1) / kTileX, (rd.out_h + kTileY - 1) / kTileY), 1, L.num_views);
   switch (C) {
     case 1: return launch_fwd_fm<1>(fm, bm, bl, grid, s, in, out, rd, L);
     case 2: return launch_fwd_fm<2>(fm, bm, bl, grid, s, in, out, rd, L);
@@ -486,10 +528,10 @@ template <int C, int BM, bool EX>
 static hipError_t launch_bwd_bl(int bl, dim3 grid, hipStream_t s, const float* in, const float* o, const float* og,
                                 float* g, float* w, const RayDims& rd, const RayLaunch& L) {
   switch (bl) {
-    case BL_BEER_LAMBERT: hipLaunchKernelGGL((k_raymarch_bwd<C, BM, BL_BEER_LAMBERT, EX>), grid, dim3(256), 0, s, in, o, og, g, w, rd, L); break;
-    case BL_ALPHA: hipLaunchKernelGGL((k_raymarch_bwd<C, BM, BL_ALPHA, EX>), grid, dim3(256), 0, s, in, o, og, g, w, rd, L); break;
-    case BL_ALPHA_ADDITIVE: hipLaunchKernelGGL((k_raymarch_bwd<C, BM, BL_ALPHA_ADDITIVE, EX>), grid, dim3(256), 0, s, in, o, og, g, w, rd, L); break;
-    default: hipLaunchKernelGGL((k_raymarch_bwd<C, BM, BL_ADDITIVE, EX>), grid, dim3(256), 0, s, in, o, og, g, w, rd, L); break;
+    case BL_BEER_LAMBERT: hipLaunchKernelGGL((k_raymarch_bwd<C, BM, BL_BEER_LAMBERT, EX>), grid, dim3(kTile), 0, s, in, o, og, g, w, rd, L); break;
+    case BL_ALPHA: hipLaunchKernelGGL((k_raymarch_bwd<C, BM, BL_ALPHA, EX>), grid, dim3(kTile), 0, s, in, o, og, g, w, rd, L); break;
+    case BL_ALPHA_ADDITIVE: hipLaunchKernelGGL((k_raymarch_bwd<C, BM, BL_ALPHA_ADDITIVE, EX>), grid, dim3(kTile), 0, s, in, o, og, g, w, rd, L); break;
+    default: hipLaunchKernelGGL((k_raymarch_bwd<C, BM, BL_ADDITIVE, EX>), grid, dim3(kTile), 0, s, in, o, og, g, w, rd, L); break;
   }
   return hipGetLastError();
 }
@@ -511,7 +553,7 @@ static hipError_t launch_bwd_c(bool exact, int bm, int bl, dim3 grid, hipStream_
 
 hipError_t raymarch_bwd_launch(int C, bool exact, int bm, int bl, hipStream_t s, const float* in, const float* o,
                                const float* og, float* g, float* w, const RayDims& rd, const RayLaunch& L) {
-  dim3 grid((rd.out_w + kTileX - 1) / kTileX, (rd.out_h + kTileY - 1) / kTileY, L.num_views);
+  dim3 grid(tile_blocks((rd.out_w + kTileX - 1) / kTileX, (rd.out_h + kTileY - 1) / kTileY), 1, L.num_views);
   switch (C) {
     case 1: return launch_bwd_c<1>(exact, bm, bl, grid, s, in, o, og, g, w, rd, L);
     case 2: return launch_bwd_c<2>(exact, bm, bl, grid, s, in, o, og, g, w, rd, L);
@@ -534,10 +576,10 @@ template <int C, bool EX>
 static hipError_t launch_walk_bl(int bl, dim3 grid, hipStream_t s, const float* in, const float* o, const float* og,
                                  float* gs, int2* rg, const RayDims& rd, const RayLaunch& L) {
   switch (bl) {
-    case BL_BEER_LAMBERT: hipLaunchKernelGGL((k_raymarch_bwd_walk<C, BL_BEER_LAMBERT, EX>), grid, dim3(256), 0, s, in, o, og, gs, rg, rd, L); break;
-    case BL_ALPHA: hipLaunchKernelGGL((k_raymarch_bwd_walk<C, BL_ALPHA, EX>), grid, dim3(256), 0, s, in, o, og, gs, rg, rd, L); break;
-    case BL_ALPHA_ADDITIVE: hipLaunchKernelGGL((k_raymarch_bwd_walk<C, BL_ALPHA_ADDITIVE, EX>), grid, dim3(256), 0, s, in, o, og, gs, rg, rd, L); break;
-    default: hipLaunchKernelGGL((k_raymarch_bwd_walk<C, BL_ADDITIVE, EX>), grid, dim3(256), 0, s, in, o, og, gs, rg, rd, L); break;
+    case BL_BEER_LAMBERT: hipLaunchKernelGGL((k_raymarch_bwd_walk<C, BL_BEER_LAMBERT, EX>), grid, dim3(kTile), kRayLds<C>, s, in, o, og, gs, rg, rd, L); break;
+    case BL_ALPHA: hipLaunchKernelGGL((k_raymarch_bwd_walk<C, BL_ALPHA, EX>), grid, dim3(kTile), kRayLds<C>, s, in, o, og, gs, rg, rd, L); break;
+    case BL_ALPHA_ADDITIVE: hipLaunchKernelGGL((k_raymarch_bwd_walk<C, BL_ALPHA_ADDITIVE, EX>), grid, dim3(kTile), kRayLds<C>, s, in, o, og, gs, rg, rd, L); break;
+    default: hipLaunchKernelGGL((k_raymarch_bwd_walk<C, BL_ADDITIVE, EX>), grid, dim3(kTile), kRayLds<C>, s, in, o, og, gs, rg, rd, L); break;
   }
   return hipGetLastError();
 }
@@ -545,7 +587,7 @@ static hipError_t launch_walk_bl(int bl, dim3 grid, hipStream_t s, const float* 
 hipError_t raymarch_bwd_walk_launch(int C, bool exact, int bl, hipStream_t s, const float* in, const float* o,
                                     const float* og, float* gsamp, int2* ranges, const RayDims& rd,
                                     const RayLaunch& L) {
-  dim3 grid((rd.out_w + kTileX - 1) / kTileX, (rd.out_h + kTileY - 1) / kTileY, L.num_views);
+  dim3 grid(tile_blocks((rd.out_w + kTileX - 1) / kTileX, (rd.out_h + kTileY - 1) / kTileY), 1, L.num_views);
   KernelTimer t(s, "raymarch_bwd_walk");
   switch (C) {
     case 1: return exact ? launch_walk_bl<1, true>(bl, grid, s, in, o, og, gsamp, ranges, rd, L)
@@ -557,14 +599,20 @@ hipError_t raymarch_bwd_walk_launch(int C, bool exact, int bl, hipStream_t s, co
   }
 }
 
-// voxel blocks per channel count: 512, 256, 128 voxels (FP64 LDS per wave <= 5 KB)
-template <int C, int WX, int WY, int WZ>
+// Voxel blocks of one wave each, GW to a workgroup (FP64 LDS per wave up to 12
+// KB). C = 4 takes slabs of one z: 128x224x128, 5 views of 256x456, forward and
+// gradient, REFERENCE / EXACT: 16x16x1 1393 / 1228 us, 16x16x2 1394 / 1272,
+// 16x8x2 1423 / 1248, 16x8x1 1454 / 1279, 8x8x2 1501 / 1803 (EXACT with 4 doubles
+// per voxel, 1600 with 5), 8x8x8 1897. A block of 8 deep has lanes that stay 1 to
+// 9 samples in it. Below 4096 blocks there are too few waves and halves of such a
+// slab are better: 48x86x48, 3 views of 100x180: 16x16x1 184 us, 16x8x1 168.
+template <int C, int WX, int WY, int WZ, int GW>
 static hipError_t launch_gather(bool exact, hipStream_t s, const float* gsamp, const int2* ranges, float* grad,
                                 const RayDims& rd, const ProjLaunch& PL) {
   const int nb = ((rd.in.x + WX - 1) / WX) * ((rd.in.y + WY - 1) / WY) * ((rd.in.z + WZ - 1) / WZ);
-  const dim3 grid((nb + 3) / 4);
-  if (exact) hipLaunchKernelGGL((k_raymarch_bwd_gather<C, WX, WY, WZ, true>), grid, dim3(256), 0, s, gsamp, ranges, grad, rd, PL);
-  else hipLaunchKernelGGL((k_raymarch_bwd_gather<C, WX, WY, WZ, false>), grid, dim3(256), 0, s, gsamp, ranges, grad, rd, PL);
+  const dim3 grid((nb + GW - 1) / GW);
+  if (exact) hipLaunchKernelGGL((k_raymarch_bwd_gather<C, WX, WY, WZ, GW, true>), grid, dim3(64 * GW), 0, s, gsamp, ranges, grad, rd, PL);
+  else hipLaunchKernelGGL((k_raymarch_bwd_gather<C, WX, WY, WZ, GW, false>), grid, dim3(64 * GW), 0, s, gsamp, ranges, grad, rd, PL);
   return hipGetLastError();
 }
 
@@ -572,9 +620,13 @@ hipError_t raymarch_bwd_gather_launch(int C, bool exact, hipStream_t s, const fl
                                       float* grad, const RayDims& rd, const ProjLaunch& PL) {
   KernelTimer t(s, "raymarch_bwd_gather");
   switch (C) {
-    case 1: return launch_gather<1, 16, 16, 2>(exact, s, gsamp, ranges, grad, rd, PL);
-    case 2: return launch_gather<2, 16, 8, 2>(exact, s, gsamp, ranges, grad, rd, PL);
-    default: return launch_gather<4, 8, 8, 2>(exact, s, gsamp, ranges, grad, rd, PL);
+    case 1: return launch_gather<1, 16, 16, 2, 4>(exact, s, gsamp, ranges, grad, rd, PL);
+    case 2: return launch_gather<2, 16, 8, 2, 4>(exact, s, gsamp, ranges, grad, rd, PL);
+    default: {
+      const size_t slabs = (size_t)((rd.in.x + 15) / 16) * ((rd.in.y + 15) / 16) * rd.in.z;
+      return slabs < 4096 ? launch_gather<4, 16, 8, 1, 1>(exact, s, gsamp, ranges, grad, rd, PL)
+                          : launch_gather<4, 16, 16, 1, 4>(exact, s, gsamp, ranges, grad, rd, PL);
+    }
   }
 }
 
