@@ -38,6 +38,13 @@ namespace gft {
 
 constexpr int kRTileX = 16;
 constexpr int kRTileY = 16;
+// The forwards' workgroups are one wave of 16 x 4 pixels. BORDER rays are of
+// very different lengths, so their tiles are spread by tile_of_block
+// (128x224x128, 5 views of 256x456: 157 -> 127 us, four waves a workgroup 133;
+// lit 328 -> 241, 259); CLAMP and WRAP rays are all as long, and row order reads
+// a little less (96x170x96: 111 us, 115 spread).
+constexpr int kFwdTileY = 4;
+constexpr int kFwdThreads = kRTileX * kFwdTileY;
 
 // ----------------------------------------------------------------- helpers
 __device__ __forceinline__ void pixel_ray(const RayView& v, const RayDims& rd, int x, int y, float3& nearp,
@@ -203,12 +210,20 @@ __device__ __forceinline__ int wave_max(int v) {
 // samples[sample_base(pixel) + i * kSampleRun] (wave-major: one instruction's
 // stores fill two whole lines; a NaN mark for a sample outside the grid).
 template <int BM, class Q = float4>
-__global__ __launch_bounds__(256) void k_render_density_fwd(const float* __restrict__ dens, float* __restrict__ img,
+__global__ __launch_bounds__(kFwdThreads) void k_render_density_fwd(const float* __restrict__ dens, float* __restrict__ img,
                                                             RayDims rd, RayLaunch L, RenderParams rp, QuadDims q,
                                                             RenderSaved sv) {
   const RayView& v = L.view[blockIdx.z];
-  const int x = blockIdx.x * kRTileX + (threadIdx.x % kRTileX);
-  const int y = blockIdx.y * kRTileY + (threadIdx.x / kRTileX);
+  int tx, ty;
+  const int ntx = (rd.out_w + kRTileX - 1) / kRTileX;
+  if (BM == B_BORDER) {
+    tile_of_block(blockIdx.x, ntx, tx, ty);
+  } else {
+    ty = (int)(blockIdx.x / (unsigned)ntx);
+    tx = (int)(blockIdx.x - (unsigned)(ty * ntx));
+  }
+  const int x = tx * kRTileX + (threadIdx.x % kRTileX);
+  const int y = ty * kFwdTileY + (threadIdx.x / kRTileX);
   const bool valid = x < rd.out_w && y < rd.out_h;
   float D = 0.f, E = 0.f;
   if (BM == B_BORDER || BM == B_CLAMP) {
@@ -282,13 +297,18 @@ __global__ __launch_bounds__(256) void k_render_density_fwd(const float* __restr
 // mark outside the grid) and u_i (sv.samples2): the backward's absorption
 // gradient is alpha c_i + beta and its emission gradient alpha u_i.
 constexpr int kLitBatch = 4;
-__global__ __launch_bounds__(256) void k_render_density_lit_fwd(const float4* __restrict__ dq,
+// LDS asked for to keep 12 waves on a CU (20 fit): more evict each other's lines
+// of the two copies from the L1 (20 / 12 / 8 / 6 waves: 241 / 221 / 221 / 225 us)
+constexpr unsigned kLitLds = 13000;
+__global__ __launch_bounds__(kFwdThreads) void k_render_density_lit_fwd(const float4* __restrict__ dq,
                                                                 const float4* __restrict__ eq,
                                                                 float* __restrict__ img, RayDims rd, RayLaunch L,
                                                                 RenderParams rp, QuadDims q, RenderSaved sv) {
   const RayView& v = L.view[blockIdx.z];
-  const int x = blockIdx.x * kRTileX + (threadIdx.x % kRTileX);
-  const int y = blockIdx.y * kRTileY + (threadIdx.x / kRTileX);
+  int tx, ty;
+  tile_of_block(blockIdx.x, (rd.out_w + kRTileX - 1) / kRTileX, tx, ty);
+  const int x = tx * kRTileX + (threadIdx.x % kRTileX);
+  const int y = ty * kFwdTileY + (threadIdx.x / kRTileX);
   const bool valid = x < rd.out_w && y < rd.out_h;
   float D = 0.f, E = 0.f;
   float3 nearp = make_float3(0.f, 0.f, 0.f), step = make_float3(0.f, 0.f, 0.f);
@@ -961,6 +981,11 @@ static dim3 tile_grid(const RayDims& rd, int views) {
   return dim3((rd.out_w + kRTileX - 1) / kRTileX, (rd.out_h + kRTileY - 1) / kRTileY, views);
 }
 
+static dim3 fwd_grid(const RayDims& rd, bool spread, int views) {
+  const int ntx = (rd.out_w + kRTileX - 1) / kRTileX, nty = (rd.out_h + kFwdTileY - 1) / kFwdTileY;
+  return dim3(spread ? tile_blocks(ntx, nty) : (unsigned)ntx * (unsigned)nty, 1, views);
+}
+
 size_t quad_copy_floats(Dims3 d) { return quad_entries(make_quad_dims(d)) * 4; }
 size_t quad_copy_bf16_bytes(Dims3 d) { return quad_entries<uint2>(make_quad_dims<uint2>(d)) * sizeof(uint2); }
 
@@ -977,10 +1002,10 @@ hipError_t quad_copy_bf16_launch(hipStream_t s, const float* lin, void* out, Dim
 // BORDER forward from the bfloat16 corner-quad copy
 hipError_t render_density_fwd_bf16_launch(hipStream_t s, const void* quad, float* img, const RayDims& rd,
                                           const RayLaunch& L, const RenderParams& rp, const RenderSaved& sv) {
-  const dim3 grid = tile_grid(rd, L.num_views);
+  const dim3 grid = fwd_grid(rd, true, L.num_views);
   const QuadDims q = make_quad_dims<uint2>(rd.in);
   KernelTimer t(s, "render_fwd");
-  hipLaunchKernelGGL((k_render_density_fwd<B_BORDER, uint2>), grid, dim3(256), 0, s,
+  hipLaunchKernelGGL((k_render_density_fwd<B_BORDER, uint2>), grid, dim3(kFwdThreads), 0, s,
                      reinterpret_cast<const float*>(quad), img, rd, L, rp, q, sv);
   return hipGetLastError();
 }
@@ -1004,10 +1029,10 @@ hipError_t quad_copy_launch(hipStream_t s, int bm, const float* lin, float* out,
 hipError_t render_density_lit_fwd_launch(hipStream_t s, const float* dq, const float* eq, float* img,
                                          const RayDims& rd, const RayLaunch& L, const RenderParams& rp,
                                          const RenderSaved& sv) {
-  const dim3 grid = tile_grid(rd, L.num_views);
+  const dim3 grid = fwd_grid(rd, true, L.num_views);
   const QuadDims q = make_quad_dims(rd.in);
   KernelTimer t(s, "render_lit_fwd");
-  hipLaunchKernelGGL(k_render_density_lit_fwd, grid, dim3(256), 0, s, reinterpret_cast<const float4*>(dq),
+  hipLaunchKernelGGL(k_render_density_lit_fwd, grid, dim3(kFwdThreads), kLitLds, s, reinterpret_cast<const float4*>(dq),
                      reinterpret_cast<const float4*>(eq), img, rd, L, rp, q, sv);
   return hipGetLastError();
 }
@@ -1015,14 +1040,14 @@ hipError_t render_density_lit_fwd_launch(hipStream_t s, const float* dq, const f
 // BORDER, CLAMP: dens is the corner-quad copy of that boundary.
 hipError_t render_density_fwd_launch(int bm, hipStream_t s, const float* dens, float* img, const RayDims& rd,
                                      const RayLaunch& L, const RenderParams& rp, const RenderSaved& sv) {
-  const dim3 grid = tile_grid(rd, L.num_views);
+  const dim3 grid = fwd_grid(rd, bm == B_BORDER, L.num_views);
   const QuadDims q = make_quad_dims(rd.in);
   const RenderSaved none{nullptr, nullptr, nullptr};
   KernelTimer t(s, "render_fwd");
   switch (bm) {
-    case B_BORDER: hipLaunchKernelGGL(k_render_density_fwd<B_BORDER>, grid, dim3(256), 0, s, dens, img, rd, L, rp, q, sv); break;
-    case B_CLAMP: hipLaunchKernelGGL(k_render_density_fwd<B_CLAMP>, grid, dim3(256), 0, s, dens, img, rd, L, rp, q, none); break;
-    default: hipLaunchKernelGGL(k_render_density_fwd<B_WRAP>, grid, dim3(256), 0, s, dens, img, rd, L, rp, q, none); break;
+    case B_BORDER: hipLaunchKernelGGL(k_render_density_fwd<B_BORDER>, grid, dim3(kFwdThreads), 0, s, dens, img, rd, L, rp, q, sv); break;
+    case B_CLAMP: hipLaunchKernelGGL(k_render_density_fwd<B_CLAMP>, grid, dim3(kFwdThreads), 0, s, dens, img, rd, L, rp, q, none); break;
+    default: hipLaunchKernelGGL(k_render_density_fwd<B_WRAP>, grid, dim3(kFwdThreads), 0, s, dens, img, rd, L, rp, q, none); break;
   }
   return hipGetLastError();
 }
