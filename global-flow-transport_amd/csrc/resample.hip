@@ -247,7 +247,9 @@ __global__ __launch_bounds__(256) void k_mip_collapse(const float* __restrict__ 
 // LINEAR mips, 100x178x100) takes 123 us, 224-265 with rows, and C = 1 of a
 // 256x128x128 light volume 60, before 71. VALU work bounds it: the folded forms
 // and leaving out what lies outside the grid took the forward from 825 us (IEEE
-// divides, four maps per level of detail) to 332.
+// divides, four maps per level of detail) to 335. Its tiles are spread by
+// tile_of_block (those inside the grid take longest): with the mips 382 us, now
+// 340, and a blend that reads its output next 231, now 198.
 // SUM: one thread loops over the launch's views and writes (or adds) the sum
 // into slot 0, the view-summed gather of the production sampling gradient.
 constexpr int kSampleX = 8, kSampleY = 4, kSampleZ = 8;
@@ -256,9 +258,16 @@ __global__ __launch_bounds__(256) void k_sample_transform(const float* __restric
                                                           const float* __restrict__ atlas, MipTable mt, SampleCfg s,
                                                           Dims3 dout, SampleLaunch L, int runs,
                                                           float* __restrict__ out) {
-  const unsigned ntx = (unsigned)(dout.x + kSampleX - 1) / kSampleX, ty = blockIdx.x / ntx, tx = blockIdx.x - ty * ntx;
-  const int x = (int)tx * kSampleX + (int)(threadIdx.x % kSampleX);
-  const int y0 = (int)ty * kSampleY * runs + (int)(threadIdx.x / (kSampleX * kSampleZ));
+  const int ntx = (dout.x + kSampleX - 1) / kSampleX;
+  int tx, ty;
+  if (SUM) {
+    ty = (int)(blockIdx.x / (unsigned)ntx);
+    tx = (int)(blockIdx.x - (unsigned)(ty * ntx));
+  } else {
+    tile_of_block(blockIdx.x, ntx, tx, ty);
+  }
+  const int x = tx * kSampleX + (int)(threadIdx.x % kSampleX);
+  const int y0 = ty * kSampleY * runs + (int)(threadIdx.x / (kSampleX * kSampleZ));
   const size_t n = (size_t)dout.x * dout.y * dout.z;
   // (one z tile per block, but for grids deeper than the launch limit)
   for (int z = (int)(blockIdx.y * kSampleZ + threadIdx.x / kSampleX % kSampleZ); z < dout.z;
@@ -1261,7 +1270,8 @@ hipError_t sample_transform_launch(int C, int bm, bool sum, hipStream_t st, cons
   const int runs = sum ? 1 : 2;
   const int ntx = (dout.x + kSampleX - 1) / kSampleX, nty = (dout.y + kSampleY * runs - 1) / (kSampleY * runs),
             ntz = (dout.z + kSampleZ - 1) / kSampleZ;
-  const dim3 grid((unsigned)ntx * (unsigned)nty, (unsigned)std::min(ntz, 65535), sum ? 1 : L.num_views);
+  const dim3 grid(sum ? (unsigned)ntx * (unsigned)nty : tile_blocks(ntx, nty), (unsigned)std::min(ntz, 65535),
+                  sum ? 1 : L.num_views);
   const bool lod = s.mm != MIP_NONE;
   GFT_DISPATCH_C(C, GFT_DISPATCH_BM(bm, {
     auto run = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, in, atlas, mt, s, dout, L, runs, out); };
