@@ -350,6 +350,30 @@ __device__ __forceinline__ float column_lod(const Column& c, float fi) {
   return fmaxf(0.f, 0.5f * log2f(fmaxf(fx, fmaxf(fy, fz))));
 }
 
+// The same for a run of samples from index i0: the squared footprints are
+// quadratics in the index, taken around i0 (no large terms cancel there).
+struct LodRun {
+  float3 a, b, c;
+};
+__device__ __forceinline__ LodRun lod_run(const Column& k, float i0) {
+  const float3 ex = fma3(i0, k.ex1, k.ex0), ey = fma3(i0, k.ey1, k.ey0);
+  LodRun r;
+  r.a = make_float3(fmaf(ex.x, ex.x, fmaf(ey.x, ey.x, k.dp.x * k.dp.x)),
+                    fmaf(ex.y, ex.y, fmaf(ey.y, ey.y, k.dp.y * k.dp.y)),
+                    fmaf(ex.z, ex.z, fmaf(ey.z, ey.z, k.dp.z * k.dp.z)));
+  r.b = make_float3(2.f * fmaf(ex.x, k.ex1.x, ey.x * k.ey1.x), 2.f * fmaf(ex.y, k.ex1.y, ey.y * k.ey1.y),
+                    2.f * fmaf(ex.z, k.ex1.z, ey.z * k.ey1.z));
+  r.c = make_float3(fmaf(k.ex1.x, k.ex1.x, k.ey1.x * k.ey1.x), fmaf(k.ex1.y, k.ex1.y, k.ey1.y * k.ey1.y),
+                    fmaf(k.ex1.z, k.ex1.z, k.ey1.z * k.ey1.z));
+  return r;
+}
+// level of detail of sample i0 + j (a subnormal square is below level 0 anyway)
+__device__ __forceinline__ float run_lod(const LodRun& r, float j) {
+  const float fx = fmaf(j, fmaf(j, r.c.x, r.b.x), r.a.x), fy = fmaf(j, fmaf(j, r.c.y, r.b.y), r.a.y),
+              fz = fmaf(j, fmaf(j, r.c.z, r.b.z), r.a.z);
+  return fmaxf(0.f, 0.5f * __builtin_amdgcn_logf(fmaxf(fx, fmaxf(fy, fz))));
+}
+
 // U samples' BORDER trilinear values at one level from its corner-quad copy,
 // (p / 2^m - 0.5) in cell coordinates, every load in flight before any value
 // is used: make_taps' inside test, corners and lerp order, as read_linear (an
@@ -430,50 +454,75 @@ __global__ __launch_bounds__(kTilePix) void k_batch_fwd(const BatchRec* __restri
       int lo, hi;
       clip_ray(col.p0, col.dp, R.mt.dims[0], S, 0.f, lo, hi);
       float* __restrict__ cs = R.csave + (size_t)local * S * kTilePix + threadIdx.x;
-      for (int ib = lo; ib <= hi; ib += kFwdBatch) {
-        // kFwdBatch samples at a time: per mip level any of them reads, all
-        // their loads in flight
-        float3 p[kFwdBatch];
-        int lv[kFwdBatch][2], nl[kFwdBatch];
-        float lw[kFwdBatch][2], vf[kFwdBatch], vc[kFwdBatch];
-#pragma unroll
-        for (int u = 0; u < kFwdBatch; ++u) {
-          const float fi = (float)(ib + u);
-          p[u] = fma3(fi, col.dp, col.p0);
-          nl[u] = level_taps(cfg, mips ? column_lod(col, fi) : 0.f, lv[u], lw[u]);
-          vf[u] = vc[u] = 0.f;
-        }
-#pragma unroll
-        for (int m = 0; m <= kBatchMaxLevels; ++m) {
-          if (m > R.mt.levels) break;
-          bool use[kFwdBatch], any = false;
+      auto blend = [&](int i, float val) {
+        const float sigma = R.step * val;
+        D += sigma;
+        const float e = __expf(-D);
+        cs[(size_t)i * kTilePix] = e + E;
+        E = fmaf(e, sigma, E);
+      };
+      if (mips && lo <= hi) lmax = fmaxf(column_lod(col, (float)lo), column_lod(col, (float)hi));
+      if (__ballot(lmax > 0.f) == 0) {
+        // no column of the wave leaves level 0 (a camera of at least a pixel and
+        // a depth sample to the cell)
+        for (int ib = lo; ib <= hi; ib += kFwdBatch) {
+          float3 p[kFwdBatch];
+          bool use[kFwdBatch];
 #pragma unroll
           for (int u = 0; u < kFwdBatch; ++u) {
-            use[u] = (ib + u <= hi) & ((lv[u][0] == m) | ((nl[u] == 2) & (lv[u][1] == m)));
-            any |= use[u];
+            p[u] = fma3((float)(ib + u), col.dp, col.p0);
+            use[u] = ib + u <= hi;
           }
-          if (!any) continue;
           float val[kFwdBatch];
-          quad_read_batch<kFwdBatch>((const gcf32x4*)R.quad[m], R.qd[m], R.mt.dims[m], p, 1.f / (float)(1 << m),
-                                     use, val);
+          quad_read_batch<kFwdBatch>((const gcf32x4*)R.quad[0], R.qd[0], R.mt.dims[0], p, 1.f, use, val);
 #pragma unroll
-          for (int u = 0; u < kFwdBatch; ++u)
-            if (use[u]) {
-              if (lv[u][0] == m) vf[u] = val[u];
-              else vc[u] = val[u];
-            }
+          for (int u = 0; u < kFwdBatch; ++u) {
+            if (ib + u > hi) break;
+            blend(ib + u, val[u]);
+          }
         }
+      } else {
+        const LodRun run = lod_run(col, (float)lo);
+        for (int ib = lo; ib <= hi; ib += kFwdBatch) {
+          // kFwdBatch samples at a time: per mip level any of them reads, all
+          // their loads in flight
+          float3 p[kFwdBatch];
+          int lv[kFwdBatch][2], nl[kFwdBatch];
+          float lw[kFwdBatch][2], vf[kFwdBatch], vc[kFwdBatch];
 #pragma unroll
-        for (int u = 0; u < kFwdBatch; ++u) {
-          if (ib + u > hi) break;
-          const float sigma = R.step * (nl[u] == 2 ? lerpf(vf[u], vc[u], lw[u][1]) : vf[u]);
-          D += sigma;
-          const float e = __expf(-D);
-          cs[(size_t)(ib + u) * kTilePix] = e + E;
-          E = fmaf(e, sigma, E);
+          for (int u = 0; u < kFwdBatch; ++u) {
+            const float fi = (float)(ib + u);
+            p[u] = fma3(fi, col.dp, col.p0);
+            nl[u] = level_taps(cfg, run_lod(run, (float)(ib + u - lo)), lv[u], lw[u]);
+            vf[u] = vc[u] = 0.f;
+          }
+#pragma unroll
+          for (int m = 0; m <= kBatchMaxLevels; ++m) {
+            if (m > R.mt.levels) break;
+            bool use[kFwdBatch], any = false;
+#pragma unroll
+            for (int u = 0; u < kFwdBatch; ++u) {
+              use[u] = (ib + u <= hi) & ((lv[u][0] == m) | ((nl[u] == 2) & (lv[u][1] == m)));
+              any |= use[u];
+            }
+            if (!any) continue;
+            float val[kFwdBatch];
+            quad_read_batch<kFwdBatch>((const gcf32x4*)R.quad[m], R.qd[m], R.mt.dims[m], p, 1.f / (float)(1 << m),
+                                       use, val);
+#pragma unroll
+            for (int u = 0; u < kFwdBatch; ++u)
+              if (use[u]) {
+                if (lv[u][0] == m) vf[u] = val[u];
+                else vc[u] = val[u];
+              }
+          }
+#pragma unroll
+          for (int u = 0; u < kFwdBatch; ++u) {
+            if (ib + u > hi) break;
+            blend(ib + u, nl[u] == 2 ? lerpf(vf[u], vc[u], lw[u][1]) : vf[u]);
+          }
         }
       }
-      if (mips && lo <= hi) lmax = fmaxf(column_lod(col, (float)lo), column_lod(col, (float)hi));
       const size_t pix = ((size_t)vi * R.out_h + y) * R.out_w + x;
       reinterpret_cast<float4*>(R.images)[pix] = make_float4(R.light[0] * E, R.light[1] * E, R.light[2] * E, D);
       const float* tg = R.target + pix * 3;
@@ -514,7 +563,13 @@ __global__ __launch_bounds__(kTilePix) void k_batch_fwd(const BatchRec* __restri
 // c_a|)); samples outside a level (BORDER) add nothing to it. The sums run in
 // a fixed order and one store per voxel follows.
 typedef __attribute__((address_space(3))) double lds_f64;  // an FP64 LDS region
-constexpr int kGatherBatch = 4;  // c_k loaded per round trip
+// c_k loaded per round trip, and the waves per SIMD that the registers are held
+// to (110 VGPRs, 4 waves, otherwise). The gather is bound by VALU work and LDS
+// atomics together; ten uneven reconstructions with mips, us (batch 1 / 2 / 3 /
+// 4): 4 waves - / - / - / 1534; 5: 1468 / 1395 / - / 1385; 6: 1454 / 1336 / 1333 /
+// 1358. Without mips: 4: 651 (4); 5: 597 (2), 592 (4); 6: 595 (2), 589 (3), 608 (4).
+constexpr int kGatherBatch = 3;
+constexpr int kGatherOccupancy = 6;
 // waves that share a voxel block: they take its pixel batches in turn, each
 // into regions of its own
 // (ten uneven reconstructions, gather: 1 wave 2.80 ms, 2: 2.02, 4: 1.66, 8:
@@ -532,11 +587,10 @@ constexpr int kL1Stride = kBlockVox / 8 + 1;  // odd: the copies start on differ
 constexpr int kL0Stride = kBlockVox + 1;
 
 // add a sample's level tap to the block region acc (block W x H x Z with
-// WXY = W H, origin o, (qx, qy, qz) in the level's cell coordinates, g the
-// weighted gradient); corners outside the block are skipped
+// WXY = W H, (rx, ry, rz) in the level's cell coordinates from the block's
+// origin, g the weighted gradient); corners outside the block are skipped
 __device__ __forceinline__ void gather_tap(__attribute__((address_space(3))) double* acc, int WX, int WY, int WZ,
-                                           int WXY, int ox, int oy, int oz, float qx, float qy, float qz, float g) {
-  const float rx = qx - (float)ox, ry = qy - (float)oy, rz = qz - (float)oz;
+                                           float rx, float ry, float rz, float g) {
   const float flx = floorf(rx), fly = floorf(ry), flz = floorf(rz);
   const float tx = rx - flx, ty = ry - fly, tz = rz - flz;
   const int lx = (int)flx, ly = (int)fly, lz = (int)flz;
@@ -552,11 +606,11 @@ __device__ __forceinline__ void gather_tap(__attribute__((address_space(3))) dou
     for (int ky = 0; ky < 2; ++ky) {
       if (!vy[ky]) continue;
       const float wyz = wy[ky] * wz[kz];
-      const int row = base + (kz ? WXY : 0) + (ky ? WX : 0);
+      const int at = base + (kz ? WX * WY : 0) + (ky ? WX : 0);
 #pragma unroll
       for (int kx = 0; kx < 2; ++kx) {
         if (!vx[kx]) continue;
-        __hip_atomic_fetch_add(acc + row + kx, (double)(wx[kx] * wyz), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __hip_atomic_fetch_add(acc + at + kx, (double)(wx[kx] * wyz), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
     }
   }
@@ -592,13 +646,12 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
   for (int k = lane; k < kVox; k += 64) acc[k] = 0.0;
   int turn = wave;  // pixel batches, counted through the views, until this wave's next one
   // support box (object space) of the block's cells; PAIR: of its level-1 cells
-  const int mb = two ? 1 : m;
-  const float s2 = (float)(1 << mb), sc = 1.f / (float)(1 << m);
-  const int bx = two ? x0 / 2 : x0, by = two ? y0 / 2 : y0, bz = two ? z0 / 2 : z0;
-  const int bwx = two ? WX / 2 : WX, bwy = two ? WY / 2 : WY, bwz = two ? WZ / 2 : WZ;
-  const float b0[3] = {((float)bx - 0.5f) * s2, ((float)by - 0.5f) * s2, ((float)bz - 0.5f) * s2};
-  const float b1[3] = {((float)(bx + bwx) + 0.5f) * s2, ((float)(by + bwy) + 0.5f) * s2,
-                       ((float)(bz + bwz) + 0.5f) * s2};
+  const float sm = (float)(1 << m), sc = 1.f / sm;
+  // a sample that reaches a cell of a block clear of the grids' faces lies in the
+  // grid of that cell's level
+  const bool inner = (x0 > 0) & (y0 > 0) & (z0 > 0) &
+                     (two ? (x0 + WX < 2 * d1.x) & (y0 + WY < 2 * d1.y) & (z0 + WZ < 2 * d1.z)
+                          : (x0 + WX < dm.x) & (y0 + WY < dm.y) & (z0 + WZ < dm.z));
   const int S = R.out_d;
   const float inv_s1 = column_rcp(S);
   const bool mips = R.mt.levels > 0;
@@ -608,6 +661,15 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
   for (int vi = 0; vi < R.num_views; ++vi) {
     if (!PAIR && __int_as_float(R.lodmax[vi]) <= (float)(m - 1)) continue;  // no sample reads level m
     const ColumnView& cv = R.view[vi];
+    // a view whose samples all read level 0 alone takes the voxels' own box and
+    // no level of detail
+    const bool pair = two && __int_as_float(R.lodmax[vi]) > 0.f;
+    const float s2 = pair ? 2.f : sm;
+    const int bx = pair ? x0 / 2 : x0, by = pair ? y0 / 2 : y0, bz = pair ? z0 / 2 : z0;
+    const int bwx = pair ? WX / 2 : WX, bwy = pair ? WY / 2 : WY, bwz = pair ? WZ / 2 : WZ;
+    const float b0[3] = {((float)bx - 0.5f) * s2, ((float)by - 0.5f) * s2, ((float)bz - 0.5f) * s2};
+    const float b1[3] = {((float)(bx + bwx) + 0.5f) * s2, ((float)(by + bwy) + 0.5f) * s2,
+                         ((float)(bz + bwz) + 0.5f) * s2};
     const float* A = cv.pmv;
     float mnx = 3.4e38f, mxx = -3.4e38f, mny = 3.4e38f, mxy = -3.4e38f;
     bool behind = false;
@@ -665,7 +727,7 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
       }
       const int lo = __float_as_int(rec.x), hi = __float_as_int(rec.y);
       if (lo > hi) continue;
-      const Column col = column_of(cv, cpx, cpy, inv_s1, mips);
+      const Column col = column_of(cv, cpx, cpy, inv_s1, PAIR ? pair : true);
       // the column's samples in the support box (one hundredth of a sample of
       // slack); a zero step component (reciprocal inf) gives (-inf, inf) for
       // a column inside that slab and an empty range outside it
@@ -681,6 +743,9 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
       if (!(tlo <= thi + 1.f)) continue;  // (also a NaN slab: 0 * inf)
       // tlo, thi lie within [lo, hi] here, so the conversions stay in range
       const int i0 = max(lo, (int)ceilf(tlo - 1e-2f)), i1 = min(hi, (int)floorf(thi + 1e-2f));
+      const LodRun run = lod_run(col, (float)i0);
+      const float r0x = col.p0.x - 0.5f - (float)x0, r0y = col.p0.y - 0.5f - (float)y0,
+                  r0z = col.p0.z - 0.5f - (float)z0;
       const gcfloat* __restrict__ cs = (const gcfloat*)R.csave + ((size_t)it * S) * kTilePix + slot;
       for (int ib = i0; ib <= i1; ib += kGatherBatch) {
         float cv4[kGatherBatch];
@@ -691,24 +756,32 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
           const int i = ib + u;
           if (i > i1) break;
           const float fi = (float)i;
-          const float l = mips ? fminf(column_lod(col, fi), lmaxf) : 0.f;
-          const int fl = (int)l;
-          const float fr = l - (float)fl;
           const float g = fmaf(rec.z, cv4[u], rec.w);
-          const float3 p = fma3(fi, col.dp, col.p0);
-          const float wm = mip_weight(m, fl, fr);
-          if (wm != 0.f) {
-            const float qx = p.x * sc - 0.5f, qy = p.y * sc - 0.5f, qz = p.z * sc - 0.5f;
-            if (inside_level(qx, qy, qz, dm)) gather_tap(acc, WX, WY, WZ, WX * WY, x0, y0, z0, qx, qy, qz, g * wm);
-          }
-          if (two) {
-            const float w1 = mip_weight(1, fl, fr);
-            if (w1 != 0.f) {
-              const float qx = p.x * 0.5f - 0.5f, qy = p.y * 0.5f - 0.5f, qz = p.z * 0.5f - 0.5f;
-              if (inside_level(qx, qy, qz, d1))
-                gather_tap(acc1, WX / 2, WY / 2, WZ / 2, (WX / 2) * (WY / 2), x0 / 2, y0 / 2, z0 / 2, qx, qy, qz,
-                           g * w1);
+          if constexpr (PAIR) {
+            // weights of levels 0 and 1 (mip_weight), zero outside a level
+            const float l = pair ? fminf(run_lod(run, (float)(i - i0)), lmaxf) : 0.f;
+            float w0 = fmaxf(1.f - l, 0.f), w1 = pair ? fmaxf(fminf(l, 2.f - l), 0.f) : 0.f;
+            float rx = fmaf(fi, col.dp.x, r0x), ry = fmaf(fi, col.dp.y, r0y), rz = fmaf(fi, col.dp.z, r0z);
+            if (!inner) {
+              const float3 p = fma3(fi, col.dp, col.p0);
+              const float qx = p.x - 0.5f, qy = p.y - 0.5f, qz = p.z - 0.5f;
+              w0 = inside_level(qx, qy, qz, dm) ? w0 : 0.f;
+              w1 = inside_level(p.x * 0.5f - 0.5f, p.y * 0.5f - 0.5f, p.z * 0.5f - 0.5f, d1) ? w1 : 0.f;
             }
+            if (w0 != 0.f) gather_tap(acc, WX, WY, WZ, rx, ry, rz, g * w0);
+            // (x0, y0, z0 are even: level 1 is (p / 2 - 0.5) - x0 / 2)
+            if (w1 != 0.f)
+              gather_tap(acc1, WX / 2, WY / 2, WZ / 2, fmaf(0.5f, rx, -0.25f),
+                         fmaf(0.5f, ry, -0.25f), fmaf(0.5f, rz, -0.25f), g * w1);
+          } else {
+            const float l = fminf(run_lod(run, (float)(i - i0)), lmaxf);
+            const int fl = (int)l;
+            const float wm = mip_weight(m, fl, l - (float)fl);
+            if (wm == 0.f) continue;
+            const float3 p = fma3(fi, col.dp, col.p0);
+            const float qx = p.x * sc - 0.5f, qy = p.y * sc - 0.5f, qz = p.z * sc - 0.5f;
+            if (inside_level(qx, qy, qz, dm))
+              gather_tap(acc, WX, WY, WZ, qx - (float)x0, qy - (float)y0, qz - (float)z0, g * wm);
           }
         }
       }
@@ -775,7 +848,7 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
 }
 
 template <bool PAIR>
-__global__ __launch_bounds__(64 * kGatherWaves) void k_batch_gather(const BatchRec* __restrict__ recs, int nrec, int m,
+__global__ __launch_bounds__(64 * kGatherWaves, kGatherOccupancy) void k_batch_gather(const BatchRec* __restrict__ recs, int nrec, int m,
                                                                     int total_items) {
   constexpr int kVox = kL0Stride + (PAIR ? kL1Copies * kL1Stride : 0);
   __shared__ double region[kGatherWaves * kVox];
