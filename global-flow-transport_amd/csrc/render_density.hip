@@ -397,14 +397,15 @@ __device__ __forceinline__ void pixel_grad(const float* __restrict__ img, const 
   }
 }
 
+template <int NT>
 __device__ __forceinline__ void block_loss(float sq, float* __restrict__ loss, float scale) {
-  __shared__ float red[256 / 64];
+  __shared__ float red[NT / 64];
   for (int off = 32; off > 0; off >>= 1) sq += __shfl_down(sq, off, 64);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sq;
   __syncthreads();
   if (threadIdx.x == 0) {
     float s = 0.f;
-    for (int w = 0; w < 256 / 64; ++w) s += red[w];
+    for (int w = 0; w < NT / 64; ++w) s += red[w];
     atomic_addf(loss, s * scale);
   }
 }
@@ -687,7 +688,7 @@ __global__ __launch_bounds__(64 * NW) void k_render_density_bwd_gather(RenderSav
 }
 
 // ----------------------------------------- CLAMP: tiled LDS pre-reduction
-// A workgroup owns a 16x16 pixel tile and walks its rays in lock-step
+// A workgroup is one wave of 16x4 pixels and walks its rays in lock-step
 // segments of K samples from far to near. The samples of a segment lie in the
 // convex hull of the tile's four corner rays at the segment's first and last
 // sample (the index->object map is projective), so their trilinear corners fit
@@ -695,7 +696,10 @@ __global__ __launch_bounds__(64 * NW) void k_render_density_bwd_gather(RenderSav
 // and flushed once per segment with coalesced global atomics (zero entries
 // skipped). A brick over the LDS capacity goes straight to global atomics.
 constexpr int kSegK = 8;
-constexpr int kCap = 6144;  // FP64 brick cells: ds_add_f64 is ~20x faster than ds_add_f32 on gfx950
+// FP64 brick cells (ds_add_f64 is ~20x faster than ds_add_f32 on gfx950): as many
+// as leave room for 8 waves on a CU. One more wave less costs more than the few
+// larger bricks gain, smaller bricks much more (below).
+constexpr int kCap = 2400;
 // more than any rounding of a sample's position against the corner rays'
 constexpr float kBrickSlack = 1e-2f;
 
@@ -740,7 +744,8 @@ __device__ __forceinline__ Brick segment_brick(const float3* cn, const float3* c
     }
     b.lo[a] = lo;
     b.n[a] = hi - lo + 2;
-    b.size = hi < lo ? 0 : b.size * b.n[a];
+    // (past the capacity it only has to stay there)
+    b.size = hi < lo ? 0 : (b.size > kCap ? b.size : b.size * min(b.n[a], 1 << 19));
   }
   return b;
 }
@@ -754,33 +759,36 @@ __device__ __forceinline__ Brick segment_brick(const float3* cn, const float3* c
 // and the next one weight 0. Most of a CLAMP ray's samples lie outside along
 // some axis, often a whole wave's, so the upper corners of an axis are left
 // out where no lane of the wave has a weight there.
-// The kernel is bound by VALU work (half its cycles) and LDS atomics (0.4)
-// together at 12 waves a CU; 128x224x128, 5 views of 256x456: 0.912 ms, 1.060
-// with a bounds test per corner and a flush per segment; segments of 4, 5, 6 or
-// 12 samples and bricks of 3072 to 8192 cells: 0.95 to 2.6 ms.
+// The kernel is bound by VALU work, LDS atomics and, with few tiles, its serial
+// chain of segments. Tiles of one wave wait for no other and are four times as
+// many as 16x16 ones (in brackets; bricks of 6144 cells). us: 30x34x29, 1 view
+// of 72x85 36 (72); 60x104x59, 3 of 130x220 124 (141); 96x170x96, 5 of 222x395
+// 504 (562); 128x224x128, 5 of 256x456 917 (913). There, bricks of 1536 / 2048 /
+// 2304 / 2560 / 3072 cells: 3114 / 1064 / 912 / 990 / 1073; segments of 4 / 6:
+// 1020 / 905, but 585 / 518 at 96x170x96. BORDER at 128x224x128: 560 (953).
 // BORDER (the recompute alternative to the saved-state gather: nothing is
 // kept from the forward but the images) walks only the segments of the
 // tile's clipped sample ranges; samples outside the grid read 0 and corners
 // outside it take no gradient. Its global float atomics make the summation
 // order, and so the last bits, vary from run to run.
-template <bool L2, int BM = B_CLAMP>
-__global__ __launch_bounds__(256) void k_render_density_bwd_clamp(const float4* __restrict__ quad, QuadDims q,
+template <bool L2, int BM>
+__global__ __launch_bounds__(64) void k_render_density_bwd_clamp(const float4* __restrict__ quad, QuadDims q,
                                                                   const float* __restrict__ img,
                                                                   const float* __restrict__ second,
                                                                   float* __restrict__ grad, float* __restrict__ loss,
                                                                   RayDims rd, RayLaunch L, RenderParams rp) {
-  __shared__ double lg[kCap];
-  __shared__ int seg_range[2];
+  __shared__ double cells[kCap];
   typedef __attribute__((address_space(3))) double lds_double;
-  lds_double* brick = (lds_double*)lg;
+  const int lane = (int)threadIdx.x;
+  lds_double* brick = (lds_double*)cells;
   const RayView& v = L.view[blockIdx.z];
-  const int x0 = blockIdx.x * kRTileX, y0 = blockIdx.y * kRTileY;
-  const int x = x0 + (threadIdx.x % kRTileX), y = y0 + (threadIdx.x / kRTileX);
+  const int x0 = blockIdx.x * kRTileX, y0 = blockIdx.y * kFwdTileY;
+  const int x = x0 + lane % kRTileX, y = y0 + lane / kRTileX;
   const bool active = x < rd.out_w && y < rd.out_h;
   float* gout = grad + rd.in_batch_stride * v.in_batch;
   float3 cn[4], cs[4];
   {
-    const int x1 = min(x0 + kRTileX - 1, rd.out_w - 1), y1 = min(y0 + kRTileY - 1, rd.out_h - 1);
+    const int x1 = min(x0 + kRTileX - 1, rd.out_w - 1), y1 = min(y0 + kFwdTileY - 1, rd.out_h - 1);
     const int px[4] = {x0, x1, x0, x1}, py[4] = {y0, y0, y1, y1};
 #pragma unroll
     for (int c = 0; c < 4; ++c) pixel_ray(v, rd, px[c], py[c], cn[c], cs[c]);
@@ -792,7 +800,13 @@ __global__ __launch_bounds__(256) void k_render_density_bwd_clamp(const float4* 
     pixel_ray(v, rd, x, y, nearp, step);
   }
   const bool walk = active && (G != 0.f || gD != 0.f);
-  for (int i = threadIdx.x; i < kCap; i += 256) lg[i] = 0.0;
+  // the workgroup is one wave, whose LDS operations are in order: no barrier
+  auto wave_sync = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  for (int i = lane; i < kCap; i += 64) brick[i] = 0.0;
+  wave_sync();
   const int S = rd.out_d;
   const float mx = (float)(rd.in.x - 1), my = (float)(rd.in.y - 1), mz = (float)(rd.in.z - 1);
   int sg_lo = 0, sg_hi = (S + kSegK - 1) / kSegK - 1;
@@ -801,37 +815,25 @@ __global__ __launch_bounds__(256) void k_render_density_bwd_clamp(const float4* 
     int lo = 1, hi = 0;
     if (walk) clip_ray(nearp, step, rd.in, S, 0.f, lo, hi);
     const int wlo = wave_min(lo <= hi ? lo : S), whi = wave_max(lo <= hi ? hi : -1);
-    if (threadIdx.x == 0) {
-      seg_range[0] = S;
-      seg_range[1] = -1;
-    }
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) {
-      atomicMin(&seg_range[0], wlo);
-      atomicMax(&seg_range[1], whi);
-    }
-    __syncthreads();
-    sg_lo = seg_range[0] / kSegK;
-    sg_hi = seg_range[1] < 0 ? -1 : seg_range[1] / kSegK;
-  } else {
-    __syncthreads();
+    sg_lo = wlo / kSegK;
+    sg_hi = whi < 0 ? -1 : whi / kSegK;
   }
-  // adds the brick's sums to the gradient and clears it (every thread of the workgroup)
+  // adds the brick's sums to the gradient and clears it
   auto flush = [&](const Brick& br) {
     if (br.size == 0 || br.size > kCap) return;
-    __syncthreads();
+    wave_sync();
     const int nx = br.n[0], ny = br.n[1];
-    const int q = 256 / nx, r = 256 - q * nx;
-    int bx = threadIdx.x % nx, t = threadIdx.x / nx;
+    const int q = 64 / nx, r = 64 - q * nx;
+    int bx = lane % nx, t = lane / nx;
     int by = t % ny, bz = t / ny;
-    for (int idx = threadIdx.x; idx < br.size; idx += 256) {
-      const float val = (float)lg[idx];
+    for (int idx = lane; idx < br.size; idx += 64) {
+      const float val = (float)brick[idx];
       if (val != 0.f) {
         const int cx = br.lo[0] + bx, cy = br.lo[1] + by, cz = br.lo[2] + bz;
         if (((unsigned)cx < (unsigned)rd.in.x) & ((unsigned)cy < (unsigned)rd.in.y) & ((unsigned)cz < (unsigned)rd.in.z))
           atomic_addf(gout + flat3(cx, cy, cz, rd.in), val);
       }
-      lg[idx] = 0.0;
+      brick[idx] = 0.0;
       bx += r;
       by += q;
       if (bx >= nx) {
@@ -843,7 +845,7 @@ __global__ __launch_bounds__(256) void k_render_density_bwd_clamp(const float4* 
         ++bz;
       }
     }
-    __syncthreads();
+    wave_sync();
   };
   // consecutive segments often share a brick (all their samples clamp to the
   // same boundary cells): it is flushed when the next one differs
@@ -919,7 +921,18 @@ __global__ __launch_bounds__(256) void k_render_density_bwd_clamp(const float4* 
     }
   }
   flush(held);
-  if (L2) block_loss(sq, loss, rp.loss_scale);
+  if (L2 && (blockIdx.y & 3) == 0) {
+    // one wave adds the loss of four tiles: as many additions as there are waves
+    // would leave 1.5e-6 of rounding in it (7000 of them)
+    for (int r = 1; r < 4; ++r) {
+      const int yr = y + r * kFwdTileY;
+      if (x >= rd.out_w || yr >= rd.out_h) break;
+      float g, gd, d, t;
+      pixel_grad<L2>(img, second, rd, v, size_t(yr) * rd.out_w + x, rp, g, gd, d, t);
+      sq += t;
+    }
+    block_loss<64>(sq, loss, rp.loss_scale);
+  }
 }
 
 // -------------------------------------------------- WRAP: global atomics
@@ -973,7 +986,7 @@ __global__ __launch_bounds__(256) void k_render_density_bwd_wrap(const float* __
       }
     }
   }
-  if (L2) block_loss(sq, loss, rp.loss_scale);
+  if (L2) block_loss<256>(sq, loss, rp.loss_scale);
 }
 
 // ---------------------------------------------------------------- launches
@@ -1126,16 +1139,17 @@ hipError_t render_density_scatter_launch(int bm, bool l2, hipStream_t s, const f
                                          const RayLaunch& L, const RenderParams& rp) {
   const dim3 grid = tile_grid(rd, L.num_views);
   KernelTimer t(s, "render_bwd_scatter");
-  if (bm == B_CLAMP) {
+  if (bm == B_CLAMP || bm == B_BORDER) {
     const float4* quad = reinterpret_cast<const float4*>(dens);
     const QuadDims q = make_quad_dims(rd.in);
-    if (l2) hipLaunchKernelGGL(k_render_density_bwd_clamp<true>, grid, dim3(256), 0, s, quad, q, img, second, grad, loss, rd, L, rp);
-    else hipLaunchKernelGGL(k_render_density_bwd_clamp<false>, grid, dim3(256), 0, s, quad, q, img, second, grad, loss, rd, L, rp);
-  } else if (bm == B_BORDER) {
-    const float4* quad = reinterpret_cast<const float4*>(dens);
-    const QuadDims q = make_quad_dims(rd.in);
-    if (l2) hipLaunchKernelGGL((k_render_density_bwd_clamp<true, B_BORDER>), grid, dim3(256), 0, s, quad, q, img, second, grad, loss, rd, L, rp);
-    else hipLaunchKernelGGL((k_render_density_bwd_clamp<false, B_BORDER>), grid, dim3(256), 0, s, quad, q, img, second, grad, loss, rd, L, rp);
+    const dim3 tiles(grid.x, (rd.out_h + kFwdTileY - 1) / kFwdTileY, grid.z);
+    auto run = [&](auto kern) {
+      hipLaunchKernelGGL(kern, tiles, dim3(64), 0, s, quad, q, img, second, grad, loss, rd, L, rp);
+    };
+    if (bm == B_CLAMP && l2) run(k_render_density_bwd_clamp<true, B_CLAMP>);
+    else if (bm == B_CLAMP) run(k_render_density_bwd_clamp<false, B_CLAMP>);
+    else if (l2) run(k_render_density_bwd_clamp<true, B_BORDER>);
+    else run(k_render_density_bwd_clamp<false, B_BORDER>);
   } else {
     if (l2) hipLaunchKernelGGL(k_render_density_bwd_wrap<true>, grid, dim3(256), 0, s, dens, img, second, grad, loss, rd, L, rp);
     else hipLaunchKernelGGL(k_render_density_bwd_wrap<false>, grid, dim3(256), 0, s, dens, img, second, grad, loss, rd, L, rp);
