@@ -623,6 +623,7 @@ struct LutLaunch {
   int relative;
   int normalized;
   int batch0;
+  int fresh;      // LINEAR gradient: the table's gradient is written, not added to
 };
 
 // ------------------------------------------------------ kernel timers

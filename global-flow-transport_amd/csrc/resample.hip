@@ -767,7 +767,7 @@ __global__ __launch_bounds__(256) void k_sample_lut_bwd(const float* __restrict_
         ly *= dout.y;
         lz *= dout.z;
       }
-      float4 o = *dst;
+      const float4 o = L.fresh ? make_float4(0.f, 0.f, 0.f, 0.f) : *dst;
       *dst = make_float4(o.x + lx, o.y + ly, o.z + lz, o.w);
     } else {
       *dst = make_float4(lx, ly, lz, 0.f);
@@ -852,7 +852,7 @@ __global__ __launch_bounds__(256) void k_sample_lut_bwd_tiled(const float* __res
           ly *= dout.y;
           lz *= dout.z;
         }
-        const float4 o = *dst;
+        const float4 o = L.fresh ? make_float4(0.f, 0.f, 0.f, 0.f) : *dst;
         *dst = make_float4(o.x + lx, o.y + ly, o.z + lz, o.w);
       } else {
         *dst = make_float4(lx, ly, lz, 0.f);
