@@ -382,7 +382,7 @@ __device__ __forceinline__ float run_lod(const LodRun& r, float j) {
 template <int U>
 __device__ __forceinline__ void quad_read_batch(const gcf32x4* __restrict__ quad, const QuadDims& qd, Dims3 d,
                                                 const float3* p, float sc, const bool* use, float* val) {
-  unsigned a0[U], a1[U];
+  unsigned a0[U], a1[U], ix[U], iy[U], iz[U];
   float w[U][3];
   bool in[U];
 #pragma unroll
@@ -395,12 +395,11 @@ __device__ __forceinline__ void quad_read_batch(const gcf32x4* __restrict__ quad
     w[u][0] = px - fx;
     w[u][1] = py - fy;
     w[u][2] = pz - fz;
-    const unsigned ix = (unsigned)clampi((int)fx + 1, 0, (int)qd.qx - 1);
-    const unsigned iy = (unsigned)clampi((int)fy + 1, 0, (int)qd.qy - 1);
-    const unsigned iz = (unsigned)clampi((int)fz + 1, 0, (int)qd.qz - 2);
-    a0[u] = quad_index(qd, ix, iy, iz);
-    a1[u] = quad_index(qd, ix, iy, iz + 1);
+    ix[u] = (unsigned)clampi((int)fx + 1, 0, (int)qd.qx - 1);
+    iy[u] = (unsigned)clampi((int)fy + 1, 0, (int)qd.qy - 1);
+    iz[u] = (unsigned)clampi((int)fz + 1, 0, (int)qd.qz - 2);
   }
+  quad_pairs<float4, U>(qd, ix, iy, iz, a0, a1);
   f32x4 c0[U], c1[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {

@@ -95,7 +95,7 @@ template <int U, int BM = B_BORDER, class Q = float4>
 __device__ __forceinline__ void read_border_batch(const Q* __restrict__ quad, Dims3 d, QuadDims q, float3 n,
                                                   float3 st, int i0, int dir, int last, float val[U],
                                                   bool inside[U]) {
-  unsigned a[U], a1[U];
+  unsigned a[U], a1[U], ix[U], iy[U], iz[U];
   float w[U][3];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -111,11 +111,11 @@ __device__ __forceinline__ void read_border_batch(const Q* __restrict__ quad, Di
     w[u][0] = px - fx;
     w[u][1] = py - fy;
     w[u][2] = pz - fz;
-    const unsigned ix = (unsigned)(clampi((int)fx, -1, d.x - 1) + 1), iy = (unsigned)(clampi((int)fy, -1, d.y - 1) + 1),
-                   iz = (unsigned)(clampi((int)fz, -1, d.z - 1) + 1);
-    a[u] = quad_index<Q>(q, ix, iy, iz);
-    a1[u] = quad_index<Q>(q, ix, iy, iz + 1);
+    ix[u] = (unsigned)(clampi((int)fx, -1, d.x - 1) + 1);
+    iy[u] = (unsigned)(clampi((int)fy, -1, d.y - 1) + 1);
+    iz[u] = (unsigned)(clampi((int)fz, -1, d.z - 1) + 1);
   }
+  quad_pairs<Q, U>(q, ix, iy, iz, a, a1);
   Q r0[U], r1[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -138,7 +138,7 @@ template <int U>
 __device__ __forceinline__ void read_border_batch2(const float4* __restrict__ qa, const float4* __restrict__ qb,
                                                    Dims3 d, QuadDims q, float3 n, float3 st, int i0, int last,
                                                    float va[U], float vb[U], bool inside[U]) {
-  unsigned a[U], a1[U];
+  unsigned a[U], a1[U], ix[U], iy[U], iz[U];
   float w[U][3];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -152,11 +152,11 @@ __device__ __forceinline__ void read_border_batch2(const float4* __restrict__ qa
     w[u][0] = px - fx;
     w[u][1] = py - fy;
     w[u][2] = pz - fz;
-    const unsigned ix = (unsigned)(clampi((int)fx, -1, d.x - 1) + 1), iy = (unsigned)(clampi((int)fy, -1, d.y - 1) + 1),
-                   iz = (unsigned)(clampi((int)fz, -1, d.z - 1) + 1);
-    a[u] = quad_index(q, ix, iy, iz);
-    a1[u] = quad_index(q, ix, iy, iz + 1);
+    ix[u] = (unsigned)(clampi((int)fx, -1, d.x - 1) + 1);
+    iy[u] = (unsigned)(clampi((int)fy, -1, d.y - 1) + 1);
+    iz[u] = (unsigned)(clampi((int)fz, -1, d.z - 1) + 1);
   }
+  quad_pairs<float4, U>(q, ix, iy, iz, a, a1);
   float4 c0[U], c1[U], e0[U], e1[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -763,7 +763,7 @@ __device__ __forceinline__ Brick segment_brick(const float3* cn, const float3* c
 // chain of segments. Tiles of one wave wait for no other and are four times as
 // many as 16x16 ones (in brackets; bricks of 6144 cells). us: 30x34x29, 1 view
 // of 72x85 36 (72); 60x104x59, 3 of 130x220 124 (141); 96x170x96, 5 of 222x395
-// 504 (562); 128x224x128, 5 of 256x456 917 (913). There, bricks of 1536 / 2048 /
+// 480 (562); 128x224x128, 5 of 256x456 917 (913). There, bricks of 1536 / 2048 /
 // 2304 / 2560 / 3072 cells: 3114 / 1064 / 912 / 990 / 1073; segments of 4 / 6:
 // 1020 / 905, but 585 / 518 at 96x170x96. BORDER at 128x224x128: 560 (953).
 // BORDER (the recompute alternative to the saved-state gather: nothing is
