@@ -600,19 +600,20 @@ hipError_t raymarch_bwd_walk_launch(int C, bool exact, int bl, hipStream_t s, co
 }
 
 // Voxel blocks of one wave each, GW to a workgroup (FP64 LDS per wave up to 12
-// KB). C = 4 takes slabs of one z: 128x224x128, 5 views of 256x456, forward and
-// gradient, REFERENCE / EXACT: 16x16x1 1393 / 1228 us, 16x16x2 1394 / 1272,
-// 16x8x2 1423 / 1248, 16x8x1 1454 / 1279, 8x8x2 1501 / 1803 (EXACT with 4 doubles
-// per voxel, 1600 with 5), 8x8x8 1897. A block of 8 deep has lanes that stay 1 to
-// 9 samples in it. Below 4096 blocks there are too few waves and halves of such a
-// slab are better: 48x86x48, 3 views of 100x180: 16x16x1 184 us, 16x8x1 168.
-template <int C, int WX, int WY, int WZ, int GW>
-static hipError_t launch_gather(bool exact, hipStream_t s, const float* gsamp, const int2* ranges, float* grad,
-                                const RayDims& rd, const ProjLaunch& PL) {
+// KB). EXACT C = 4 takes slabs of one z: 128x224x128, 5 views of 256x456, forward
+// and gradient: 16x16x1 1228 us, 16x8x2 1248, 16x16x2 1272, 16x8x1 1279, 8x8x2 1600
+// (1803 with 4 doubles per voxel). A block of 8 deep has lanes that stay 1 to 9
+// samples in it. Below 4096 blocks there are too few waves and halves of such a
+// slab are better (48x86x48, 3 views of 100x180, 184 and 168 us).
+// REFERENCE divides by weight sums, which at a ray's edge are as small as the
+// rounding of positions, and that follows a block's origin: its blocks stay 8x8x2
+// (16x16x1 would take 1393 us, 8x8x2 1501, with single voxels 1e-2 apart).
+template <int C, int WX, int WY, int WZ, int GW, bool EXACT>
+static hipError_t launch_gather(hipStream_t s, const float* gsamp, const int2* ranges, float* grad, const RayDims& rd,
+                                const ProjLaunch& PL) {
   const int nb = ((rd.in.x + WX - 1) / WX) * ((rd.in.y + WY - 1) / WY) * ((rd.in.z + WZ - 1) / WZ);
   const dim3 grid((nb + GW - 1) / GW);
-  if (exact) hipLaunchKernelGGL((k_raymarch_bwd_gather<C, WX, WY, WZ, GW, true>), grid, dim3(64 * GW), 0, s, gsamp, ranges, grad, rd, PL);
-  else hipLaunchKernelGGL((k_raymarch_bwd_gather<C, WX, WY, WZ, GW, false>), grid, dim3(64 * GW), 0, s, gsamp, ranges, grad, rd, PL);
+  hipLaunchKernelGGL((k_raymarch_bwd_gather<C, WX, WY, WZ, GW, EXACT>), grid, dim3(64 * GW), 0, s, gsamp, ranges, grad, rd, PL);
   return hipGetLastError();
 }
 
@@ -620,12 +621,15 @@ hipError_t raymarch_bwd_gather_launch(int C, bool exact, hipStream_t s, const fl
                                       float* grad, const RayDims& rd, const ProjLaunch& PL) {
   KernelTimer t(s, "raymarch_bwd_gather");
   switch (C) {
-    case 1: return launch_gather<1, 16, 16, 2, 4>(exact, s, gsamp, ranges, grad, rd, PL);
-    case 2: return launch_gather<2, 16, 8, 2, 4>(exact, s, gsamp, ranges, grad, rd, PL);
+    case 1: return exact ? launch_gather<1, 16, 16, 2, 4, true>(s, gsamp, ranges, grad, rd, PL)
+                         : launch_gather<1, 16, 16, 2, 4, false>(s, gsamp, ranges, grad, rd, PL);
+    case 2: return exact ? launch_gather<2, 16, 8, 2, 4, true>(s, gsamp, ranges, grad, rd, PL)
+                         : launch_gather<2, 16, 8, 2, 4, false>(s, gsamp, ranges, grad, rd, PL);
     default: {
+      if (!exact) return launch_gather<4, 8, 8, 2, 4, false>(s, gsamp, ranges, grad, rd, PL);
       const size_t slabs = (size_t)((rd.in.x + 15) / 16) * ((rd.in.y + 15) / 16) * rd.in.z;
-      return slabs < 4096 ? launch_gather<4, 16, 8, 1, 1>(exact, s, gsamp, ranges, grad, rd, PL)
-                          : launch_gather<4, 16, 16, 1, 4>(exact, s, gsamp, ranges, grad, rd, PL);
+      return slabs < 4096 ? launch_gather<4, 16, 8, 1, 1, true>(s, gsamp, ranges, grad, rd, PL)
+                          : launch_gather<4, 16, 16, 1, 4, true>(s, gsamp, ranges, grad, rd, PL);
     }
   }
 }
