@@ -1106,18 +1106,12 @@ static void launch_render_gather(hipStream_t s, const RenderSaved& sv, const flo
 //   nb =    64 (32x32x32, 2 views)      428 /  208 /  119 /   96
 // The last has a block for every fourth CU only: 4x4x4-voxel blocks, 512 of
 // them, take 29 us with 8 waves (8x4x4 blocks: 31, 8x8x2: 34).
-// LIT keeps two regions a wave, and from 640 blocks on halves of 16x16x1 leave
-// room for twice the waves (the lit render and its gradients, 16x16x2 / 16x16x1, 4
-// waves: 128x224x128, 5 views 573 / 566 us, 100x178x100, 3 views 320 / 313,
-// 64x112x64, 4 views 111 / 107); alone, the shape is slower without LIT (163 / 222
-// at nb = 7168).
 template <bool LIT>
 static void render_gather(hipStream_t s, const RenderSaved& sv, const float* dens, const float* lam, float* grad,
                           float* lam_grad, const RayDims& rd, const ProjLaunch& PL, float* loss, float loss_scale) {
   const int64_t nb = (int64_t)((rd.in.x + 15) / 16) * ((rd.in.y + 15) / 16) * ((rd.in.z + 1) / 2);
   if (nb < 256) launch_render_gather<4, 4, 4, 8, LIT>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
   else if (nb < 640) launch_render_gather<16, 16, 2, 8, LIT>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
-  else if (LIT) launch_render_gather<16, 16, 1, 4, LIT>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
   else if (nb < 8192) launch_render_gather<16, 16, 2, 4, LIT>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
   else launch_render_gather<16, 16, 2, 2, LIT>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
 }
