@@ -154,37 +154,43 @@ __device__ __forceinline__ void clip_ray(float3 n, float3 st, Dims3 d, int S, fl
   }
 }
 
-// Trilinear value, lerp order x, y, z as in read3DInterpolated. Where every
-// lane's 8 corners lie in the grid (most waves) they are read from one base
-// address without clamping or corner tests; the values are the same.
+// Trilinear value, lerp order x, y, z as in read3DInterpolated. BORDER waves
+// whose lanes all have their 8 corners in the grid (most of those that read
+// anything) take them from one base address without clamping or corner tests;
+// the values are the same. CLAMP and WRAP waves mostly straddle a wall, so they
+// have the general path alone (a CLAMP resample of 64x112x64, C = 4, to two
+// 90x100x110: 30 us, 54 with both).
 template <int C, int BM>
 __device__ __forceinline__ Vec<C> read_linear(const float* __restrict__ buf, Dims3 d, float px, float py, float pz) {
   Vec<C> c[2][2][2];
   float wx, wy, wz;
+  bool one_base = false;
   if constexpr (BM == B_BORDER) {
     const float qx = px + 0.5f, qy = py + 0.5f, qz = pz + 0.5f;
     if (!((0.f <= qx) & (qx < (float)d.x) & (0.f <= qy) & (qy < (float)d.y) & (0.f <= qz) & (qz < (float)d.z)))
       return vzero<C>();
+    const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
+    const int ix = (int)fx, iy = (int)fy, iz = (int)fz;
+    const bool inner = ((unsigned)ix < (unsigned)(d.x - 1)) & ((unsigned)iy < (unsigned)(d.y - 1)) &
+                       ((unsigned)iz < (unsigned)(d.z - 1));
+    one_base = __ballot(!inner) == 0;
+    if (one_base) {
+      wx = px - fx;
+      wy = py - fy;
+      wz = pz - fz;
+      const float* p = buf + flat3(ix, iy, iz, d) * C;
+      const size_t row = (size_t)d.x * C, slice = row * d.y;
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const float* r = p + (k ? slice : 0) + (j ? row : 0);
+          c[k][j][0] = vload<C>(r, 0);
+          c[k][j][1] = vload<C>(r, 1);
+        }
+    }
   }
-  const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
-  const int ix = (int)fx, iy = (int)fy, iz = (int)fz;
-  const bool inner = ((unsigned)ix < (unsigned)(d.x - 1)) & ((unsigned)iy < (unsigned)(d.y - 1)) &
-                     ((unsigned)iz < (unsigned)(d.z - 1));
-  if (__ballot(!inner) == 0) {
-    wx = px - fx;
-    wy = py - fy;
-    wz = pz - fz;
-    const float* p = buf + flat3(ix, iy, iz, d) * C;
-    const size_t row = (size_t)d.x * C, slice = row * d.y;
-#pragma unroll
-    for (int k = 0; k < 2; ++k)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const float* r = p + (k ? slice : 0) + (j ? row : 0);
-        c[k][j][0] = vload<C>(r, 0);
-        c[k][j][1] = vload<C>(r, 1);
-      }
-  } else {
+  if (!one_base) {
     const Taps t = make_taps<BM>(px, py, pz, d);
     wx = t.wx;
     wy = t.wy;
@@ -222,14 +228,15 @@ template <int C> __device__ __forceinline__ bool offsets_fit(Dims3 d) {
 // U trilinear reads with all 8U loads issued before any value is used: the
 // same corners, zeroing and lerp order as read_linear, so every value equals
 // read_linear's, and a BORDER sample outside the grid reads 0. `use` masks
-// samples whose value the caller drops. With `fits` (offsets_fit<C>), where
-// every lane's samples have their 8 corners in the grid or read 0 (most of a
-// ray), they are addressed by one offset each from 4 rows' uniform bases,
+// samples whose value the caller drops. BORDER with `fits` (offsets_fit<C>):
+// where every lane's samples have their 8 corners in the grid or read 0 (most of
+// a ray), they are addressed by one offset each from 4 rows' uniform bases,
 // without clamping or corner tests (a C = 4 sample: 120 instructions, 210 with).
 template <int C, int BM, int U>
 __device__ __forceinline__ void read_linear_batch(const float* __restrict__ buf, Dims3 d, bool fits, const float px[U],
                                                   const float py[U], const float pz[U], const bool use[U],
                                                   Vec<C> out[U]) {
+  constexpr bool kOneBase = BM == B_BORDER || (BM == B_CLAMP && C == 1);
   Vec<C> c[U][2][2][2];
   float wx[U], wy[U], wz[U];
   bool zero[U];
@@ -238,25 +245,27 @@ __device__ __forceinline__ void read_linear_batch(const float* __restrict__ buf,
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     zero[u] = !use[u];
-    if (BM == B_BORDER) {
-      const float qx = px[u] + 0.5f, qy = py[u] + 0.5f, qz = pz[u] + 0.5f;
-      zero[u] |=
-          !((0.f <= qx) & (qx < (float)d.x) & (0.f <= qy) & (qy < (float)d.y) & (0.f <= qz) & (qz < (float)d.z));
-    }
     const float fx = floorf(px[u]), fy = floorf(py[u]), fz = floorf(pz[u]);
     wx[u] = px[u] - fx;
     wy[u] = py[u] - fy;
     wz[u] = pz[u] - fz;
-    const int ix = (int)fx, iy = (int)fy, iz = (int)fz;
-    const bool inner = ((unsigned)ix < (unsigned)(d.x - 1)) & ((unsigned)iy < (unsigned)(d.y - 1)) &
-                       ((unsigned)iz < (unsigned)(d.z - 1));
-    slow |= !(inner | zero[u]);
-    const unsigned f = __umul24(__umul24((unsigned)iz, (unsigned)d.y) + (unsigned)iy, (unsigned)d.x) + (unsigned)ix;
-    at[u] = zero[u] ? 0u : f * (unsigned)(C * sizeof(float));
+    if constexpr (BM == B_BORDER) {
+      const float qx = px[u] + 0.5f, qy = py[u] + 0.5f, qz = pz[u] + 0.5f;
+      zero[u] |=
+          !((0.f <= qx) & (qx < (float)d.x) & (0.f <= qy) & (qy < (float)d.y) & (0.f <= qz) & (qz < (float)d.z));
+    }
+    if constexpr (kOneBase) {
+      const int ix = (int)fx, iy = (int)fy, iz = (int)fz;
+      const bool inner = ((unsigned)ix < (unsigned)(d.x - 1)) & ((unsigned)iy < (unsigned)(d.y - 1)) &
+                         ((unsigned)iz < (unsigned)(d.z - 1));
+      slow |= !(inner | zero[u]);
+      const unsigned f = __umul24(__umul24((unsigned)iz, (unsigned)d.y) + (unsigned)iy, (unsigned)d.x) + (unsigned)ix;
+      at[u] = zero[u] ? 0u : f * (unsigned)(C * sizeof(float));
+    }
   }
   // (a sample that reads 0 loads from the first cells, which an axis of one
   // cell does not have)
-  if (__ballot(slow) == 0 && (d.x > 1) & (d.y > 1) & (d.z > 1)) {
+  if (kOneBase && __ballot(slow) == 0 && (d.x > 1) & (d.y > 1) & (d.z > 1)) {
     const char* base = (const char*)buf;
     const unsigned row = (unsigned)d.x * (unsigned)(C * sizeof(float)), slice = row * (unsigned)d.y;
 #pragma unroll

@@ -22,20 +22,41 @@
 
 namespace gft {
 
-// A ray kernel's workgroup is one wave of 8 x 8 pixels: its 64 samples at one
-// depth lie in a compact patch of the grid, of few cache lines.
-constexpr int kTileX = 8;
-constexpr int kTileY = 8;
-constexpr int kTile = kTileX * kTileY;
+// The forward's and the walk's workgroup is one wave of 8 x 8 pixels, spread by
+// tile_of_block: its 64 samples at one depth lie in a compact patch of the grid,
+// of few cache lines. (CLAMP LINEAR, 128x224x128, 5 views of 256x448, 16 x 16 in
+// rows / 8 x 8 in rows / 8 x 8 spread: C = 1 842 / 533 / 587 us, 4 827 / 765 / 657.)
+constexpr int kSide = 8;
+constexpr int kTile = kSide * kSide;
+// The CLAMP and WRAP scatter is bound by its global atomics and keeps row order,
+// neighbours together. REFERENCE, a launch a view, runs in the same tiles; EXACT,
+// all views at once, in 16 x 16, whose waves meet at fewer cells at a time
+// (48x86x48, 5 views of 96x172, 16 x 16 / 8 x 8 / 8 x 8 spread: REFERENCE C = 1
+// CLAMP 27.8 / 25.7 / 26.2 ms, WRAP 3.55 / 3.53 / 3.77; EXACT CLAMP 20.0 / 20.5 /
+// 22.3, WRAP 1.82 / 1.82 / 2.04).
+template <bool EXACT> constexpr int kScatterSide = EXACT ? 16 : 8;
+
+template <int SIDE, bool SPREAD> __device__ __forceinline__ void tile_pixel(const RayDims& rd, int& x, int& y) {
+  int tx = blockIdx.x, ty = blockIdx.y;
+  if (SPREAD) tile_of_block(blockIdx.x, (rd.out_w + SIDE - 1) / SIDE, tx, ty);
+  x = tx * SIDE + (int)(threadIdx.x % SIDE);
+  y = ty * SIDE + (int)(threadIdx.x / SIDE);
+}
+template <int SIDE, bool SPREAD> static dim3 tile_grid(const RayDims& rd, int views) {
+  const int ntx = (rd.out_w + SIDE - 1) / SIDE, nty = (rd.out_h + SIDE - 1) / SIDE;
+  return SPREAD ? dim3(tile_blocks(ntx, nty), 1, views) : dim3(ntx, nty, views);
+}
+
 // samples read per round trip by the LINEAR ray walks (8 float4 corners per
 // C=4 sample: two samples already hold 64 values in registers)
 template <int C> constexpr int kRayBatch = C == 4 ? 2 : (C == 2 ? 4 : 8);
 
-// LDS asked for to keep 10 waves of a C = 4 walk on a CU (16 fit): a sample
-// reads 8 x 16 bytes, so that more waves evict each other's lines from the 32 KB
-// L1 before the next depth reads them again. 128x224x128, 5 views of 256x456
+// LDS asked for to keep 10 waves of a C = 4 LINEAR BORDER walk on a CU (16 fit): a
+// sample reads 8 x 16 bytes, so that more waves evict each other's lines from the
+// 32 KB L1 before the next depth reads them again. 128x224x128, 5 views of 256x456
 // (16 / 12 / 10 / 8 / 6 waves): forward 368 / - / 283 / 292 / 293 us.
-template <int C> constexpr unsigned kRayLds = C == 4 ? 16000 : 0;
+template <int C, int FM, int BM> constexpr unsigned kRayLds =
+    C == 4 && (BM == B_BORDER ? FM == F_LINEAR : BM == B_WRAP && FM != F_NEAREST) ? 16000 : 0;
 
 template <int C, int FM, int BM>
 __device__ __forceinline__ Vec<C> sample_ray(const float* __restrict__ buf, Dims3 d, float3 p) {
@@ -69,10 +90,8 @@ __global__ __launch_bounds__(kTile) void k_raymarch_fwd(const float* __restrict_
                                                       RayDims rd, RayLaunch L) {
   const int vi = blockIdx.z;
   const RayView& v = L.view[vi];
-  int tx, ty;
-  tile_of_block(blockIdx.x, (rd.out_w + kTileX - 1) / kTileX, tx, ty);
-  const int x = tx * kTileX + (threadIdx.x % kTileX);
-  const int y = ty * kTileY + (threadIdx.x / kTileX);
+  int x, y;
+  tile_pixel<kSide, true>(rd, x, y);
   if (x >= rd.out_w || y >= rd.out_h) return;
   float3 nearp, farp, step;
   ray_endpoints(v, x, y, rd, nearp, farp, step);
@@ -150,16 +169,14 @@ __device__ __forceinline__ void scatter_sample(float* __restrict__ grad, float* 
 }
 
 template <int C, int BM, int BL, bool EXACT>
-__global__ __launch_bounds__(kTile) void k_raymarch_bwd(const float* __restrict__ input,
+__global__ __launch_bounds__(kScatterSide<EXACT> * kScatterSide<EXACT>) void k_raymarch_bwd(const float* __restrict__ input,
                                                       const float* __restrict__ output,
                                                       const float* __restrict__ output_grad, float* __restrict__ grad,
                                                       float* __restrict__ wsum, RayDims rd, RayLaunch L) {
   const int vi = blockIdx.z;
   const RayView& v = L.view[vi];
-  int tx, ty;
-  tile_of_block(blockIdx.x, (rd.out_w + kTileX - 1) / kTileX, tx, ty);
-  const int x = tx * kTileX + (threadIdx.x % kTileX);
-  const int y = ty * kTileY + (threadIdx.x / kTileX);
+  int x, y;
+  tile_pixel<kScatterSide<EXACT>, false>(rd, x, y);
   if (x >= rd.out_w || y >= rd.out_h) return;
   float3 nearp, farp, step;
   ray_endpoints(v, x, y, rd, nearp, farp, step);
@@ -228,10 +245,8 @@ __global__ __launch_bounds__(kTile) void k_raymarch_bwd_walk(const float* __rest
                                                            RayDims rd, RayLaunch L) {
   const int vi = blockIdx.z;
   const RayView& v = L.view[vi];
-  int tx, ty;
-  tile_of_block(blockIdx.x, (rd.out_w + kTileX - 1) / kTileX, tx, ty);
-  const int x = tx * kTileX + (threadIdx.x % kTileX);
-  const int y = ty * kTileY + (threadIdx.x / kTileX);
+  int x, y;
+  tile_pixel<kSide, true>(rd, x, y);
   if (x >= rd.out_w || y >= rd.out_h) return;
   float3 nearp, farp, step;
   ray_endpoints(v, x, y, rd, nearp, farp, step);
@@ -484,80 +499,84 @@ __global__ __launch_bounds__(64 * GW) void k_raymarch_bwd_gather(const float* __
 
 // ------------------------------------------------------------- dispatch
 template <int C, int FM, int BM>
-static hipError_t launch_fwd_bl(int bl, dim3 grid, hipStream_t s, const float* in, float* out, const RayDims& rd,
+static hipError_t launch_fwd_bl(int bl, hipStream_t s, const float* in, float* out, const RayDims& rd,
                                 const RayLaunch& L) {
+  const dim3 grid = tile_grid<kSide, true>(rd, L.num_views), tile(kTile);
+  const unsigned lds = kRayLds<C, FM, BM>;
+  auto run = [&](auto kern) { hipLaunchKernelGGL(kern, grid, tile, lds, s, in, out, rd, L); };
   switch (bl) {
-    case BL_BEER_LAMBERT: hipLaunchKernelGGL((k_raymarch_fwd<C, FM, BM, BL_BEER_LAMBERT>), grid, dim3(kTile), kRayLds<C>, s, in, out, rd, L); break;
-    case BL_ALPHA: hipLaunchKernelGGL((k_raymarch_fwd<C, FM, BM, BL_ALPHA>), grid, dim3(kTile), kRayLds<C>, s, in, out, rd, L); break;
-    case BL_ALPHA_ADDITIVE: hipLaunchKernelGGL((k_raymarch_fwd<C, FM, BM, BL_ALPHA_ADDITIVE>), grid, dim3(kTile), kRayLds<C>, s, in, out, rd, L); break;
-    default: hipLaunchKernelGGL((k_raymarch_fwd<C, FM, BM, BL_ADDITIVE>), grid, dim3(kTile), kRayLds<C>, s, in, out, rd, L); break;
+    case BL_BEER_LAMBERT: run(k_raymarch_fwd<C, FM, BM, BL_BEER_LAMBERT>); break;
+    case BL_ALPHA: run(k_raymarch_fwd<C, FM, BM, BL_ALPHA>); break;
+    case BL_ALPHA_ADDITIVE: run(k_raymarch_fwd<C, FM, BM, BL_ALPHA_ADDITIVE>); break;
+    default: run(k_raymarch_fwd<C, FM, BM, BL_ADDITIVE>); break;
   }
   return hipGetLastError();
 }
 template <int C, int FM>
-static hipError_t launch_fwd_bm(int bm, int bl, dim3 grid, hipStream_t s, const float* in, float* out,
+static hipError_t launch_fwd_bm(int bm, int bl, hipStream_t s, const float* in, float* out,
                                 const RayDims& rd, const RayLaunch& L) {
   switch (bm) {
-    case B_BORDER: return launch_fwd_bl<C, FM, B_BORDER>(bl, grid, s, in, out, rd, L);
-    case B_CLAMP: return launch_fwd_bl<C, FM, B_CLAMP>(bl, grid, s, in, out, rd, L);
-    default: return launch_fwd_bl<C, FM, B_WRAP>(bl, grid, s, in, out, rd, L);
+    case B_BORDER: return launch_fwd_bl<C, FM, B_BORDER>(bl, s, in, out, rd, L);
+    case B_CLAMP: return launch_fwd_bl<C, FM, B_CLAMP>(bl, s, in, out, rd, L);
+    default: return launch_fwd_bl<C, FM, B_WRAP>(bl, s, in, out, rd, L);
   }
 }
 template <int C>
-static hipError_t launch_fwd_fm(int fm, int bm, int bl, dim3 grid, hipStream_t s, const float* in, float* out,
+static hipError_t launch_fwd_fm(int fm, int bm, int bl, hipStream_t s, const float* in, float* out,
                                 const RayDims& rd, const RayLaunch& L) {
   switch (fm) {
-    case F_LINEAR: return launch_fwd_bm<C, F_LINEAR>(bm, bl, grid, s, in, out, rd, L);
-    case F_NEAREST: return launch_fwd_bm<C, F_NEAREST>(bm, bl, grid, s, in, out, rd, L);
-    case F_MIN: return launch_fwd_bm<C, F_MIN>(bm, bl, grid, s, in, out, rd, L);
-    default: return launch_fwd_bm<C, F_MAX>(bm, bl, grid, s, in, out, rd, L);
+    case F_LINEAR: return launch_fwd_bm<C, F_LINEAR>(bm, bl, s, in, out, rd, L);
+    case F_NEAREST: return launch_fwd_bm<C, F_NEAREST>(bm, bl, s, in, out, rd, L);
+    case F_MIN: return launch_fwd_bm<C, F_MIN>(bm, bl, s, in, out, rd, L);
+    default: return launch_fwd_bm<C, F_MAX>(bm, bl, s, in, out, rd, L);
   }
 }
 
 hipError_t raymarch_fwd_launch(int C, int fm, int bm, int bl, hipStream_t s, const float* in, float* out,
                                const RayDims& rd, const RayLaunch& L) {
-  dim3 grid(tile_blocks((rd.out_w + kTileX - 1) / kTileX, (rd.out_h + kTileY - 1) / kTileY), 1, L.num_views);
   switch (C) {
-    case 1: return launch_fwd_fm<1>(fm, bm, bl, grid, s, in, out, rd, L);
-    case 2: return launch_fwd_fm<2>(fm, bm, bl, grid, s, in, out, rd, L);
-    default: return launch_fwd_fm<4>(fm, bm, bl, grid, s, in, out, rd, L);
+    case 1: return launch_fwd_fm<1>(fm, bm, bl, s, in, out, rd, L);
+    case 2: return launch_fwd_fm<2>(fm, bm, bl, s, in, out, rd, L);
+    default: return launch_fwd_fm<4>(fm, bm, bl, s, in, out, rd, L);
   }
 }
 
 template <int C, int BM, bool EX>
-static hipError_t launch_bwd_bl(int bl, dim3 grid, hipStream_t s, const float* in, const float* o, const float* og,
+static hipError_t launch_bwd_bl(int bl, hipStream_t s, const float* in, const float* o, const float* og,
                                 float* g, float* w, const RayDims& rd, const RayLaunch& L) {
+  constexpr int kS = kScatterSide<EX>;
+  const dim3 grid = tile_grid<kS, false>(rd, L.num_views), tile(kS * kS);
+  auto run = [&](auto kern) { hipLaunchKernelGGL(kern, grid, tile, 0, s, in, o, og, g, w, rd, L); };
   switch (bl) {
-    case BL_BEER_LAMBERT: hipLaunchKernelGGL((k_raymarch_bwd<C, BM, BL_BEER_LAMBERT, EX>), grid, dim3(kTile), 0, s, in, o, og, g, w, rd, L); break;
-    case BL_ALPHA: hipLaunchKernelGGL((k_raymarch_bwd<C, BM, BL_ALPHA, EX>), grid, dim3(kTile), 0, s, in, o, og, g, w, rd, L); break;
-    case BL_ALPHA_ADDITIVE: hipLaunchKernelGGL((k_raymarch_bwd<C, BM, BL_ALPHA_ADDITIVE, EX>), grid, dim3(kTile), 0, s, in, o, og, g, w, rd, L); break;
-    default: hipLaunchKernelGGL((k_raymarch_bwd<C, BM, BL_ADDITIVE, EX>), grid, dim3(kTile), 0, s, in, o, og, g, w, rd, L); break;
+    case BL_BEER_LAMBERT: run(k_raymarch_bwd<C, BM, BL_BEER_LAMBERT, EX>); break;
+    case BL_ALPHA: run(k_raymarch_bwd<C, BM, BL_ALPHA, EX>); break;
+    case BL_ALPHA_ADDITIVE: run(k_raymarch_bwd<C, BM, BL_ALPHA_ADDITIVE, EX>); break;
+    default: run(k_raymarch_bwd<C, BM, BL_ADDITIVE, EX>); break;
   }
   return hipGetLastError();
 }
 template <int C, bool EX>
-static hipError_t launch_bwd_bm(int bm, int bl, dim3 grid, hipStream_t s, const float* in, const float* o,
+static hipError_t launch_bwd_bm(int bm, int bl, hipStream_t s, const float* in, const float* o,
                                 const float* og, float* g, float* w, const RayDims& rd, const RayLaunch& L) {
   switch (bm) {
-    case B_BORDER: return launch_bwd_bl<C, B_BORDER, EX>(bl, grid, s, in, o, og, g, w, rd, L);
-    case B_CLAMP: return launch_bwd_bl<C, B_CLAMP, EX>(bl, grid, s, in, o, og, g, w, rd, L);
-    default: return launch_bwd_bl<C, B_WRAP, EX>(bl, grid, s, in, o, og, g, w, rd, L);
+    case B_BORDER: return launch_bwd_bl<C, B_BORDER, EX>(bl, s, in, o, og, g, w, rd, L);
+    case B_CLAMP: return launch_bwd_bl<C, B_CLAMP, EX>(bl, s, in, o, og, g, w, rd, L);
+    default: return launch_bwd_bl<C, B_WRAP, EX>(bl, s, in, o, og, g, w, rd, L);
   }
 }
 template <int C>
-static hipError_t launch_bwd_c(bool exact, int bm, int bl, dim3 grid, hipStream_t s, const float* in, const float* o,
+static hipError_t launch_bwd_c(bool exact, int bm, int bl, hipStream_t s, const float* in, const float* o,
                                const float* og, float* g, float* w, const RayDims& rd, const RayLaunch& L) {
-  return exact ? launch_bwd_bm<C, true>(bm, bl, grid, s, in, o, og, g, w, rd, L)
-               : launch_bwd_bm<C, false>(bm, bl, grid, s, in, o, og, g, w, rd, L);
+  return exact ? launch_bwd_bm<C, true>(bm, bl, s, in, o, og, g, w, rd, L)
+               : launch_bwd_bm<C, false>(bm, bl, s, in, o, og, g, w, rd, L);
 }
 
 hipError_t raymarch_bwd_launch(int C, bool exact, int bm, int bl, hipStream_t s, const float* in, const float* o,
                                const float* og, float* g, float* w, const RayDims& rd, const RayLaunch& L) {
-  dim3 grid(tile_blocks((rd.out_w + kTileX - 1) / kTileX, (rd.out_h + kTileY - 1) / kTileY), 1, L.num_views);
   switch (C) {
-    case 1: return launch_bwd_c<1>(exact, bm, bl, grid, s, in, o, og, g, w, rd, L);
-    case 2: return launch_bwd_c<2>(exact, bm, bl, grid, s, in, o, og, g, w, rd, L);
-    default: return launch_bwd_c<4>(exact, bm, bl, grid, s, in, o, og, g, w, rd, L);
+    case 1: return launch_bwd_c<1>(exact, bm, bl, s, in, o, og, g, w, rd, L);
+    case 2: return launch_bwd_c<2>(exact, bm, bl, s, in, o, og, g, w, rd, L);
+    default: return launch_bwd_c<4>(exact, bm, bl, s, in, o, og, g, w, rd, L);
   }
 }
 
@@ -573,13 +592,16 @@ hipError_t normalize_add_launch(int C, hipStream_t s, float* total, float* buf, 
 
 // BORDER walk for one chunk of views (launch-local view index vi)
 template <int C, bool EX>
-static hipError_t launch_walk_bl(int bl, dim3 grid, hipStream_t s, const float* in, const float* o, const float* og,
+static hipError_t launch_walk_bl(int bl, hipStream_t s, const float* in, const float* o, const float* og,
                                  float* gs, int2* rg, const RayDims& rd, const RayLaunch& L) {
+  const dim3 grid = tile_grid<kSide, true>(rd, L.num_views), tile(kTile);
+  const unsigned lds = kRayLds<C, F_LINEAR, B_BORDER>;
+  auto run = [&](auto kern) { hipLaunchKernelGGL(kern, grid, tile, lds, s, in, o, og, gs, rg, rd, L); };
   switch (bl) {
-    case BL_BEER_LAMBERT: hipLaunchKernelGGL((k_raymarch_bwd_walk<C, BL_BEER_LAMBERT, EX>), grid, dim3(kTile), kRayLds<C>, s, in, o, og, gs, rg, rd, L); break;
-    case BL_ALPHA: hipLaunchKernelGGL((k_raymarch_bwd_walk<C, BL_ALPHA, EX>), grid, dim3(kTile), kRayLds<C>, s, in, o, og, gs, rg, rd, L); break;
-    case BL_ALPHA_ADDITIVE: hipLaunchKernelGGL((k_raymarch_bwd_walk<C, BL_ALPHA_ADDITIVE, EX>), grid, dim3(kTile), kRayLds<C>, s, in, o, og, gs, rg, rd, L); break;
-    default: hipLaunchKernelGGL((k_raymarch_bwd_walk<C, BL_ADDITIVE, EX>), grid, dim3(kTile), kRayLds<C>, s, in, o, og, gs, rg, rd, L); break;
+    case BL_BEER_LAMBERT: run(k_raymarch_bwd_walk<C, BL_BEER_LAMBERT, EX>); break;
+    case BL_ALPHA: run(k_raymarch_bwd_walk<C, BL_ALPHA, EX>); break;
+    case BL_ALPHA_ADDITIVE: run(k_raymarch_bwd_walk<C, BL_ALPHA_ADDITIVE, EX>); break;
+    default: run(k_raymarch_bwd_walk<C, BL_ADDITIVE, EX>); break;
   }
   return hipGetLastError();
 }
@@ -587,15 +609,14 @@ static hipError_t launch_walk_bl(int bl, dim3 grid, hipStream_t s, const float* 
 hipError_t raymarch_bwd_walk_launch(int C, bool exact, int bl, hipStream_t s, const float* in, const float* o,
                                     const float* og, float* gsamp, int2* ranges, const RayDims& rd,
                                     const RayLaunch& L) {
-  dim3 grid(tile_blocks((rd.out_w + kTileX - 1) / kTileX, (rd.out_h + kTileY - 1) / kTileY), 1, L.num_views);
   KernelTimer t(s, "raymarch_bwd_walk");
   switch (C) {
-    case 1: return exact ? launch_walk_bl<1, true>(bl, grid, s, in, o, og, gsamp, ranges, rd, L)
-                         : launch_walk_bl<1, false>(bl, grid, s, in, o, og, gsamp, ranges, rd, L);
-    case 2: return exact ? launch_walk_bl<2, true>(bl, grid, s, in, o, og, gsamp, ranges, rd, L)
-                         : launch_walk_bl<2, false>(bl, grid, s, in, o, og, gsamp, ranges, rd, L);
-    default: return exact ? launch_walk_bl<4, true>(bl, grid, s, in, o, og, gsamp, ranges, rd, L)
-                          : launch_walk_bl<4, false>(bl, grid, s, in, o, og, gsamp, ranges, rd, L);
+    case 1: return exact ? launch_walk_bl<1, true>(bl, s, in, o, og, gsamp, ranges, rd, L)
+                         : launch_walk_bl<1, false>(bl, s, in, o, og, gsamp, ranges, rd, L);
+    case 2: return exact ? launch_walk_bl<2, true>(bl, s, in, o, og, gsamp, ranges, rd, L)
+                         : launch_walk_bl<2, false>(bl, s, in, o, og, gsamp, ranges, rd, L);
+    default: return exact ? launch_walk_bl<4, true>(bl, s, in, o, og, gsamp, ranges, rd, L)
+                          : launch_walk_bl<4, false>(bl, s, in, o, og, gsamp, ranges, rd, L);
   }
 }
 
