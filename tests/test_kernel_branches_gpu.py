@@ -49,3 +49,16 @@ def test_raymarch_scatter_tiles(cuda, image, channels, boundary, grad_mode):
 @pytest.mark.parametrize("filt", ["MIN", "MAX"])
 def test_raymarch_min_max_channels(cuda, boundary, filt):
     _raymarch((9, 17, 12), (17, 8), 4, boundary, None, filt=filt)
+
+
+# 2^24 rows of cells: offsets no longer fit the batched reads' 24-bit products
+@pytest.mark.parametrize("boundary,grad_mode", [("BORDER", "EXACT"), ("CLAMP", None)])
+def test_raymarch_many_rows(cuda, boundary, grad_mode):
+    _raymarch((4096, 4097, 2), (3, 2), 1, boundary, grad_mode, views=1)
+
+
+# slabs of 16 x 16 x 1 voxels (4096 of them or more), ragged in x and y, the last workgroup part empty
+def test_raymarch_gather_slabs(cuda):
+    grid = (457, 41, 37)
+    assert grid[0] * 3 * 3 >= 4096 and grid[0] * 3 * 3 % 4
+    _raymarch(grid, (13, 9), 4, "BORDER", "EXACT")
