@@ -154,12 +154,13 @@ __device__ __forceinline__ void clip_ray(float3 n, float3 st, Dims3 d, int S, fl
   }
 }
 
-// Trilinear value, lerp order x, y, z as in read3DInterpolated. BORDER waves
-// whose lanes all have their 8 corners in the grid (most of those that read
-// anything) take them from one base address without clamping or corner tests;
-// the values are the same. CLAMP and WRAP waves mostly straddle a wall, so they
-// have the general path alone (a CLAMP resample of 64x112x64, C = 4, to two
-// 90x100x110: 30 us, 54 with both).
+// Trilinear value, lerp order x, y, z as in read3DInterpolated. Waves whose
+// lanes all have their 8 corners in the grid take them from one base address
+// without clamping or corner tests; the values are the same. Most WRAP waves
+// straddle a wall, and a C = 4 CLAMP wave gains no more than the test costs: those
+// have the general path alone (a WRAP render forward of 128x224x128 to one view
+// of 166x291 takes 134 us, 149 with both; a CLAMP resample of 64x112x64, C = 4, to
+// 2 of 90x100x110 27, 29).
 template <int C, int BM>
 __device__ __forceinline__ Vec<C> read_linear(const float* __restrict__ buf, Dims3 d, float px, float py, float pz) {
   Vec<C> c[2][2][2];
@@ -169,6 +170,8 @@ __device__ __forceinline__ Vec<C> read_linear(const float* __restrict__ buf, Dim
     const float qx = px + 0.5f, qy = py + 0.5f, qz = pz + 0.5f;
     if (!((0.f <= qx) & (qx < (float)d.x) & (0.f <= qy) & (qy < (float)d.y) & (0.f <= qz) & (qz < (float)d.z)))
       return vzero<C>();
+  }
+  if constexpr (BM == B_BORDER || (BM == B_CLAMP && C < 4)) {
     const float fx = floorf(px), fy = floorf(py), fz = floorf(pz);
     const int ix = (int)fx, iy = (int)fy, iz = (int)fz;
     const bool inner = ((unsigned)ix < (unsigned)(d.x - 1)) & ((unsigned)iy < (unsigned)(d.y - 1)) &

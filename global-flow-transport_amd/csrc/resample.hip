@@ -8,6 +8,7 @@
 // Sampler semantics follow the v1 sampler of the reference
 // (phitest/render/cuda/src/sampling.hpp:158-252,356-491,539-764).
 #include <algorithm>
+#include <type_traits>
 
 #include "gft_device.hpp"
 #include "sampler_v1.hpp"
@@ -82,11 +83,14 @@ __device__ __forceinline__ Vec<C> fetch_v1(const float* __restrict__ buf, Dims3 
   return read_minmax_v1<C, BM>(buf, d, px, py, pz, fm == F_MAX, nullptr);
 }
 
-// The levels are walked with one index for the whole wave (lanes of a wave
-// rarely need more than two), so that a level's dims and address are scalars.
-template <int C, int BM>
+// MIPS: the levels are walked with one index for the whole wave (lanes of a
+// wave rarely need more than two), so that a level's dims and address are scalars.
+template <int C, int BM, bool MIPS>
 __device__ __forceinline__ Vec<C> sample_v1(const float* base, const float* atlas, const MipTable& mt, int b,
                                             const SampleCfg& s, float3 p, float lod) {
+  if constexpr (!MIPS)
+    return fetch_v1<C, BM>(level_ptr(base, atlas, mt, b, 0), mt.dims[0], s.fm, p.x - s.offset, p.y - s.offset,
+                           p.z - s.offset);
   int lv[2];
   float w[2];
   const int n = level_taps(s, lod, lv, w);
@@ -108,10 +112,9 @@ __device__ __forceinline__ Vec<C> sample_v1(const float* base, const float* atla
 // outside the box [0, dims) reads 0 at every mip level (a level's box is no
 // larger), so its level of detail and taps are left out. The samplers decide
 // on a rounded position; the slack covers that.
-template <int BM> __device__ __forceinline__ bool may_read(int fm, float3 p, Dims3 d) {
-  return BM != B_BORDER || fm != F_LINEAR ||
-         ((-1e-2f <= p.x) & (p.x < (float)d.x) & (-1e-2f <= p.y) & (p.y < (float)d.y) & (-1e-2f <= p.z) &
-          (p.z < (float)d.z));
+__device__ __forceinline__ bool may_read(float3 p, Dims3 d) {
+  return (-1e-2f <= p.x) & (p.x < (float)d.x) & (-1e-2f <= p.y) & (p.y < (float)d.y) & (-1e-2f <= p.z) &
+         (p.z < (float)d.z);
 }
 
 // ---------------------------------------------------------------- mips
@@ -238,71 +241,83 @@ __global__ __launch_bounds__(256) void k_mip_collapse(const float* __restrict__ 
 }
 
 // ------------------------------------------------------ transform forward
-// kSample3D (resample_grid.cu.cc:240-252). blockIdx.z = view of the launch. A
-// wave takes 8 x 8 cells in x and z, the block's four waves consecutive y, and
-// a thread `runs` of its cells at every fourth y.
-// Neighbours in the output's xz-plane are neighbours in the input's for cameras
-// that orbit around y, so an 8 x 8 wave reads a compact patch; 64 cells of a row
-// per wave touch a cache line each. The view-summed gather (C = 4, 3 views,
-// LINEAR mips, 100x178x100) takes 123 us, 224-265 with rows, and C = 1 of a
-// 256x128x128 light volume 60, before 71. VALU work bounds it: the folded forms
-// and leaving out what lies outside the grid took the forward from 825 us (IEEE
-// divides, four maps per level of detail) to 335. Its tiles are spread by
-// tile_of_block (those inside the grid take longest): with the mips 382 us, now
-// 340, and a blend that reads its output next 231, now 198.
+// kSample3D (resample_grid.cu.cc:240-252), the view of the launch in the grid's
+// last axis. Two layouts of the output's cells:
+// - rows (TILED false): 256 consecutive cells a workgroup, whole rows stored.
+// - tiles: a wave takes 8 x 8 cells in x and z, the block's four waves
+//   consecutive y, and a thread `runs` of its cells at every fourth y. Neighbours
+//   in the output's xz-plane are neighbours in the input's for cameras that orbit
+//   around y, so an 8 x 8 wave reads a compact patch; 64 cells of a row touch a
+//   cache line each. Its tiles are spread by tile_of_block (those inside the grid
+//   take longest), and a blend that reads its output next takes 198 us, 231 in
+//   row order. Its stores are 8 cells wide.
+// VALU work bounds both: the folded forms and leaving out what lies outside the
+// grid took the forward of 100x178x100 to 3 frusta of 142x270x480 (C = 4, LINEAR
+// mips) from 799 us (IEEE divides, four maps per level of detail) to 333.
 // SUM: one thread loops over the launch's views and writes (or adds) the sum
 // into slot 0, the view-summed gather of the production sampling gradient.
 constexpr int kSampleX = 8, kSampleY = 4, kSampleZ = 8;
-template <int C, int BM, bool SUM, bool LOD>
+// one cell's sample in a view
+template <int C, int BM, bool LOD>
+__device__ __forceinline__ Vec<C> sample_view(const float* __restrict__ in, const float* __restrict__ atlas,
+                                              const MipTable& mt, const SampleCfg& s, const SampleView& v, int cm,
+                                              float qx, float qy, float qz) {
+  if (BM == B_BORDER && s.fm == F_LINEAR && !may_read(map_pos(v, cm, qx, qy, qz), mt.dims[0])) return vzero<C>();
+  float l;
+  const float3 p = map_sample<LOD>(v, cm, qx, qy, qz, l);
+  return sample_v1<C, BM, LOD>(in, atlas, mt, v.in_batch, s, p, l);
+}
+
+template <int C, int BM, bool SUM, bool LOD, bool TILED>
 __global__ __launch_bounds__(256) void k_sample_transform(const float* __restrict__ in,
                                                           const float* __restrict__ atlas, MipTable mt, SampleCfg s,
                                                           Dims3 dout, SampleLaunch L, int runs,
                                                           float* __restrict__ out) {
-  const int ntx = (dout.x + kSampleX - 1) / kSampleX;
-  int tx, ty;
-  if (SUM) {
-    ty = (int)(blockIdx.x / (unsigned)ntx);
-    tx = (int)(blockIdx.x - (unsigned)(ty * ntx));
-  } else {
-    tile_of_block(blockIdx.x, ntx, tx, ty);
-  }
-  const int x = tx * kSampleX + (int)(threadIdx.x % kSampleX);
-  const int y0 = ty * kSampleY * runs + (int)(threadIdx.x / (kSampleX * kSampleZ));
   const size_t n = (size_t)dout.x * dout.y * dout.z;
-  // (one z tile per block, but for grids deeper than the launch limit)
-  for (int z = (int)(blockIdx.y * kSampleZ + threadIdx.x / kSampleX % kSampleZ); z < dout.z;
-       z += (int)(gridDim.y * kSampleZ)) {
-    for (int k = 0; k < runs; ++k) {
-      const int y = y0 + k * kSampleY;
-      if ((x >= dout.x) | (y >= dout.y)) break;
-      const size_t f = flat3(x, y, z, dout);
-      float l;
-      if constexpr (SUM) {
-        Vec<C> acc = vzero<C>();
-        for (int vi = 0; vi < L.num_views; ++vi) {
-          const SampleView& v = L.view[vi];
-          const float3 p0 = map_pos(v, L.cm, x + 0.5f, y + 0.5f, z + 0.5f);
-          if (!may_read<BM>(s.fm, p0, mt.dims[0])) continue;
-          const float3 p = map_sample<LOD>(v, L.cm, x + 0.5f, y + 0.5f, z + 0.5f, l);
-          const Vec<C> r = sample_v1<C, BM>(in, atlas, mt, v.in_batch, s, p, l);
+  auto cell = [&](size_t f, int x, int y, int z, int view) {
+    if constexpr (SUM) {
+      Vec<C> acc = vzero<C>();
+      for (int vi = 0; vi < L.num_views; ++vi) {
+        const Vec<C> r = sample_view<C, BM, LOD>(in, atlas, mt, s, L.view[vi], L.cm, x + 0.5f, y + 0.5f, z + 0.5f);
 #pragma unroll
-          for (int ch = 0; ch < C; ++ch) acc.v[ch] += r.v[ch];
-        }
-        if (L.accumulate) {
-          const Vec<C> o = vload<C>(out, f);
+        for (int ch = 0; ch < C; ++ch) acc.v[ch] += r.v[ch];
+      }
+      if (L.accumulate) {
+        const Vec<C> o = vload<C>(out, f);
 #pragma unroll
-          for (int ch = 0; ch < C; ++ch) acc.v[ch] += o.v[ch];
-        }
-        vstore<C>(out, f, acc);
-      } else {
-        const SampleView& v = L.view[blockIdx.z];
-        Vec<C> r = vzero<C>();
-        const float3 p0 = map_pos(v, L.cm, x + 0.5f, y + 0.5f, z + 0.5f);
-        if (may_read<BM>(s.fm, p0, mt.dims[0])) {
-          const float3 p = map_sample<LOD>(v, L.cm, x + 0.5f, y + 0.5f, z + 0.5f, l);
-          r = sample_v1<C, BM>(in, atlas, mt, v.in_batch, s, p, l);
-        }
-        vstore<C>(out + (size_t)v.out_slot * n * C, f, r);
+        for (int ch = 0; ch < C; ++ch) acc.v[ch] += o.v[ch];
+      }
+      vstore<C>(out, f, acc);
+    } else {
+      const SampleView& v = L.view[view];
+      vstore<C>(out + (size_t)v.out_slot * n * C, f,
+                sample_view<C, BM, LOD>(in, atlas, mt, s, v, L.cm, x + 0.5f, y + 0.5f, z + 0.5f));
+    }
+  };
+  if constexpr (!TILED) {
+    const size_t f = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (f >= n) return;
+    int x, y, z;
+    unflat(f, dout, x, y, z);
+    cell(f, x, y, z, blockIdx.y);
+  } else {
+    const int ntx = (dout.x + kSampleX - 1) / kSampleX;
+    int tx, ty;
+    if (SUM) {
+      ty = (int)(blockIdx.x / (unsigned)ntx);
+      tx = (int)(blockIdx.x - (unsigned)(ty * ntx));
+    } else {
+      tile_of_block(blockIdx.x, ntx, tx, ty);
+    }
+    const int x = tx * kSampleX + (int)(threadIdx.x % kSampleX);
+    const int y0 = ty * kSampleY * runs + (int)(threadIdx.x / (kSampleX * kSampleZ));
+    // (one z tile per block, but for grids deeper than the launch limit)
+    for (int z = (int)(blockIdx.y * kSampleZ + threadIdx.x / kSampleX % kSampleZ); z < dout.z;
+         z += (int)(gridDim.y * kSampleZ)) {
+      for (int k = 0; k < runs; ++k) {
+        const int y = y0 + k * kSampleY;
+        if ((x >= dout.x) | (y >= dout.y)) break;
+        cell(flat3(x, y, z, dout), x, y, z, blockIdx.z);
       }
     }
   }
@@ -665,7 +680,7 @@ __global__ __launch_bounds__(256) void k_sample_lut(const float* __restrict__ in
   unflat(f, dout, x, y, z);
   float lod;
   float3 p = lut_pos(lut, L, cam, f, x, y, z, lod);
-  Vec<C> r = sample_v1<C, BM>(in, atlas, mt, b, s, p, lod);
+  const Vec<C> r = sample_v1<C, BM, true>(in, atlas, mt, b, s, p, lod);
   vstore<C>(out + (size_t)slot * n * C, f, r);
 }
 
@@ -1111,7 +1126,8 @@ __global__ __launch_bounds__(kShadowWaves * 64) void k_shadow_fwd(const float* _
       float val = 0.f;
       if (live && z < dout.z) {
         float l;
-        if (may_read<BM>(FM, map_pos(v, CM_LINDEPTH, x + 0.5f, y + 0.5f, z + 0.5f), mt.dims[0])) {
+        if (BM != B_BORDER || FM != F_LINEAR ||
+            may_read(map_pos(v, CM_LINDEPTH, x + 0.5f, y + 0.5f, z + 0.5f), mt.dims[0])) {
           const float3 q = map_sample<LOD>(v, CM_LINDEPTH, x + 0.5f, y + 0.5f, z + 0.5f, l);
           val = sample_scaled<BM, FM>(dens, atlas, mt, cfg, q, l, step);
         }
@@ -1261,24 +1277,56 @@ hipError_t mip_collapse_launch(int C, hipStream_t st, const float* gp, size_t gp
   return hipGetLastError();
 }
 
+// Rows or tiles. us, rows / tiles:
+// - view sums read several frusta, or many bytes a sample: C = 4 LINEAR mips, 3
+//   views of 142x270x480 -> 100x178x100 425 / 335; C = 1, 3 of 142x270x240 ->
+//   64x112x64 20 / 12; but one scalar view of 256x196x196 -> 128x224x128 70 / 78.
+// - forward, LINEAR: tiles where the grid is beyond an XCD's 4 MB of L2 and the
+//   output does not far outnumber it (C = 1 128x224x128 -> 2 views of 90x200x120 40 / 26,
+//   of 142x270x480 138 / 167; C = 4 78 / 46, 226 / 239, but 3 views of 100x178x100
+//   with mips 350 / 333; C = 4 24x40x24 -> 90x200x120 28 / 30, 64x112x64 35 / 30).
+//   Two of CLAMP, a reverse map and mips: rows (C = 4 128x224x128 -> 2 of 90x200x120
+//   CLAMP mips 94 / 102, reverse mips 76 / 85, 64x112x64 reverse CLAMP 44 / 50).
+// - NEAREST: rows (C = 1 64x112x64 -> 90x200x120 17 / 24).
+// - a thin output leaves lanes idle, a small one CUs (C = 4 128x224x128 -> 2 of
+//   1x1024x1024 16 / 78, of 32x32x32 5 / 10).
+static bool sample_in_tiles(int C, int bm, bool sum, const SampleCfg& s, Dims3 din, Dims3 dout,
+                            const SampleLaunch& L) {
+  if (std::min({dout.x, dout.y, dout.z}) < 24 || std::min({din.x, din.y, din.z}) < 8) return false;
+  if (sum) return C > 1 || L.num_views > 1;
+  const size_t vox = (size_t)din.x * din.y * din.z, cells = (size_t)dout.x * dout.y * dout.z;
+  const bool reverse = L.cm != CM_TRANSFORM && L.cm != CM_LINDEPTH;
+  if (s.fm != F_LINEAR || (s.mm != MIP_NONE) + (bm == B_CLAMP) + reverse > 1) return false;
+  return vox * C * sizeof(float) > (size_t(4) << 20) && cells >= (1u << 18) && (C == 4 || cells <= 3 * C * vox);
+}
+
 hipError_t sample_transform_launch(int C, int bm, bool sum, hipStream_t st, const float* in, const float* atlas,
                                    const MipTable& mt, const SampleCfg& s, Dims3 dout, const SampleLaunch& L,
                                    float* out) {
+  const bool tiled = sample_in_tiles(C, bm, sum, s, mt.dims[0], dout, L);
   // y runs per thread (100x178x100 grid, 3 views of 480x270 in 142 slices, C = 4,
   // LINEAR mips; 1 / 2 / 4 / 8): the frusta 363 / 314 / 315 / 359 us (more cells
   // share a block's set-up), the view-summed grid 105 / 110 / 119 / 124
   const int runs = sum ? 1 : 2;
-  const int ntx = (dout.x + kSampleX - 1) / kSampleX, nty = (dout.y + kSampleY * runs - 1) / (kSampleY * runs),
-            ntz = (dout.z + kSampleZ - 1) / kSampleZ;
-  const dim3 grid(sum ? (unsigned)ntx * (unsigned)nty : tile_blocks(ntx, nty), (unsigned)std::min(ntz, 65535),
-                  sum ? 1 : L.num_views);
-  const bool lod = s.mm != MIP_NONE;
+  dim3 grid = grid_for((size_t)dout.x * dout.y * dout.z, sum ? 1 : L.num_views);
+  if (tiled) {
+    const int ntx = (dout.x + kSampleX - 1) / kSampleX, nty = (dout.y + kSampleY * runs - 1) / (kSampleY * runs),
+              ntz = (dout.z + kSampleZ - 1) / kSampleZ;
+    grid = dim3(sum ? (unsigned)ntx * (unsigned)nty : tile_blocks(ntx, nty), (unsigned)std::min(ntz, 65535),
+                sum ? 1 : L.num_views);
+  }
+  auto run = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, in, atlas, mt, s, dout, L, runs, out); };
   GFT_DISPATCH_C(C, GFT_DISPATCH_BM(bm, {
-    auto run = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, in, atlas, mt, s, dout, L, runs, out); };
-    if (sum && lod) run(k_sample_transform<CC, BB, true, true>);
-    else if (sum) run(k_sample_transform<CC, BB, true, false>);
-    else if (lod) run(k_sample_transform<CC, BB, false, true>);
-    else run(k_sample_transform<CC, BB, false, false>);
+    auto pick = [&](auto t) {
+      constexpr bool T = decltype(t)::value;
+      const bool lod = s.mm != MIP_NONE;
+      if (sum && lod) run(k_sample_transform<CC, BB, true, true, T>);
+      else if (sum) run(k_sample_transform<CC, BB, true, false, T>);
+      else if (lod) run(k_sample_transform<CC, BB, false, true, T>);
+      else run(k_sample_transform<CC, BB, false, false, T>);
+    };
+    if (tiled) pick(std::true_type{});
+    else pick(std::false_type{});
   }));
   return hipGetLastError();
 }

@@ -62,3 +62,50 @@ def test_raymarch_gather_slabs(cuda):
     grid = (457, 41, 37)
     assert grid[0] * 3 * 3 >= 4096 and grid[0] * 3 * 3 % 4
     _raymarch(grid, (13, 9), 4, "BORDER", "EXACT")
+
+
+def _smooth(shape, channels):
+    """Smooth positive cells that vanish at the faces, so that a sample a rounding
+    away from a face or a cell changes by far less than the tolerance."""
+    axes = [np.sin(np.pi * (np.arange(n) + 0.5) / n) ** 2 for n in shape]
+    d = axes[0][:, None, None] * axes[1][:, None] * axes[2]
+    return (d[None, ..., None] * (1.0 + 0.25 * np.arange(channels))).astype(np.float32)
+
+
+# resample layouts: rows, and tiles of 8 x 8 x 8 cells from a 4 MB grid, 2^18
+# output cells and 24 cells an axis on, where not two of CLAMP, a reverse map and
+# mips meet; ragged in every axis. Values 1e-5 (the field's slope is below 0.13 a
+# cell, positions of 100 cells err by 1e-5).
+RESAMPLES = [(c, g, o, cm, bm, m) for c, g, o in (
+    (4, (64, 65, 67), (66, 61, 67)), (4, (64, 65, 67), (63, 61, 63)), (4, (64, 65, 67), (23, 120, 99)),
+    (4, (62, 63, 61), (66, 61, 67)), (1, (104, 101, 101), (25, 101, 109)), (1, (104, 101, 101), (152, 148, 151)),
+    (2, (81, 80, 82), (24, 91, 131))) for cm, bm, m in (
+    ("TRANSFORM_LINDEPTH", "BORDER", 0), ("TRANSFORM", "CLAMP", 0), ("TRANSFORM_LINDEPTH", "BORDER", 3),
+    ("TRANSFORM_REVERSE", "CLAMP", 0), ("TRANSFORM_LINDEPTH_REVERSE", "BORDER", 0))]
+
+
+@pytest.mark.parametrize("channels,grid,out,coord,boundary,mips", RESAMPLES)
+def test_resample_layouts(cuda, channels, grid, out, coord, boundary, mips):
+    from gft.ops import sampling_ops as ops
+    sc = scene(grid=(40, 44, 42) if coord.endswith("REVERSE") else grid, image=out[1:], views=2, seed=3)
+    data = _smooth(grid, channels)
+    cam = (sc["M"], sc["V"], sc["P"], sc["F"])
+    kw = dict(interpolation="LINEAR", boundary=boundary, mipmapping="LINEAR" if mips else "NONE", num_mipmaps=mips,
+              coordinate_mode=coord)
+    got = ops.sample_grid_transform(_t(data), *cam, out, **kw).cpu().numpy()
+    assert norm_err(got, orc.sample_transform_fwd(data, *cam, out, prec=1, **kw)) < 1e-5
+
+
+# view sums: tiles for several channels or views, rows for one scalar view or a thin grid
+@pytest.mark.parametrize("channels,views,grid", [(1, 1, (26, 25, 27)), (1, 2, (26, 25, 27)), (4, 1, (26, 25, 27)),
+                                                 (4, 2, (23, 25, 27)), (2, 10, (24, 33, 24))])
+@pytest.mark.parametrize("boundary,mips", [("BORDER", 0), ("CLAMP", 0), ("BORDER", 2)])
+def test_view_sum_layouts(cuda, channels, views, grid, boundary, mips):
+    from gft.ops import sampling_ops as ops
+    sc = scene(grid=grid, image=(19, 22), views=views, seed=3)
+    og = np.stack([_smooth((17, 19, 22), channels)[0] * (1.0 + v) for v in range(views)])[None]
+    cam = (sc["M"], sc["V"], sc["P"], sc["F"])
+    kw = dict(interpolation="LINEAR", boundary=boundary, mipmapping="LINEAR" if mips else "NONE", num_mipmaps=mips,
+              coordinate_mode="TRANSFORM_LINDEPTH")
+    got = ops.sample_grid_transform_gather_grad(_t(og), *cam, grid, **kw).cpu().numpy()
+    assert norm_err(got, orc.sample_transform_gather_grad(og, *cam, grid, **kw)) < 1e-5
