@@ -108,6 +108,27 @@ __device__ __forceinline__ Vec<C> sample_v1(const float* base, const float* atla
   return a;
 }
 
+// The same where a table gives each cell its level: a lane goes to its own
+// levels, however many a wave has.
+template <int C, int BM>
+__device__ __forceinline__ Vec<C> sample_lanes(const float* base, const float* atlas, const MipTable& mt, int b,
+                                               const SampleCfg& s, float3 p, float lod) {
+  int lv[2];
+  float w[2];
+  const int n = level_taps(s, lod, lv, w);
+  const float sc = level_scale(lv[0]);
+  Vec<C> a = fetch_v1<C, BM>(level_ptr(base, atlas, mt, b, lv[0]), mt.dims[lv[0]], s.fm, p.x * sc - s.offset,
+                             p.y * sc - s.offset, p.z * sc - s.offset);
+  if (n == 2) {
+    const float sc1 = level_scale(lv[1]);
+    const Vec<C> c = fetch_v1<C, BM>(level_ptr(base, atlas, mt, b, lv[1]), mt.dims[lv[1]], s.fm, p.x * sc1 - s.offset,
+                                     p.y * sc1 - s.offset, p.z * sc1 - s.offset);
+#pragma unroll
+    for (int ch = 0; ch < C; ++ch) a.v[ch] = lerpf(a.v[ch], c.v[ch], w[1]);
+  }
+  return a;
+}
+
 // Most cells of a camera frustum lie outside the grid: a BORDER LINEAR sample
 // outside the box [0, dims) reads 0 at every mip level (a level's box is no
 // larger), so its level of detail and taps are left out. The samplers decide
@@ -680,7 +701,10 @@ __global__ __launch_bounds__(256) void k_sample_lut(const float* __restrict__ in
   unflat(f, dout, x, y, z);
   float lod;
   float3 p = lut_pos(lut, L, cam, f, x, y, z, lod);
-  const Vec<C> r = sample_v1<C, BM, true>(in, atlas, mt, b, s, p, lod);
+  // (128x224x128, random levels, lanes / wave: C = 4 NEAREST mips 60 / 82 us, LINEAR
+  // 80 / 88; C = 1 LINEAR 58 / 49)
+  const Vec<C> r = C == 1 && s.mm == MIP_LINEAR ? sample_v1<C, BM, true>(in, atlas, mt, b, s, p, lod)
+                                                : sample_lanes<C, BM>(in, atlas, mt, b, s, p, lod);
   vstore<C>(out + (size_t)slot * n * C, f, r);
 }
 

@@ -109,3 +109,20 @@ def test_view_sum_layouts(cuda, channels, views, grid, boundary, mips):
               coordinate_mode="TRANSFORM_LINDEPTH")
     got = ops.sample_grid_transform_gather_grad(_t(og), *cam, grid, **kw).cpu().numpy()
     assert norm_err(got, orc.sample_transform_gather_grad(og, *cam, grid, **kw)) < 1e-5
+
+
+# a table's levels, all in one wave: lane by lane, and level by level (one channel, LINEAR mips)
+@pytest.mark.parametrize("channels", [1, 2, 4])
+@pytest.mark.parametrize("boundary", ["BORDER", "CLAMP", "WRAP"])
+@pytest.mark.parametrize("mip", ["NEAREST", "LINEAR"])
+def test_lut_levels(cuda, channels, boundary, mip):
+    from gft.ops import sampling_ops as ops
+    shape = (24, 26, 28)
+    data = _smooth(shape, channels)
+    rng = np.random.Generator(np.random.PCG64(8))
+    lut = rng.uniform(-3, 3, size=(1, 9, 11, 13, 4)).astype(np.float32)
+    # levels away from the halves, where NEAREST turns
+    lut[..., 3] = rng.integers(-1, 5, size=lut.shape[:-1]) + rng.uniform(-0.4, 0.4, size=lut.shape[:-1])
+    kw = dict(interpolation="LINEAR", boundary=boundary, mipmapping=mip, num_mipmaps=3, cell_center_offset=0.5)
+    got = ops.sample_grid_lut(_t(data), _t(lut), **kw).cpu().numpy()
+    assert norm_err(got, orc.sample_lut_fwd(data, lut, prec=1, **kw)) < 1e-5
