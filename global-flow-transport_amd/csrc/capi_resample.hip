@@ -12,7 +12,7 @@ namespace gft {
 hipError_t fill_launch(hipStream_t s, float* p, size_t n, float v);
 hipError_t mip_down_launch(hipStream_t st, const float* src, size_t src_stride, const MipTable& mt, int first, int n,
                            float* atlas, int batches, float scale);
-int mip_levels_per_launch();
+int mip_levels_of_launch(const MipTable& mt, int first, int batches);
 hipError_t mip_collapse_launch(int C, hipStream_t st, const float* gp, size_t gp_stride, Dims3 o, float* gc,
                                size_t gc_stride, Dims3 s, int batches);
 hipError_t sample_transform_launch(int C, int bm, bool sum, hipStream_t st, const float* in, const float* atlas,
@@ -80,11 +80,11 @@ static size_t atlas_bytes(Dims3 d, int C, int levels, int batches) {
 // grid's values as they are read (the pyramid of base * base_scale).
 static hipError_t build_atlas(hipStream_t st, const float* base, const MipTable& mt, int batches, float* atlas,
                               float base_scale = 1.f) {
-  for (int m = 0; m < mt.levels; m += mip_levels_per_launch()) {
+  for (int m = 0, n; m < mt.levels; m += n) {
     const float* src = m == 0 ? base : atlas + mt.offset[m];
     const size_t src_stride = m == 0 ? mt.base_stride : mt.atlas_stride;
-    hipError_t e = mip_down_launch(st, src, src_stride, mt, m, std::min(mt.levels - m, mip_levels_per_launch()), atlas,
-                                   batches, m == 0 ? base_scale : 1.f);
+    n = mip_levels_of_launch(mt, m, batches);
+    hipError_t e = mip_down_launch(st, src, src_stride, mt, m, n, atlas, batches, m == 0 ? base_scale : 1.f);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

@@ -143,8 +143,9 @@ __device__ __forceinline__ bool may_read(float3 p, Dims3 d) {
 // then x; blockIdx.y = batch. Every source value is multiplied by `scale` first
 // (1 leaves it unchanged): the pyramid of a scaled grid without materialising
 // the scaled grid.
-// A workgroup takes a tile of 32 x 16 x 16 source cells and builds up to
-// kMipLevels levels of it, each from the one before in LDS (a level's cells only
+// k_mip_level: one level, a thread per cell in row order.
+// k_mip_down: a workgroup takes a tile of 32 x 16 x 16 source cells and builds up
+// to kMipLevels levels of it, each from the one before in LDS (a level's cells only
 // read the two cells under them per axis, so tiles are independent): one launch
 // reads the source once instead of a launch and a read per level. A pyramid of
 // a 128x224x128 grid took 4 launches of 4 us and more each, mostly latency.
@@ -172,6 +173,30 @@ __device__ __forceinline__ Vec<C> mip_mean(const Vec<C> v[2][2][2]) {  // [x][y]
     r.v[ch] = (ya[0] + ya[1]) * 0.5f;
   }
   return r;
+}
+
+template <int C>
+__global__ __launch_bounds__(256) void k_mip_level(const float* __restrict__ src, size_t src_stride, Dims3 s,
+                                                   float* __restrict__ dst, size_t dst_stride, Dims3 o, float scale) {
+#pragma clang fp contract(off)
+  const size_t n = (size_t)o.x * o.y * o.z;
+  const size_t f = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (f >= n) return;
+  const float* in = src + (size_t)blockIdx.y * src_stride;
+  int x, y, z;
+  unflat(f, o, x, y, z);
+  Vec<C> v[2][2][2];
+#pragma unroll
+  for (int xi = 0; xi < 2; ++xi)
+#pragma unroll
+    for (int yi = 0; yi < 2; ++yi)
+#pragma unroll
+      for (int zi = 0; zi < 2; ++zi) {
+        v[xi][yi][zi] = vload<C>(in, flat3(2 * x + xi, 2 * y + yi, 2 * z + zi, s));
+#pragma unroll
+        for (int ch = 0; ch < C; ++ch) v[xi][yi][zi].v[ch] *= scale;
+      }
+  vstore<C>(dst + (size_t)blockIdx.y * dst_stride, f, mip_mean<C>(v));
 }
 
 template <int C>
@@ -207,7 +232,7 @@ __global__ __launch_bounds__(256) void k_mip_down(const float* __restrict__ src,
       r = mip_mean<C>(v);
       vstore<C>(atlas + m.offset[1], flat3(x, y, z, m.dims[1]), r);
     }
-    if (m.levels > 1) vstore<C>(lds, c, r);
+    vstore<C>(lds, c, r);
   }
   int wx = kMipX, wy = kMipY, wz = kMipZ;
   float *from = lds, *to = lds + kMipX * kMipY * kMipZ * C;
@@ -1275,23 +1300,43 @@ static inline dim3 grid_for(size_t n, unsigned views) { return dim3((unsigned)((
     default: { constexpr int BB = B_WRAP; __VA_ARGS__; } break;         \
   }
 
-// levels first + 1 .. first + n of the pyramid mt (n <= kMipLevels), from level `first`
+// Levels of the pyramid that the launch from level `first` builds. A single one
+// goes in rows (200x356x200, C = 1, rows / tiles: 11.3 / 18.8 us; 100x178x100, C = 4
+// 5.4 / 8.6), and so does a narrow grid, whose tiles are mostly idle lanes
+// (512x512x4, C = 4, 2 levels 6.8 / 7.6). Where rows of cells end within a 128-byte
+// line, a tile's 32 cells straddle two, which neighbours on other XCDs read again:
+// beyond 48 MB such a level goes in rows, and the tiles take those after it
+// (200x356x200, 3 levels: 16.8 in rows, 20.1 in tiles; 100x178x100, C = 4, of 28 MB,
+// 11.3 with the first level in rows, 9.8 in tiles).
+int mip_levels_of_launch(const MipTable& mt, int first, int batches) {
+  const Dims3 s = mt.dims[first], o = mt.dims[first + 1];
+  const size_t row = (size_t)s.x * mt.C * sizeof(float), bytes = row * s.y * s.z * batches;
+  if ((o.x < 4 && (size_t)o.y * o.z > 1024) || (row % 128 != 0 && bytes > (size_t(48) << 20))) return 1;
+  return std::min(mt.levels - first, kMipLevels);
+}
+
+// levels first + 1 .. first + n of the pyramid mt, from level `first` (n: mip_levels_of_launch)
 hipError_t mip_down_launch(hipStream_t st, const float* src, size_t src_stride, const MipTable& mt, int first, int n,
                            float* atlas, int batches, float scale) {
+  const Dims3 o = mt.dims[first + 1];
+  if (n == 1) {
+    const dim3 grid = grid_for((size_t)o.x * o.y * o.z, batches);
+    GFT_DISPATCH_C(mt.C, hipLaunchKernelGGL(k_mip_level<CC>, grid, dim3(256), 0, st, src, src_stride, mt.dims[first],
+                                            atlas + mt.offset[first + 1], mt.atlas_stride, o, scale));
+    return hipGetLastError();
+  }
   MipChain m{};
   m.levels = n;
   for (int l = 0; l <= n; ++l) {
     m.dims[l] = mt.dims[first + l];
     m.offset[l] = mt.offset[first + l];
   }
-  const Dims3 o = m.dims[1];
   const size_t tiles = (size_t)((o.x + kMipX - 1) / kMipX) * ((o.y + kMipY - 1) / kMipY) * ((o.z + kMipZ - 1) / kMipZ);
   const dim3 grid((unsigned)tiles, batches);
   GFT_DISPATCH_C(mt.C, hipLaunchKernelGGL(k_mip_down<CC>, grid, dim3(256), 0, st, src, src_stride, atlas,
                                           mt.atlas_stride, m, scale));
   return hipGetLastError();
 }
-int mip_levels_per_launch() { return kMipLevels; }
 
 hipError_t mip_collapse_launch(int C, hipStream_t st, const float* gp, size_t gp_stride, Dims3 o, float* gc,
                                size_t gc_stride, Dims3 s, int batches) {

@@ -126,3 +126,20 @@ def test_lut_levels(cuda, channels, boundary, mip):
     kw = dict(interpolation="LINEAR", boundary=boundary, mipmapping=mip, num_mipmaps=3, cell_center_offset=0.5)
     got = ops.sample_grid_lut(_t(data), _t(lut), **kw).cpu().numpy()
     assert norm_err(got, orc.sample_lut_fwd(data, lut, prec=1, **kw)) < 1e-5
+
+
+# pyramid launches of one level (a narrow grid; unaligned rows beyond 48 MB) and of
+# several behind one; 1e-6 as for the other pyramids
+@pytest.mark.parametrize("shape,channels,levels", [((65, 66, 7), 1, 2), ((65, 66, 7), 4, 2), ((131, 310, 313), 1, 4),
+                                                   ((47, 48, 50), 2, 1), ((64, 65, 66), 1, 6)])
+def test_pyramid_launches(cuda, shape, channels, levels):
+    from gft.ops import sampling_ops as ops
+    rng = np.random.Generator(np.random.PCG64(5))
+    data = rng.uniform(0.1, 1.0, size=(1,) + shape + (channels,)).astype(np.float32)
+    got = ops.build_mips(_t(data), levels)
+    ref = data.astype(np.float64)
+    assert len(got) == levels
+    for m in range(levels):
+        d = [n // 2 for n in ref.shape[1:4]]
+        ref = ref[:, :2 * d[0], :2 * d[1], :2 * d[2]].reshape(1, d[0], 2, d[1], 2, d[2], 2, channels).mean((2, 4, 6))
+        assert norm_err(got[m].cpu().numpy(), ref) < 1e-6
