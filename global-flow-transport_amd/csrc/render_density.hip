@@ -41,10 +41,13 @@ constexpr int kRTileY = 16;
 // The forwards' workgroups are one wave of 16 x 4 pixels. BORDER rays are of
 // very different lengths, so their tiles are spread by tile_of_block
 // (128x224x128, 5 views of 256x456: 157 -> 127 us, four waves a workgroup 133;
-// lit 328 -> 241, 259); CLAMP and WRAP rays are all as long, and row order reads
-// a little less (96x170x96: 111 us, 115 spread).
+// lit 328 -> 241, 259); CLAMP rays are all as long, and row order reads a little
+// less (96x170x96: 111 us, 115 spread). WRAP rays read the grid itself, one sample a
+// round trip, and four waves share what their L1 holds (96x170x96, 1 view of 48x85:
+// 70 us, 90 in waves of their own; 128x224x128, 1 of 166x291 116, 134).
 constexpr int kFwdTileY = 4;
 constexpr int kFwdThreads = kRTileX * kFwdTileY;
+template <int BM> constexpr int kFwdRows = BM == B_WRAP ? kRTileY : kFwdTileY;
 
 // ----------------------------------------------------------------- helpers
 __device__ __forceinline__ void pixel_ray(const RayView& v, const RayDims& rd, int x, int y, float3& nearp,
@@ -211,20 +214,24 @@ __device__ __forceinline__ int wave_max(int v) {
 // samples[sample_base(pixel) + i * kSampleRun] (wave-major: one instruction's
 // stores fill two whole lines; a NaN mark for a sample outside the grid).
 template <int BM, class Q = float4>
-__global__ __launch_bounds__(kFwdThreads) void k_render_density_fwd(const float* __restrict__ dens, float* __restrict__ img,
-                                                            RayDims rd, RayLaunch L, RenderParams rp, QuadDims q,
-                                                            RenderSaved sv) {
+__global__ __launch_bounds__(kRTileX* kFwdRows<BM>) void k_render_density_fwd(const float* __restrict__ dens,
+                                                                             float* __restrict__ img, RayDims rd,
+                                                                             RayLaunch L, RenderParams rp, QuadDims q,
+                                                                             RenderSaved sv) {
   const RayView& v = L.view[blockIdx.z];
   int tx, ty;
   const int ntx = (rd.out_w + kRTileX - 1) / kRTileX;
   if (BM == B_BORDER) {
     tile_of_block(blockIdx.x, ntx, tx, ty);
+  } else if (BM == B_WRAP) {
+    tx = (int)blockIdx.x;
+    ty = (int)blockIdx.y;
   } else {
     ty = (int)(blockIdx.x / (unsigned)ntx);
     tx = (int)(blockIdx.x - (unsigned)(ty * ntx));
   }
   const int x = tx * kRTileX + (threadIdx.x % kRTileX);
-  const int y = ty * kFwdTileY + (threadIdx.x / kRTileX);
+  const int y = ty * kFwdRows<BM> + (threadIdx.x / kRTileX);
   const bool valid = x < rd.out_w && y < rd.out_h;
   float D = 0.f, E = 0.f;
   if (BM == B_BORDER || BM == B_CLAMP) {
@@ -995,9 +1002,10 @@ static dim3 tile_grid(const RayDims& rd, int views) {
   return dim3((rd.out_w + kRTileX - 1) / kRTileX, (rd.out_h + kRTileY - 1) / kRTileY, views);
 }
 
-static dim3 fwd_grid(const RayDims& rd, bool spread, int views) {
-  const int ntx = (rd.out_w + kRTileX - 1) / kRTileX, nty = (rd.out_h + kFwdTileY - 1) / kFwdTileY;
-  return dim3(spread ? tile_blocks(ntx, nty) : (unsigned)ntx * (unsigned)nty, 1, views);
+template <int BM> static dim3 fwd_grid(const RayDims& rd, int views) {
+  const int ntx = (rd.out_w + kRTileX - 1) / kRTileX, nty = (rd.out_h + kFwdRows<BM> - 1) / kFwdRows<BM>;
+  if (BM == B_WRAP) return dim3(ntx, nty, views);
+  return dim3(BM == B_BORDER ? tile_blocks(ntx, nty) : (unsigned)ntx * (unsigned)nty, 1, views);
 }
 
 size_t quad_copy_floats(Dims3 d) { return quad_entries(make_quad_dims(d)) * 4; }
@@ -1016,7 +1024,7 @@ hipError_t quad_copy_bf16_launch(hipStream_t s, const float* lin, void* out, Dim
 // BORDER forward from the bfloat16 corner-quad copy
 hipError_t render_density_fwd_bf16_launch(hipStream_t s, const void* quad, float* img, const RayDims& rd,
                                           const RayLaunch& L, const RenderParams& rp, const RenderSaved& sv) {
-  const dim3 grid = fwd_grid(rd, true, L.num_views);
+  const dim3 grid = fwd_grid<B_BORDER>(rd, L.num_views);
   const QuadDims q = make_quad_dims<uint2>(rd.in);
   KernelTimer t(s, "render_fwd");
   hipLaunchKernelGGL((k_render_density_fwd<B_BORDER, uint2>), grid, dim3(kFwdThreads), 0, s,
@@ -1043,7 +1051,7 @@ hipError_t quad_copy_launch(hipStream_t s, int bm, const float* lin, float* out,
 hipError_t render_density_lit_fwd_launch(hipStream_t s, const float* dq, const float* eq, float* img,
                                          const RayDims& rd, const RayLaunch& L, const RenderParams& rp,
                                          const RenderSaved& sv) {
-  const dim3 grid = fwd_grid(rd, true, L.num_views);
+  const dim3 grid = fwd_grid<B_BORDER>(rd, L.num_views);
   const QuadDims q = make_quad_dims(rd.in);
   KernelTimer t(s, "render_lit_fwd");
   hipLaunchKernelGGL(k_render_density_lit_fwd, grid, dim3(kFwdThreads), kLitLds, s, reinterpret_cast<const float4*>(dq),
@@ -1054,14 +1062,16 @@ hipError_t render_density_lit_fwd_launch(hipStream_t s, const float* dq, const f
 // BORDER, CLAMP: dens is the corner-quad copy of that boundary.
 hipError_t render_density_fwd_launch(int bm, hipStream_t s, const float* dens, float* img, const RayDims& rd,
                                      const RayLaunch& L, const RenderParams& rp, const RenderSaved& sv) {
-  const dim3 grid = fwd_grid(rd, bm == B_BORDER, L.num_views);
   const QuadDims q = make_quad_dims(rd.in);
   const RenderSaved none{nullptr, nullptr, nullptr};
   KernelTimer t(s, "render_fwd");
+  auto run = [&](auto kern, dim3 grid, int rows, const RenderSaved& to) {
+    hipLaunchKernelGGL(kern, grid, dim3(kRTileX * rows), 0, s, dens, img, rd, L, rp, q, to);
+  };
   switch (bm) {
-    case B_BORDER: hipLaunchKernelGGL(k_render_density_fwd<B_BORDER>, grid, dim3(kFwdThreads), 0, s, dens, img, rd, L, rp, q, sv); break;
-    case B_CLAMP: hipLaunchKernelGGL(k_render_density_fwd<B_CLAMP>, grid, dim3(kFwdThreads), 0, s, dens, img, rd, L, rp, q, none); break;
-    default: hipLaunchKernelGGL(k_render_density_fwd<B_WRAP>, grid, dim3(kFwdThreads), 0, s, dens, img, rd, L, rp, q, none); break;
+    case B_BORDER: run(k_render_density_fwd<B_BORDER>, fwd_grid<B_BORDER>(rd, L.num_views), kFwdRows<B_BORDER>, sv); break;
+    case B_CLAMP: run(k_render_density_fwd<B_CLAMP>, fwd_grid<B_CLAMP>(rd, L.num_views), kFwdRows<B_CLAMP>, none); break;
+    default: run(k_render_density_fwd<B_WRAP>, fwd_grid<B_WRAP>(rd, L.num_views), kFwdRows<B_WRAP>, none); break;
   }
   return hipGetLastError();
 }
