@@ -988,21 +988,12 @@ static int batch_layout(int32_t n, const gft_batch_recon* rs, int32_t num_mipmap
 // gather from the back, both with their long items first.
 static double gather_load(const gft_batch_recon& c) {
   const Mat4d m = mat_from_colmajor(c.M);
-  const double x = 0.5 * c.grid_dhw[2], y = 0.5 * c.grid_dhw[1], z = 0.5 * c.grid_dhw[0];
   double load = 0.0;
   for (int v = 0; v < c.num_views; ++v) {
     const Mat4d A = mat_mul(mat_from_colmajor(c.P + 16 * v), mat_mul(mat_from_colmajor(c.V + 16 * v), m));
-    auto row = [&](int r) { return A.m[r] * x + A.m[4 + r] * y + A.m[8 + r] * z + A.m[12 + r]; };
-    const double cx = row(0), cy = row(1), cw = row(3);
-    double gx[3], gy[3];  // the pixel coordinates' derivatives along the grid's axes
-    for (int a = 0; a < 3; ++a) {
-      gx[a] = 0.5 * c.output_shape[2] * (A.m[4 * a] * cw - cx * A.m[4 * a + 3]) / (cw * cw);
-      gy[a] = 0.5 * c.output_shape[1] * (A.m[4 * a + 1] * cw - cy * A.m[4 * a + 3]) / (cw * cw);
-    }
-    const double n0 = gx[1] * gy[2] - gx[2] * gy[1], n1 = gx[2] * gy[0] - gx[0] * gy[2],
-                 n2 = gx[0] * gy[1] - gx[1] * gy[0];
-    const double area = std::sqrt(n0 * n0 + n1 * n1 + n2 * n2);
-    if (std::isfinite(area)) load += area;
+    double n[3];
+    if (face_pixels(A.m, Dims3{c.grid_dhw[2], c.grid_dhw[1], c.grid_dhw[0]}, c.output_shape[2], c.output_shape[1], n))
+      load += std::sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
   }
   return load;
 }

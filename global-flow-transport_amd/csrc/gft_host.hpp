@@ -37,6 +37,26 @@ struct ViewPair {
 };
 std::vector<ViewPair> view_pairs(int N, int num_cameras, bool separate_camera_batch);
 
+// Pixels that look through a unit of the x-, y- and z-facing area of grid d at
+// its centre, in an image of w x h pixels: the cross products of the pixel
+// coordinates' derivatives along the grid's axes. A is projection * model-view,
+// column-major. False where the centre has no finite image.
+template <class T> bool face_pixels(const T* A, Dims3 d, double w, double h, double n[3]) {
+  const double x = 0.5 * d.x, y = 0.5 * d.y, z = 0.5 * d.z;
+  auto row = [&](int r) { return A[r] * x + A[4 + r] * y + A[8 + r] * z + A[12 + r]; };
+  const double cx = row(0), cy = row(1), cw = row(3);
+  double gx[3], gy[3];
+  for (int a = 0; a < 3; ++a) {
+    gx[a] = 0.5 * w * (A[4 * a] * cw - cx * A[4 * a + 3]) / (cw * cw);
+    gy[a] = 0.5 * h * (A[4 * a + 1] * cw - cy * A[4 * a + 3]) / (cw * cw);
+  }
+  for (int a = 0; a < 3; ++a) {
+    const int b = (a + 1) % 3, c = (a + 2) % 3;
+    n[a] = std::fabs(gx[b] * gy[c] - gx[c] * gy[b]);
+  }
+  return std::isfinite(n[0] + n[1] + n[2]);
+}
+
 // Per-view projective coefficients of the raymarch's pixel rays (near0, far0,
 // gx, gy of ProjView) from the inverse projection and inverse model-view.
 void ray_coefficients(const Mat4d& pinv, const Mat4d& mvinv, const RayDims& rd, ProjView& pv);

@@ -31,7 +31,7 @@
 //            with coalesced global atomics.
 //   WRAP   : the same walk with per-sample global atomics.
 // Samples of a BORDER ray outside the grid read 0 and are skipped (exact).
-#include "gft_device.hpp"
+#include "gft_host.hpp"
 #include "quad.hpp"
 
 namespace gft {
@@ -477,8 +477,8 @@ __global__ __launch_bounds__(256) void k_render_density_bwd_pixel(const float* _
   }
 }
 
-// Gather: one workgroup of NW waves per block of WX x WY x WZ voxels, each wave
-// accumulating in an FP64 LDS region of its own. For each view the waves
+// Gather: NW waves per block of WX x WY x WZ voxels, NB blocks to a workgroup, each
+// wave accumulating in an FP64 LDS region of its own. For each view a block's waves
 // enumerate the pixels whose rays can cross the block's support box (x0-1,
 // x0+WX) x ... (the projected box, in batches of 64 consecutive pixels in row
 // order, which the waves take in turn), cut each ray by the box and add every
@@ -497,28 +497,32 @@ constexpr int kGatherBatch = 4;  // saved values loaded per round trip (2: 0.187
 // folded in), workgroup 0 first sums the pixel pass's per-tile loss partials
 // of every view in a fixed order; the kernel boundary after the pixel pass
 // makes them visible, so no separate launch is needed.
-template <int WX, int WY, int WZ, int NW, bool LIT>
-__global__ __launch_bounds__(64 * NW) void k_render_density_bwd_gather(RenderSaved sv, float* __restrict__ grad,
-                                                                       RayDims rd, ProjLaunch PL,
-                                                                       const float* __restrict__ dens,
-                                                                       const float* __restrict__ lam,
-                                                                       float* __restrict__ lam_grad,
-                                                                       float* __restrict__ loss, float loss_scale) {
+template <int WX, int WY, int WZ, int NW, int NB, bool LIT>
+__global__ __launch_bounds__(64 * NW * NB) void k_render_density_bwd_gather(RenderSaved sv, float* __restrict__ grad,
+                                                                            RayDims rd, ProjLaunch PL,
+                                                                            const float* __restrict__ dens,
+                                                                            const float* __restrict__ lam,
+                                                                            float* __restrict__ lam_grad,
+                                                                            float* __restrict__ loss,
+                                                                            float loss_scale) {
   if (loss && blockIdx.x == 0) {
-    __shared__ float red[64 * NW];
+    __shared__ float red[64 * NW * NB];
     loss_sum_block(sv.partials, sv.n_partials, loss_scale, loss, red);
   }
   // rows padded to WX + 1 doubles: lanes at one x in neighbouring rows fall on
   // different LDS banks (16 doubles are 128 bytes, the banks' width)
   constexpr int kRX = WX + 1;
   constexpr int kVox = kRX * WY * WZ;
-  __shared__ double region[LIT ? 2 * NW : NW][kVox];
+  __shared__ double region[(LIT ? 2 : 1) * NB * NW][kVox];
   typedef __attribute__((address_space(3))) double lds_double;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  lds_double* acc = (lds_double*)region[wave];
-  lds_double* acc2 = (lds_double*)region[LIT ? NW + wave : wave];
+  const int lane = threadIdx.x & 63, all = threadIdx.x >> 6;  // the wave in its workgroup
+  const int own = NB > 1 ? all / NW : 0, wave = NB > 1 ? all % NW : all;  // the block in it, the wave in that
+  lds_double* acc = (lds_double*)region[all];
+  lds_double* acc2 = (lds_double*)region[LIT ? NB * NW + all : all];
   const Dims3 d = rd.in;
-  const int nbx = (d.x + WX - 1) / WX, nby = (d.y + WY - 1) / WY, blk = (int)blockIdx.x;
+  const int nbx = (d.x + WX - 1) / WX, nby = (d.y + WY - 1) / WY, blk = (int)blockIdx.x * NB + own;
+  // a wave past the last block only joins the barriers
+  const int views = NB == 1 || blk < nbx * nby * ((d.z + WZ - 1) / WZ) ? PL.num_views : 0;
   const int x0 = (blk % nbx) * WX, y0 = ((blk / nbx) % nby) * WY, z0 = (blk / (nbx * nby)) * WZ;
   for (int k = lane; k < kVox; k += 64) acc[k] = 0.0;
   if (LIT)
@@ -530,7 +534,7 @@ __global__ __launch_bounds__(64 * NW) void k_render_density_bwd_gather(RenderSav
   const float bx0 = fx0 - 0.5f, by0 = fy0 - 0.5f, bz0 = fz0 - 0.5f;
   const float bx1 = bx0 + (float)(WX + 1), by1 = by0 + (float)(WY + 1), bz1 = bz0 + (float)(WZ + 1);
   const float hx = 0.5f * (float)(WX + 1), hy = 0.5f * (float)(WY + 1), hz = 0.5f * (float)(WZ + 1);
-  for (int vi = 0; vi < PL.num_views; ++vi) {
+  for (int vi = 0; vi < views; ++vi) {
     const ProjView& pv = PL.view[vi];
     const float* A = pv.pmv;
     const float4 cc = mat_vec(A, fx0 + 0.5f * (float)WX, fy0 + 0.5f * (float)WY, fz0 + 0.5f * (float)WZ, 1.f);
@@ -671,19 +675,20 @@ __global__ __launch_bounds__(64 * NW) void k_render_density_bwd_gather(RenderSav
     }
   }
   __syncthreads();
-  for (int k0 = threadIdx.x; k0 < WX * WY * WZ; k0 += 64 * NW) {
+  const int r0 = own * NW;  // the block's first region
+  for (int k0 = wave * 64 + lane; k0 < WX * WY * WZ; k0 += 64 * NW) {
     const int x = x0 + k0 % WX, y = y0 + (k0 / WX) % WY, z = z0 + k0 / (WX * WY);
     const int k = (k0 / WX) * kRX + k0 % WX;
     if (x < d.x && y < d.y && z < d.z) {
       const size_t f = flat3(x, y, z, d);
       float* g = grad + f;
-      double ss = region[0][k];
+      double ss = region[r0][k];
 #pragma unroll
-      for (int w = 1; w < NW; ++w) ss += region[w][k];
+      for (int w = 1; w < NW; ++w) ss += region[r0 + w][k];
       if (LIT) {
-        double se = region[NW][k];
+        double se = region[NB * NW + r0][k];
 #pragma unroll
-        for (int w = 1; w < NW; ++w) se += region[NW + w][k];
+        for (int w = 1; w < NW; ++w) se += region[NB * NW + r0 + w][k];
         const float v = (float)(ss + (double)lam[f] * se), vl = (float)((double)dens[f] * se);
         *g = PL.accumulate ? *g + v : v;
         lam_grad[f] = PL.accumulate ? lam_grad[f] + vl : vl;
@@ -1094,36 +1099,56 @@ hipError_t render_density_pixel_launch(bool l2, hipStream_t s, const float* img,
   return hipGetLastError();
 }
 
-template <int WX, int WY, int WZ, int NW, bool LIT>
+template <int WX, int WY, int WZ, int NW, int NB, bool LIT>
 static void launch_render_gather(hipStream_t s, const RenderSaved& sv, const float* dens, const float* lam,
                                  float* grad, float* lam_grad, const RayDims& rd, const ProjLaunch& PL, float* loss,
                                  float loss_scale) {
   const int nb = ((rd.in.x + WX - 1) / WX) * ((rd.in.y + WY - 1) / WY) * ((rd.in.z + WZ - 1) / WZ);
-  auto kern = k_render_density_bwd_gather<WX, WY, WZ, NW, LIT>;
-  hipLaunchKernelGGL(kern, dim3(nb), dim3(64 * NW), 0, s, sv, grad, rd, PL, dens, lam, lam_grad, loss, loss_scale);
+  auto kern = k_render_density_bwd_gather<WX, WY, WZ, NW, NB, LIT>;
+  hipLaunchKernelGGL(kern, dim3((nb + NB - 1) / NB), dim3(64 * NW * NB), 0, s, sv, grad, rd, PL, dens, lam, lam_grad,
+                     loss, loss_scale);
 }
 
-// Block shape and waves per block, by the number of 16x16x2-voxel blocks nb.
-// A block's waves share its pixels, so more of them help wherever blocks
-// alone do not fill the 256 CUs evenly; each costs a region to clear and sum.
-// Measured (gather alone, us; 1 / 2 / 4 / 8 waves per 16x16x2 block):
-//   nb = 29900 (200x356x200, 8 views)  1619 / 1529 / 1520 / 1640
-//   nb = 14400 (160x280x160, 5 views)   246 /  223 /  246 /  318
-//   nb =  7168 (128x224x128, 5 views)   172 /  163 /  163 /  188
-//   nb =  4200 (100x178x100, 6 views)   278 /  223 /  203 /  205
-//   nb =   868 (61x107x59, 5 views)      93 /   57 /   43 /   41
-//   nb =   432 (48x86x48, 5 views)      186 /  104 /   63 /   50
-//   nb =    64 (32x32x32, 2 views)      428 /  208 /  119 /   96
-// The last has a block for every fourth CU only: 4x4x4-voxel blocks, 512 of
-// them, take 29 us with 8 waves (8x4x4 blocks: 31, 8x8x2: 34).
+// 64-pixel batches that look through a 16x16x2-voxel block's support, all views
+static double block_batches(const RayDims& rd, const ProjLaunch& PL) {
+  double pixels = 0.0, n[3];
+  for (int v = 0; v < PL.num_views; ++v)
+    if (face_pixels(PL.view[v].pmv, rd.in, rd.out_w, rd.out_h, n)) pixels += 17 * 17 * n[2] + 17 * 3 * (n[0] + n[1]);
+  return pixels / 64.0;
+}
+
+// Block shape and waves per block, by the number nb of 16x16x2-voxel blocks and
+// the pixel batches b of one. A block's waves share its batches, so more of them
+// help where blocks alone do not fill the 256 CUs evenly; each costs a region to
+// clear and sum, and the views' set-up. Measured (gather alone, us; 1 / 2 / 4 / 8 waves
+// per 16x16x2 block, the 1 with four blocks to a workgroup; / 4x4x4 with 8):
+//   nb = 29900, b = 61  (200x356x200, 8 views)  1619 / 1529 / 1520 / 1640
+//   nb = 14400, b = 17  (160x280x160, 5 views)   246 /  223 /  246 /  318
+//   nb =  7168, b = 21  (128x224x128, 5 views)   172 /  163 /  163 /  188
+//   nb =  6144, b = .3  (128x190x115, 5 views)    39 /   48 /   65 /   98
+//   nb =  5760, b = 4.5 (128x174x119, 1 view)     31 /   30 /   32 /   40
+//   nb =  4200, b = 45  (100x178x100, 6 views)   278 /  223 /  203 /  205
+//   nb =  2160, b = 1.4 (80x143x86, 5 views)      28 /   27 /   34 /   44
+//   nb =  1680, b = 11  (80x105x86, 5 views)      67 /   50 /   43 /   48
+//   nb =   868, b = 21  (61x107x59, 5 views)      93 /   57 /   43 /   41
+//   nb =   576, b = 1.5 (48x84x52, 5 views)       23 /   21 /   19 /   21 / 58
+//   nb =   216, b = 1.5 (36x59x37, 5 views)       22 /   18 /   16 /   15 / 31
+//   nb =   162, b = 42  (36x43x35, 5 views)      177 /   96 /   58 /   38 / 28
+//   nb =    64, b = 124 (32x32x32, 2 views)      428 /  208 /  119 /   96 / 29
+// The lit gather's lines lie at the same places, but for the 4x4x4 blocks (36x44x38,
+// 5 views, nb = 162, b = 20: 29 with 8 waves, 27 with those; not lit 23, 24).
 template <bool LIT>
 static void render_gather(hipStream_t s, const RenderSaved& sv, const float* dens, const float* lam, float* grad,
                           float* lam_grad, const RayDims& rd, const ProjLaunch& PL, float* loss, float loss_scale) {
-  const int64_t nb = (int64_t)((rd.in.x + 15) / 16) * ((rd.in.y + 15) / 16) * ((rd.in.z + 1) / 2);
-  if (nb < 256) launch_render_gather<4, 4, 4, 8, LIT>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
-  else if (nb < 640) launch_render_gather<16, 16, 2, 8, LIT>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
-  else if (nb < 8192) launch_render_gather<16, 16, 2, 4, LIT>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
-  else launch_render_gather<16, 16, 2, 2, LIT>(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale);
+  const double nb = (double)((rd.in.x + 15) / 16) * ((rd.in.y + 15) / 16) * ((rd.in.z + 1) / 2);
+  const double b = block_batches(rd, PL), per = 1000.0 * b / nb;
+  auto run = [&](auto launch) { launch(s, sv, dens, lam, grad, lam_grad, rd, PL, loss, loss_scale); };
+  if (nb < 256 && b * (LIT ? 12 : 8) > nb) run(launch_render_gather<4, 4, 4, 8, 1, LIT>);
+  else if (nb >= 1500 && per < 0.7) run(launch_render_gather<16, 16, 2, 1, 4, LIT>);
+  else if (nb >= 8192 || (nb >= 400 && b < 1.0)) run(launch_render_gather<16, 16, 2, 2, 1, LIT>);
+  else if (nb < 640) run(launch_render_gather<16, 16, 2, 8, 1, LIT>);
+  else if (per < 1.7 || (nb > 6000 && per < 2.8)) run(launch_render_gather<16, 16, 2, 2, 1, LIT>);
+  else run(launch_render_gather<16, 16, 2, 4, 1, LIT>);
 }
 
 // loss: null, or where workgroup 0 writes loss_scale * the sum of the loss partials

@@ -143,3 +143,31 @@ def test_pyramid_launches(cuda, shape, channels, levels):
         d = [n // 2 for n in ref.shape[1:4]]
         ref = ref[:, :2 * d[0], :2 * d[1], :2 * d[2]].reshape(1, d[0], 2, d[1], 2, d[2], 2, channels).mean((2, 4, 6))
         assert norm_err(got[m].cpu().numpy(), ref) < 1e-6
+
+
+# the render gathers' block shapes and waves, by blocks (nb) and pixel batches a block:
+# 4x4x4 blocks, many of them and ragged in every axis (nb = 24); the same count with few
+# pixels (8 waves); nb = 441 with few (2 waves); nb = 1521 with few (one wave, four
+# blocks a workgroup, the last part empty); nb = 1305 (2 waves), 1521 (4); nb = 9288 (2)
+@pytest.mark.parametrize("grid,image,views", [((11, 19, 23), (70, 85), 2), ((35, 58, 37), (8, 5), 3),
+                                              ((97, 40, 40), (6, 5), 2), ((337, 40, 37), (12, 10), 2),
+                                              ((289, 38, 34), (26, 23), 2), ((337, 40, 37), (120, 111), 2),
+                                              ((258, 130, 113), (230, 196), 1)])
+@pytest.mark.parametrize("lit", [False, True])
+def test_render_gather_waves(cuda, grid, image, views, lit):
+    from gft.pipeline import render_density, render_density_lit
+    sc = scene(grid=grid, image=image, views=views, seed=sum(grid))
+    cam = (sc["M"], sc["V"], sc["P"], sc["F"], sc["out_dhw"], sc["step"])
+    rng = np.random.Generator(np.random.PCG64(views))
+    lam = rng.uniform(0.2, 1.2, size=sc["data"].shape).astype(np.float32)
+    w = rng.uniform(-1, 1, size=(1, views) + tuple(image) + (4,)).astype(np.float32)
+    d, l = _t(sc["data"]).requires_grad_(True), _t(lam).requires_grad_(True)
+    img = render_density_lit(d, l, *cam, ambient=0.4) if lit else render_density(d, *cam)
+    img.backward(_t(w))
+    img = img.detach().cpu().numpy()
+    if lit:
+        rd, rl = orc.render_lit_bwd(sc["data"], lam, img, w, *cam, ambient=0.4)
+        assert norm_err(l.grad.cpu().numpy(), rl) < 1e-4
+    else:
+        rd = orc.render_density_bwd(sc["data"], img, w, *cam)
+    assert norm_err(d.grad.cpu().numpy(), rd) < 1e-4
