@@ -569,11 +569,8 @@ typedef __attribute__((address_space(3))) double lds_f64;  // an FP64 LDS region
 // 1358. Without mips: 4: 651 (4); 5: 597 (2), 592 (4); 6: 595 (2), 589 (3), 608 (4).
 constexpr int kGatherBatch = 3;
 constexpr int kGatherOccupancy = 6;
-// waves that share a voxel block: they take its pixel batches in turn, each
-// into regions of its own
-// (ten uneven reconstructions, gather: 1 wave 2.80 ms, 2: 2.02, 4: 1.66, 8:
-// 1.93; 32 of them 6.15 / 5.11 / 4.86 / 5.65; three small ones seen through
-// large images 2.09 / 1.19 / 0.75 / 0.64)
+// waves that share a voxel block of a coarse level: they take its pixel batches in
+// turn, each into regions of its own. Levels 0 and 1: gather_waves.
 constexpr int kGatherWaves = 4;
 // copies of the level-1 region, lane l adding into copy l % kL1Copies: the
 // level-1 cells are 8 times the volume of level 0's, so neighbouring pixels'
@@ -630,7 +627,7 @@ __device__ __forceinline__ bool inside_level(float qx, float qy, float qz, Dims3
 // One item of the gather: the block (blk = item's block) of reconstruction
 // R at level m (PAIR: levels 0 and 1), with the block shape WX x WY x WZ as
 // compile-time constants (index arithmetic and bounds on immediates).
-template <bool PAIR, int WX, int WY, int WZ>
+template <bool PAIR, int NW, int WX, int WY, int WZ>
 __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, int wave, int lane, lds_f64* all) {
   constexpr int kVox = kL0Stride + (PAIR ? kL1Copies * kL1Stride : 0);
   lds_f64* acc = all + wave * kVox;                                     // this wave's block cells
@@ -639,7 +636,7 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
   const Dims3 dm = R.mt.dims[m];
   const bool two = PAIR && R.mt.levels > 0;
   const Dims3 d1 = R.mt.dims[two ? 1 : 0];
-  const int nbx = (dm.x + WX - 1) / WX, nby = (dm.y + WY - 1) / WY, nbz = (dm.z + WZ - 1) / WZ;
+  const int nbx = (dm.x + WX - 1) / WX, nby = (dm.y + WY - 1) / WY;
   const int blk = item - R.pass_item0[kGatherPass + m];
   const int x0 = (blk % nbx) * WX, y0 = ((blk / nbx) % nby) * WY, z0 = (blk / (nbx * nby)) * WZ;
   for (int k = lane; k < kVox; k += 64) acc[k] = 0.0;
@@ -653,7 +650,6 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
                           : (x0 + WX < dm.x) & (y0 + WY < dm.y) & (z0 + WZ < dm.z));
   const int S = R.out_d;
   const float inv_s1 = column_rcp(S);
-  const bool mips = R.mt.levels > 0;
   const float lmaxf = (float)R.mt.levels;
   const int per_view = R.tiles_x * R.tiles_y;
   const float4* __restrict__ recv = reinterpret_cast<const float4*>(R.records);
@@ -695,10 +691,10 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
     const int nxr = xe - xs + 1, cnt = nxr * (ye - ys + 1);
     // this lane's first place in the box's row-major pixel list; its next
     // record (64 kGatherWaves on) is loaded while the current one is walked
-    constexpr int kStride = 64 * kGatherWaves;
+    constexpr int kStride = 64 * NW;
     const int first = turn * 64 + lane;
-    turn -= (cnt + 63) / 64 % kGatherWaves;
-    turn += turn < 0 ? kGatherWaves : 0;
+    turn -= (cnt + 63) / 64 % NW;
+    turn += turn < 0 ? NW : 0;
     const int dys = kStride / nxr, dxs = kStride - dys * nxr;
     int px = xs + first % nxr, py = ys + first / nxr;
     auto rec_at = [&](int qx, int qy, int& it, int& slot) {
@@ -793,7 +789,7 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
     // from their gathers, which ran before; each level's value rounded to
     // float and accumulated by fma from level 1 up
     const int W1 = WX / 2, H1 = WY / 2;
-    for (int k = threadIdx.x; k < kBlockVox; k += 64 * kGatherWaves) {
+    for (int k = threadIdx.x; k < kBlockVox; k += 64 * NW) {
       const int lx = k % WX, ly = (k / WX) % WY, lz = k / (WX * WY);
       const int x = x0 + lx, y = y0 + ly, z = z0 + lz;
       if (x >= dm.x || y >= dm.y || z >= dm.z) continue;
@@ -808,7 +804,7 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
             const int c1 = (lx >> 1) + W1 * ((ly >> 1) + H1 * (lz >> 1));
             double t1 = 0.0;
 #pragma unroll
-            for (int w = 0; w < kGatherWaves; ++w)
+            for (int w = 0; w < NW; ++w)
 #pragma unroll
               for (int c = 0; c < kL1Copies; ++c) t1 += all[w * kVox + kL0Stride + c * kL1Stride + c1];
             gl = (float)t1;
@@ -820,7 +816,7 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
       }
       double t0 = all[k];
 #pragma unroll
-      for (int w = 1; w < kGatherWaves; ++w) t0 += all[w * kVox + k];
+      for (int w = 1; w < NW; ++w) t0 += all[w * kVox + k];
       R.grad[flat3(x, y, z, dm)] = (float)t0 + g;
     }
     if (blk == 0 && wave == 0) {
@@ -834,23 +830,23 @@ __device__ __forceinline__ void gather_item(const BatchRec& R, int m, int item, 
     }
   } else {
     float* __restrict__ gout = grad_cells(R, m);
-    for (int k = threadIdx.x; k < kBlockVox; k += 64 * kGatherWaves) {
+    for (int k = threadIdx.x; k < kBlockVox; k += 64 * NW) {
       const int x = x0 + k % WX, y = y0 + (k / WX) % WY, z = z0 + k / (WX * WY);
       if (x >= dm.x || y >= dm.y || z >= dm.z) continue;
       double t0 = all[k];
 #pragma unroll
-      for (int w = 1; w < kGatherWaves; ++w) t0 += all[w * kVox + k];
+      for (int w = 1; w < NW; ++w) t0 += all[w * kVox + k];
       gout[pad_index(x + 1, y + 1, z + 1, dm)] = (float)t0;
     }
   }
   __syncthreads();  // the regions are cleared by the next item
 }
 
-template <bool PAIR>
-__global__ __launch_bounds__(64 * kGatherWaves, kGatherOccupancy) void k_batch_gather(const BatchRec* __restrict__ recs, int nrec, int m,
-                                                                    int total_items) {
+template <bool PAIR, int NW>
+__global__ __launch_bounds__(64 * NW, kGatherOccupancy) void k_batch_gather(const BatchRec* __restrict__ recs,
+                                                                            int nrec, int m, int total_items) {
   constexpr int kVox = kL0Stride + (PAIR ? kL1Copies * kL1Stride : 0);
-  __shared__ double region[kGatherWaves * kVox];
+  __shared__ double region[NW * kVox];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   lds_f64* all = (lds_f64*)region;
   for (int at = blockIdx.x; at < total_items; at += gridDim.x) {
@@ -859,9 +855,9 @@ __global__ __launch_bounds__(64 * kGatherWaves, kGatherOccupancy) void k_batch_g
     const int item = total_items - 1 - at;
     const BatchRec& R = recs[rec_of(recs, nrec, item, kGatherPass + m)];
     // the reconstruction's block shape (bricks 0, 1, 2: 16x16x2, 8x8x8, 16x8x4)
-    if (R.bd == 2) gather_item<PAIR, 16, 16, 2>(R, m, item, wave, lane, all);
-    else if (R.bd == 8) gather_item<PAIR, 8, 8, 8>(R, m, item, wave, lane, all);
-    else gather_item<PAIR, 16, 8, 4>(R, m, item, wave, lane, all);
+    if (R.bd == 2) gather_item<PAIR, NW, 16, 16, 2>(R, m, item, wave, lane, all);
+    else if (R.bd == 8) gather_item<PAIR, NW, 8, 8, 8>(R, m, item, wave, lane, all);
+    else gather_item<PAIR, NW, 16, 8, 4>(R, m, item, wave, lane, all);
   }
 }
 
@@ -996,6 +992,26 @@ static double gather_load(const gft_batch_recon& c) {
       load += std::sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
   }
   return load;
+}
+
+// Waves per block of the level-0/1 gather. One more wave costs each of the `blocks`
+// a set-up and regions to clear and sum (1.9 ns of the launch), and halves the
+// chain of the heaviest block's pixel batches (1.7 us each with one wave), which
+// ends the launch; their number from the shapes, for a grid that fills its images.
+// us, 1 / 2 / 4 waves: eight of 96x170x96, 5 views at 0.5 pixels a voxel 148 / 216 / 331,
+// at 2.3 686 / 735 / 832; 128x224x128, 5 views at 1.0 80 / 91 / 118, at 2.0 202 / 199 /
+// 223; 64x112x64, 5 at 1.0 41 / 31 / 27; with mips ten uneven 2059 / 1243 / 1356, 32 of
+// them 3300 / 3442 / 3738, three of them 1901 / 1030 / 559; 16 of 32x40x32, 2 views at
+// 1.0 81 / 63 / 55 (too few blocks for less than 4).
+static int gather_waves(int32_t n, const gft_batch_recon* rs, int blocks) {
+  double heaviest = 0.0;
+  for (int r = 0; r < n; ++r) {
+    const gft_batch_recon& c = rs[r];
+    heaviest = std::max(heaviest, 3.2 * c.num_views * c.output_shape[1] * c.output_shape[2] /
+                                      ((double)c.grid_dhw[1] * c.grid_dhw[2]));
+  }
+  if (blocks < 2000 || blocks < 109.0 * heaviest) return kGatherWaves;
+  return blocks < 437.0 * heaviest ? 2 : 1;
 }
 
 // item counts of the launches: render items; the level passes (bordered
@@ -1185,10 +1201,15 @@ int gft_batch_render_run(void* stream, int32_t n, const gft_batch_recon* recons,
     // the coarse levels first: the level-0/1 gather adds them into the density gradient
     for (int m = kBatchMaxLevels; m >= 2; --m)
       if (pass[kGatherPass + m])
-        hipLaunchKernelGGL(k_batch_gather<false>, dim3(pass[kGatherPass + m]), dim3(64 * kGatherWaves), 0, s, recs, n, m,
+        hipLaunchKernelGGL((k_batch_gather<false, kGatherWaves>), dim3(pass[kGatherPass + m]), dim3(64 * kGatherWaves), 0, s, recs, n, m,
                            pass[kGatherPass + m]);
-    hipLaunchKernelGGL(k_batch_gather<true>, dim3(pass[kGatherPass]), dim3(64 * kGatherWaves), 0, s, recs, n, 0,
-                       pass[kGatherPass]);
+    auto run = [&](auto kern, int w) {
+      hipLaunchKernelGGL(kern, dim3(pass[kGatherPass]), dim3(64 * w), 0, s, recs, n, 0, pass[kGatherPass]);
+    };
+    const int waves = gather_waves(n, recons, pass[kGatherPass]);
+    if (waves == 1) run(k_batch_gather<true, 1>, 1);
+    else if (waves == 2) run(k_batch_gather<true, 2>, 2);
+    else run(k_batch_gather<true, kGatherWaves>, kGatherWaves);
   }
   return check_hip(hipGetLastError(), "batched render gather");
 }

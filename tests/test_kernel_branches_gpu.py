@@ -171,3 +171,21 @@ def test_render_gather_waves(cuda, grid, image, views, lit):
     else:
         rd = orc.render_density_bwd(sc["data"], img, w, *cam)
     assert norm_err(d.grad.cpu().numpy(), rd) < 1e-4
+
+
+# waves per block of the batched level-0/1 gather: 2070 blocks or more with 0.5, 9.5 and 43
+# estimated pixel batches (1, 2 and 4 waves), in every brick, with and without mips
+@pytest.mark.parametrize("image", [(12, 10), (60, 42), (120, 95)])
+@pytest.mark.parametrize("brick,mips", [(0, 3), (1, 3), (2, 1), (0, 0)])
+def test_batched_gather_waves(cuda, image, brick, mips):
+    from gft.batch import BatchedRenderStep
+    grid, views = (460, 41, 41), 2
+    sc = scene(grid=grid, image=image, views=views, seed=7)
+    tgt = np.random.Generator(np.random.PCG64(3)).uniform(0, 0.5, size=(views,) + image + (3,)).astype(np.float32)
+    b = BatchedRenderStep([dict(grid=grid, M=sc["M"], V=sc["V"], P=sc["P"], F=sc["F"], out_dhw=sc["out_dhw"],
+                                depth_step=sc["step"], brick=brick)], num_mipmaps=mips)
+    b.bind([_t(sc["data"])], [_t(tgt)])
+    b.run()
+    ref = orc.mip_render_fwd_bwd(sc["data"], tgt, sc["M"], sc["V"], sc["P"], sc["F"], sc["out_dhw"], sc["step"],
+                                 num_mipmaps=mips)
+    assert norm_err(b.grads[0].cpu().numpy(), ref["gd"]) < 1e-4
