@@ -399,7 +399,11 @@ __device__ __forceinline__ void quad_read_batch(const gcf32x4* __restrict__ quad
     iy[u] = (unsigned)clampi((int)fy + 1, 0, (int)qd.qy - 1);
     iz[u] = (unsigned)clampi((int)fz + 1, 0, (int)qd.qz - 2);
   }
-  quad_pairs<float4, U>(qd, ix, iy, iz, a0, a1);
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    a0[u] = quad_index<float4>(qd, ix[u], iy[u], iz[u]);
+    a1[u] = quad_index<float4>(qd, ix[u], iy[u], iz[u] + 1);
+  }
   f32x4 c0[U], c1[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {

@@ -59,7 +59,9 @@ __device__ __forceinline__ unsigned quad_index(const QuadDims& q, unsigned ix, u
 // both, of 24-bit numbers where the bricks' rows and each axis fit (32-bit
 // products run at a quarter of their rate): the CLAMP scatter of 96x170x96, 5
 // views of 222x395, takes 480 us, 492 with two indexes, its forward 103, 111. The
-// bfloat16 forward is faster with two (200x356x200, 8 views: 670 us, 679).
+// bfloat16 forward is faster with two (200x356x200, 8 views: 670 us, 679), and so
+// is the batched one, whose few rays wait for each other's addresses (128x224x128,
+// 2 views of 64x112: 96 us, 102).
 template <class Q, int U>
 __device__ __forceinline__ void quad_pairs(const QuadDims& q, const unsigned ix[U], const unsigned iy[U],
                                            const unsigned iz[U], unsigned a0[U], unsigned a1[U]) {
