@@ -1305,13 +1305,15 @@ static inline dim3 grid_for(size_t n, unsigned views) { return dim3((unsigned)((
 // 5.4 / 8.6), and so does a narrow grid, whose tiles are mostly idle lanes
 // (512x512x4, C = 4, 2 levels 6.8 / 7.6). Where rows of cells end within a 128-byte
 // line, a tile's 32 cells straddle two, which neighbours on other XCDs read again:
-// beyond 48 MB such a level goes in rows, and the tiles take those after it
-// (200x356x200, 3 levels: 16.8 in rows, 20.1 in tiles; 100x178x100, C = 4, of 28 MB,
-// 11.3 with the first level in rows, 9.8 in tiles).
+// beyond 48 MB (24 for one channel) such a level goes in rows, and the tiles take
+// those after it (3 levels, first in rows / all in tiles: 200x356x200 16.8 / 20.1;
+// 256x196x196 13.8 / 16.0; two of 90x200x120, 17 MB, 9.1 / 6.9; 100x178x100, C = 4, 28
+// MB, 11.3 / 9.8).
 int mip_levels_of_launch(const MipTable& mt, int first, int batches) {
   const Dims3 s = mt.dims[first], o = mt.dims[first + 1];
   const size_t row = (size_t)s.x * mt.C * sizeof(float), bytes = row * s.y * s.z * batches;
-  if ((o.x < 4 && (size_t)o.y * o.z > 1024) || (row % 128 != 0 && bytes > (size_t(48) << 20))) return 1;
+  const size_t large = size_t(mt.C == 1 ? 24 : 48) << 20;
+  if ((o.x < 4 && (size_t)o.y * o.z > 1024) || (row % 128 != 0 && bytes > large)) return 1;
   return std::min(mt.levels - first, kMipLevels);
 }
 
