@@ -713,7 +713,9 @@ constexpr int kSegK = 8;
 // as leave room for 8 waves on a CU. One more wave less costs more than the few
 // larger bricks gain, smaller bricks much more (below).
 constexpr int kCap = 2400;
-// more than any rounding of a sample's position against the corner rays'
+// Above the rounding of a sample's position against the corner rays' while positions
+// stay below 1e4 cells or so from the camera; a corner that still falls outside its
+// brick is added to global memory instead.
 constexpr float kBrickSlack = 1e-2f;
 
 struct Brick {
@@ -900,10 +902,12 @@ __global__ __launch_bounds__(64) void k_render_density_bwd_clamp(const float4* _
         const float tx = px - fx, ty = py - fy, tz = pz - fz;
         const float ux = 1.f - tx, uy = 1.f - ty, uz = 1.f - tz;
         const bool hx = __ballot(tx != 0.f) != 0, hy = __ballot(ty != 0.f) != 0, hz = __ballot(tz != 0.f) != 0;
-        // (a gradient that is not finite takes the exact corner test below: its product with a weight of 0 is not 0)
-        if (use_lds && __ballot(!(fabsf(g) < 3.4e38f)) == 0) {
-          const int lx = clampi((int)fx - br.lo[0], 0, br.n[0] - 2), ly = clampi((int)fy - br.lo[1], 0, br.n[1] - 2),
-                    lz = clampi((int)fz - br.lo[2], 0, br.n[2] - 2);
+        // (a gradient that is not finite takes the exact corner test below: its product with a weight of 0 is not 0;
+        // so does a corner outside the brick)
+        const int lx = (int)fx - br.lo[0], ly = (int)fy - br.lo[1], lz = (int)fz - br.lo[2];
+        const bool stray = ((unsigned)lx >= (unsigned)(br.n[0] - 1)) | ((unsigned)ly >= (unsigned)(br.n[1] - 1)) |
+                           ((unsigned)lz >= (unsigned)(br.n[2] - 1));
+        if (use_lds && __ballot(stray | !(fabsf(g) < 3.4e38f)) == 0) {
           lds_double* at = brick + (__mul24(lz, sz) + __mul24(ly, sy) + lx);
           const float gz[2] = {g * uz, g * tz};
 #pragma unroll

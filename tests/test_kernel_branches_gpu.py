@@ -189,3 +189,35 @@ def test_batched_gather_waves(cuda, image, brick, mips):
     ref = orc.mip_render_fwd_bwd(sc["data"], tgt, sc["M"], sc["V"], sc["P"], sc["F"], sc["out_dhw"], sc["step"],
                                  num_mipmaps=mips)
     assert norm_err(b.grads[0].cpu().numpy(), ref["gd"]) < 1e-4
+
+
+# A camera so far away (in cells) that ray positions round by more than a brick's
+# slack: a CLAMP sample outside its segment's brick still goes to its own cells. All
+# samples lie well inside the grid, where WRAP has the same positions and
+# corners and no bricks; the two then differ by the order of their sums alone
+# (float atomics of up to 100 terms a cell: 100 x 2^-24).
+@pytest.mark.parametrize("distance", [1e3, 2e6, 8e6])
+def test_clamp_scatter_far_camera(cuda, distance):
+    from gft.pipeline import render_density
+    n, half, image, S = 80, 12.0, (66, 70), 24
+    near, far = distance - half, distance + half
+    tan = half / far
+    P = np.zeros((4, 4))
+    P[0, 0] = P[1, 1] = 1.0 / tan
+    P[2, 2], P[2, 3], P[3, 2] = -(far + near) / (far - near), -2 * far * near / (far - near), -1
+    P[2, 0] = -1.2 * P[2, 2]  # near and far planes that lean: each pixel has a depth, and a rounding, of its own
+    V, M = np.eye(4), np.eye(4)
+    c, s = np.cos(0.7), np.sin(0.7)  # along a row, x hardly changes but for the rounding
+    V[0, 0], V[0, 2], V[2, 0], V[2, 2], V[2, 3] = c, s, -s, c, -distance
+    M[:3, 3] = -n / 2.0
+    M, V, P = (np.ascontiguousarray(a.T[None], dtype=np.float32) for a in (M, V, P))
+    F = np.array([[near, far, -near * tan, near * tan, near * tan, -near * tan]], dtype=np.float32)
+    rng = np.random.Generator(np.random.PCG64(5))
+    data = rng.uniform(0.0, 0.02, size=(1, n, n, n, 1)).astype(np.float32)
+    w = rng.uniform(-1, 1, size=(1, 1) + image + (4,)).astype(np.float32)
+    grads = []
+    for boundary in ("CLAMP", "WRAP"):
+        d = _t(data).requires_grad_(True)
+        render_density(d, M, V, P, F, (S,) + image, 1.0, boundary=boundary).backward(_t(w))
+        grads.append(d.grad.cpu().numpy())
+    assert norm_err(grads[0], grads[1]) < 1e-5
