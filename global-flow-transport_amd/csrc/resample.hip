@@ -204,7 +204,9 @@ __global__ __launch_bounds__(256) void k_mip_down(const float* __restrict__ src,
                                                   float* __restrict__ dst, size_t dst_stride, MipChain m,
                                                   float scale) {
 #pragma clang fp contract(off)
-  __shared__ float lds[(kMipX * kMipY * kMipZ + kMipX * kMipY * kMipZ / 8) * C];
+  // (both buffers are read and written as vectors of C floats)
+  alignas(16) __shared__ float lds[(kMipX * kMipY * kMipZ + kMipX * kMipY * kMipZ / 8) * C];
+  static_assert(kMipX * kMipY * kMipZ * sizeof(float) % 16 == 0);
   const int ntx = (m.dims[1].x + kMipX - 1) / kMipX, nty = (m.dims[1].y + kMipY - 1) / kMipY;
   const int t = (int)blockIdx.x;
   const int x0 = (t % ntx) * kMipX, y0 = ((t / ntx) % nty) * kMipY, z0 = (t / (ntx * nty)) * kMipZ;
