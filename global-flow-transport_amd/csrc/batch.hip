@@ -37,9 +37,9 @@
 //                      whose store is the density gradient itself: every
 //                      voxel's level-0 gradient plus 1/8^m of its level-m
 //                      ancestor's (the mip adjoint; level 1 from the same
-//                      wave's region); the first block of each reconstruction
-//                      also sums its loss from the per-tile partials in a
-//                      fixed order.
+//                      block's regions, a sum over its waves); the first
+//                      block of each reconstruction also sums its loss from
+//                      the per-tile partials in a fixed order.
 // The gather's block shape (16x16x2, 8x8x8 or 16x8x4 voxels) is chosen per
 // reconstruction.
 #include <algorithm>
@@ -551,9 +551,9 @@ __global__ __launch_bounds__(kTilePix) void k_batch_fwd(const BatchRec* __restri
 }
 
 // ------------------------------------------------------------------- gather
-// The transpose of the resample's trilinear scatter: kGatherWaves waves per voxel
-// block, accumulated in wave-private FP64 LDS regions that the store adds up. PAIR: levels 0 and 1 at once,
-// a block of bw x bh x bd level-0 voxels and the (bw/2) x (bh/2) x (bd/2)
+// The transpose of the resample's trilinear scatter: NW waves per voxel block,
+// accumulated in wave-private FP64 LDS regions that the store adds up. PAIR: levels
+// 0 and 1 at once, a block of bw x bh x bd level-0 voxels and the (bw/2) x (bh/2) x (bd/2)
 // level-1 cells over it (the level-1 cells' support box contains the level-0
 // voxels', so one walk over the candidate samples serves both); otherwise
 // level m alone (m >= 2, for views whose samples reach it). For each view the

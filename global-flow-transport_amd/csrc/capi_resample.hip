@@ -37,7 +37,7 @@ hipError_t sample_lut_launch(int C, int bm, hipStream_t st, const float* in, con
 hipError_t sample_lut_bwd_launch(int C, int bm, bool exact, hipStream_t st, const float* in_b, int fm, float offset,
                                  const LutLaunch& L, int views, const float* lut, const float* og, Dims3 din,
                                  float* grad_b, unsigned* cnt, float* lut_grad);
-hipError_t lod_transform_launch(hipStream_t st, Dims3 din, Dims3 dout, const SampleLaunch& L, float* out);
+hipError_t lod_transform_launch(hipStream_t st, Dims3 dout, const SampleLaunch& L, float* out);
 
 static size_t align256(size_t b) { return (b + 255) & ~size_t(255); }
 
@@ -613,8 +613,7 @@ int gft_lod_transform(void* stream, const int32_t input_dhw[3], const float* MV,
     if ((rc = build_sample_views(pairs, first, n, nullptr, -1, MV, P, frustum, cm, dims_dhw(input_dhw),
                                  dims_dhw(output_shape), L)))
       return rc;
-    if ((rc = check_hip(lod_transform_launch(st, dims_dhw(input_dhw), dims_dhw(output_shape), L, output),
-                        "lod transform launch")))
+    if ((rc = check_hip(lod_transform_launch(st, dims_dhw(output_shape), L, output), "lod transform launch")))
       return rc;
   }
   return GFT_OK;

@@ -430,7 +430,7 @@ __device__ __forceinline__ void block_loss(float sq, float* __restrict__ loss, f
 // beta) (and the L2 loss), the gather evaluates alpha * c_k + beta per sample.
 // A pixel with no gradient gets lo > hi so the gather skips it.
 // loss = scale * sum of the n tile partials, in a fixed order (deterministic):
-// 256 strided sums, then a tree over them
+// a strided sum a thread, then a tree over them
 __device__ __forceinline__ void loss_sum_block(const float* partials, int n, float scale, float* loss, float* red) {
   float t = 0.f;
   for (int i = threadIdx.x; i < n; i += blockDim.x) t += partials[i];

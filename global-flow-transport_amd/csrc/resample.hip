@@ -1005,7 +1005,7 @@ __global__ __launch_bounds__(256) void k_sample_lut_bwd_tiled(const float* __res
 // there. A neighbour's position is the same map of the same coordinates
 // ((x - 1) + 0.5 = (x + 0.5) - 1 exactly), so the result is unchanged.
 constexpr int kLodTX = 16, kLodTY = 8, kLodTZ = 4;
-__global__ __launch_bounds__(kLodTX * kLodTY * kLodTZ) void k_lod_transform(Dims3 din, Dims3 dout, SampleLaunch L,
+__global__ __launch_bounds__(kLodTX * kLodTY * kLodTZ) void k_lod_transform(Dims3 dout, SampleLaunch L,
                                                                             float* __restrict__ out) {
   constexpr int HX = kLodTX + 2, HY = kLodTY + 2, HZ = kLodTZ + 2, NH = HX * HY * HZ;
   __shared__ float hp[3][NH];
@@ -1487,11 +1487,11 @@ hipError_t sample_lut_bwd_launch(int C, int bm, bool exact, hipStream_t st, cons
   return hipGetLastError();
 }
 
-hipError_t lod_transform_launch(hipStream_t st, Dims3 din, Dims3 dout, const SampleLaunch& L, float* out) {
+hipError_t lod_transform_launch(hipStream_t st, Dims3 dout, const SampleLaunch& L, float* out) {
   const unsigned tiles = (unsigned)(((dout.x + kLodTX - 1) / kLodTX) * ((dout.y + kLodTY - 1) / kLodTY) *
                                    ((dout.z + kLodTZ - 1) / kLodTZ));
-  hipLaunchKernelGGL(k_lod_transform, dim3(tiles, (unsigned)L.num_views), dim3(kLodTX * kLodTY * kLodTZ), 0, st, din,
-                     dout, L, out);
+  hipLaunchKernelGGL(k_lod_transform, dim3(tiles, (unsigned)L.num_views), dim3(kLodTX * kLodTY * kLodTZ), 0, st, dout,
+                     L, out);
   return hipGetLastError();
 }
 

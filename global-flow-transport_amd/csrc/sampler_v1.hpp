@@ -44,15 +44,16 @@ __device__ __forceinline__ int level_taps(const SampleCfg& s, float lod, int* lv
 // 2^-m
 __device__ __forceinline__ float level_scale(int m) { return __int_as_float((127 - m) << 23); }
 
-// 1 / w to within an ulp
+// 1 / w to within an ulp: the hardware's estimate and one Newton step
 __device__ __forceinline__ float recip(float w) {
   const float r = __builtin_amdgcn_rcpf(w);
   return fmaf(fmaf(-w, r, 1.f), r, r);
 }
 
-// n / w with r = recip(w): the steps of a float division without its scaling,
-// which only quotients and divisors beyond 2^+-96 need; zeros, infinities and
-// NaN come out as in a division. Several numerators share a reciprocal.
+// n / w with r = recip(w): the product, corrected twice by its residual
+// (Markstein's method for a fused multiply-add), without a float division's
+// scaling, which only quotients and divisors beyond 2^+-96 need; zeros, infinities
+// and NaN come out as in a division. Several numerators share a reciprocal.
 __device__ __forceinline__ float quotient(float n, float w, float r) {
   float q = n * r;
   q = fmaf(fmaf(-w, q, n), r, q);
