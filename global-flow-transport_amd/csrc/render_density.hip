@@ -781,6 +781,7 @@ __device__ __forceinline__ Brick segment_brick(const float3* cn, const float3* c
 // 480 (562); 128x224x128, 5 of 256x456 917 (913). There, bricks of 1536 / 2048 /
 // 2304 / 2560 / 3072 cells: 3114 / 1064 / 912 / 990 / 1073; segments of 4 / 6:
 // 1020 / 905, but 585 / 518 at 96x170x96. BORDER at 128x224x128: 560 (953).
+// (The test for corners outside their brick, 1% since, is not in these.)
 // BORDER (the recompute alternative to the saved-state gather: nothing is
 // kept from the forward but the images) walks only the segments of the
 // tile's clipped sample ranges; samples outside the grid read 0 and corners
